@@ -11,12 +11,12 @@ Kinds:
   sweep    the one-token product of `count` matrices in turn, captured once as
            a HIP graph (a decoding loop's products)
   project  the fused RMSNorm and A8 of `rows` tokens, then their product
-  lookup   embedding rows of a batch of ids, and the sparse head over candidates
+  lookup   embedding rows of a batch of ids, and the sparse head over an agent's candidates
   pack     CQ-W4 packing of an f32 matrix and its upload
   turn     a fresh session: a prompt (with a span: a static prefix, then more
            tokens), then greedy decoding on the device
   steps    single-token steps of a session that already holds a long context
-  prefill  one prompt into a fresh session, the last position's logits
+  prefill  one prompt into a fresh session, the last position's logits or all
 """
 import functools
 import math
@@ -53,8 +53,6 @@ def listed():
         {"name": "project_1024", "kind": "project", "rows": 1024, "k": 768, "n": 3072, "bits": 4},
         # Every position of a long prompt against the head (scoring a prompt).
         {"name": "score_head", "kind": "project", "rows": 4096, "k": 768, "n": 8192, "bits": 4},
-        # Embedding rows of a prompt and an agent's candidate scoring.
-        {"name": "lookup", "kind": "lookup", "vocab": 16384, "k": 768, "ids": 512, "candidates": 200},
         # Packing and uploading a projection's f32 weights.
         {"name": "pack", "kind": "pack", "n": 3072, "k": 768},
         # A short conversation turn without a span: 118 tokens in, 32 out.
@@ -65,9 +63,11 @@ def listed():
         # Steps late in a long conversation, every key visible to the global layers.
         {"name": "steps_long", "kind": "steps", "context": 2900, "steps": 8},
         # The benchmark's prefill: one 512-token sequence.
-        {"name": "prefill_512", "kind": "prefill", "tokens": 512},
+        {"name": "prefill_512", "kind": "prefill", "tokens": 512, "outputs": "last"},
+        # Scoring a sequence: the logits of every position.
+        {"name": "prefill_all", "kind": "prefill", "tokens": 300, "outputs": "all"},
         # A document in the prompt.
-        {"name": "prefill_long", "kind": "prefill", "tokens": 3000},
+        {"name": "prefill_long", "kind": "prefill", "tokens": 3000, "outputs": "last"},
     ]
 
 
@@ -100,7 +100,8 @@ def draw(rng):
                 "ring": rng.randrange(64, 513) if span else 0, "steps": rng.randrange(1, 33)}
     if kind == "steps":
         return {"kind": kind, "context": _log(rng, 200, 2900), "steps": rng.randrange(1, 9)}
-    return {"kind": kind, "tokens": _log(rng, 2, 3000)}
+    outputs = rng.choice(("last", "last", "all"))
+    return {"kind": kind, "tokens": _log(rng, 2, 3000 if outputs == "last" else 1000), "outputs": outputs}
 
 
 # ------------------------------------------------------------------ inputs
@@ -265,7 +266,7 @@ def run(state):
             sess.rollback(len(sess) - case["context"])
         return [sess.forward(toks[i:i + 1]) for i in range(case["context"], case["context"] + case["steps"])]
     sess.reset()
-    return sess.forward(toks)
+    return sess.forward(toks) if case["outputs"] == "last" else sess.forward(toks, nh.OUT_ALL_LOGITS)
 
 
 # ------------------------------------------------------------------- work
@@ -319,7 +320,7 @@ def work(case):
     if kind == "steps":
         seen = [_forward_work(i, i + 1, 1) for i in range(case["context"], case["context"] + case["steps"])]
         return {f: sum(s[f] for s in seen) for f in ("bytes", "flops")}
-    return _forward_work(0, case["tokens"], 1)
+    return _forward_work(0, case["tokens"], 1 if case["outputs"] == "last" else case["tokens"])
 
 
 def tolerance(case):
