@@ -528,4 +528,118 @@ hipError_t launch_gemm_batch(const nh_qmat* const* w, const nh_qact* const* a, f
     return gemm_dispatch(g, block, ldy, 0, nullptr, s);
 }
 
+// ------------------------------------------------ decode combine, many rows
+// Several tokens against one matrix with every token's decode combine
+// (matmul_into at M = 1, qlinear.rs:340-350, per row): the heads of a feed
+// that returns every position's logits.  The four decode lanes of a group
+// keep sums of their own, so a token costs four conversions and four fmas an
+// (output, group) instead of the prefill combine's one of each: bound by
+// the vector ALU.  (One one-token product per row, 300 launches of the 8192
+// x 768 head, was the larger part of scoring a 300-token prompt: 1802 ->
+// 1154 us for the whole call with this one launch.)
+//
+// A wavefront owns two 16-row weight tiles (the int8 fragments, straight to
+// registers) against one 16-token tile.  Decode lane l of a group is bytes
+// 32 l .. 32 l + 32 of its activation order: k-blocks q = 2 (l & 1) + {0, 1}
+// of half l >> 1, so one v_mfma_i32_16x16x64_i8 with the other two blocks of
+// the activations zeroed is the exact lane sum.  The row norms of the
+// workgroup's weight rows go to LDS once; then per group acc[l] =
+// fma(float(L), (sx * cbs) * norm, acc[l]), and y = (l0 + l1) + (l2 + l3).
+// TW wavefronts of the workgroup's four take token tiles, the rest weight
+// tiles (TW: 1 up to 16 tokens, 2 up to 32, else 4).
+constexpr int DEC_WAVES = 4, DEC_RT = 2;
+constexpr int DEC_MAX_G = 32;
+
+template <int TW>
+__global__ __launch_bounds__(64 * DEC_WAVES) void k_gemm_decode(
+    const uint4* __restrict__ w8, const uint16_t* __restrict__ norms, const uint4* __restrict__ xq,
+    const float* __restrict__ sx, float* __restrict__ y, int ldy, int vec_store, int out, int tiles, int cap_rows,
+    int M, int G, float cbs) {
+    constexpr int WR = DEC_WAVES / TW * DEC_RT * 16;  // weight rows of the workgroup
+    __shared__ float ns[DEC_MAX_G * WR];              // [row][G]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, q = lane >> 4;
+    const int wr0 = (int)blockIdx.x * WR;
+    {
+        const int n = min(WR, tiles * 16 - wr0) * G;
+        for (int i = tid; i < n; i += 64 * DEC_WAVES) ns[i] = f16_bits_to_f32(norms[(size_t)wr0 * G + i]);
+    }
+    __syncthreads();
+    // (tiles past the matrix's, and tokens past the buffer's, read the last ones and store nothing)
+    const int lrow0 = wave / TW * DEC_RT * 16, tok = ((int)blockIdx.y * TW + wave % TW) * 16 + r;
+    const int tile0 = wr0 / 16 + wave / TW * DEC_RT;
+    if (tile0 >= tiles) return;
+    const int tokc = min(tok, cap_rows - 1);
+    const uint4* xrow = xq + (size_t)tokc * G * 8 + q;
+    const float* srow = sx + (size_t)tokc * G;
+    const uint4* wt[DEC_RT];
+#pragma unroll
+    for (int j = 0; j < DEC_RT; ++j) wt[j] = w8 + (size_t)min(tile0 + j, tiles - 1) * G * 128 + lane;
+    float acc[DEC_RT][4][4];  // [tile][decode lane][row]
+#pragma unroll
+    for (int j = 0; j < DEC_RT; ++j)
+#pragma unroll
+        for (int l = 0; l < 4; ++l)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[j][l][v] = 0.0f;
+    const int m0 = q < 2 ? -1 : 0, m1 = ~m0;  // the blocks of an even / odd decode lane
+    auto bits4 = [](uint4 a) { return v4i{(int)a.x, (int)a.y, (int)a.z, (int)a.w}; };
+    for (int g = 0; g < G; ++g) {
+        v4i a[DEC_RT][2], b[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            b[h] = bits4(xrow[g * 8 + h * 4]);
+#pragma unroll
+            for (int j = 0; j < DEC_RT; ++j) a[j][h] = bits4(wt[j][g * 128 + h * 64]);
+        }
+        const float sc = srow[g] * cbs;
+#pragma unroll
+        for (int j = 0; j < DEC_RT; ++j) {
+            float w[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) w[v] = sc * ns[(lrow0 + j * 16 + 4 * q + v) * G + g];
+#pragma unroll
+            for (int l = 0; l < 4; ++l) {
+                const v4i bl = b[l >> 1] & (l & 1 ? m1 : m0);
+                const v4i d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j][l >> 1], bl, v4i{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[j][l][v] = __builtin_fmaf((float)d[v], w[v], acc[j][l][v]);
+            }
+        }
+    }
+    if (tok >= M) return;
+#pragma unroll
+    for (int j = 0; j < DEC_RT; ++j) {
+        const int n0 = (tile0 + j) * 16 + 4 * q;
+        if (tile0 + j >= tiles) break;
+        float o[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) o[v] = (acc[j][0][v] + acc[j][1][v]) + (acc[j][2][v] + acc[j][3][v]);
+        float* dst = y + (size_t)tok * ldy + n0;
+        if (vec_store && n0 + 3 < out) {
+            *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (n0 + v < out) dst[v] = o[v];
+        }
+    }
+}
+
+hipError_t launch_gemm_decode(const nh_qmat* w, const nh_qact* a, float* y, int ldy, hipStream_t s) {
+    const QMatMeta& m = w->m;
+    if (m.groups > DEC_MAX_G || !w->d_w8 || a->rows > a->cap_rows) return hipErrorInvalidValue;
+    const int M = a->rows, tiles = m.out_pad / TILE_ROWS, vec = ldy % 4 == 0 && (uintptr_t)y % 16 == 0;
+    auto go = [&](auto tw) {
+        constexpr int TW = decltype(tw)::value, WT = DEC_WAVES / TW * DEC_RT;
+        hipLaunchKernelGGL(k_gemm_decode<TW>, dim3((tiles + WT - 1) / WT, (M + 16 * TW - 1) / (16 * TW)),
+                           dim3(64 * DEC_WAVES), 0, s, (const uint4*)w->d_w8, w->d_norms, (const uint4*)a->d_xq, a->d_sx,
+                           y, ldy, vec, m.out, tiles, a->cap_rows, M, m.groups, m.cbs);
+        return hipGetLastError();
+    };
+    if (M <= 16) return go(std::integral_constant<int, 1>{});
+    if (M <= 32) return go(std::integral_constant<int, 2>{});
+    return go(std::integral_constant<int, 4>{});
+}
+
 }  // namespace nh

@@ -150,6 +150,9 @@ hipError_t launch_read_floor(const nh_qmat* w, const nh_qact* a, int mode, float
 hipError_t launch_expand_w8(const nh_qmat* w, hipStream_t s);
 hipError_t launch_gemm(const nh_qmat* w, const nh_qact* a, const uint8_t* block, float* y, int ldy, int col0,
                        int32_t* dbg_totals, hipStream_t s);
+// a's rows against w with the decode combine of every row (y[i * ldy ..] is
+// the one-token product of row i), in one launch.
+hipError_t launch_gemm_decode(const nh_qmat* w, const nh_qact* a, float* y, int ldy, hipStream_t s);
 // Same-shaped prefill products in one launch (blockIdx.y picks the product):
 // gemv_batchable matrices, activations of equal rows, width and capacity.
 bool gemm_batchable(const nh_qmat* const* w, const nh_qact* const* a, int n);

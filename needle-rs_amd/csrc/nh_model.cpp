@@ -314,7 +314,7 @@ int build_model(nh_model* m, const nh::ArchiveSmall& sm) {
         return A.put(b.data(), b.size() * 2);
     };
     // The tables of the layer kernel, as one block per layer: the six
-    // Kronecker factors and cond_v [d][8] (staged into LDS), then cond_u
+    // Kronecker factors (MFMA fragments) and cond_v [d][8] (staged into LDS), then cond_u
     // by column, [hada_n][8] (f16; thread t reads its column's 16 bytes).
     std::vector<size_t> stage(D.layers);
     for (int l = 0; l < D.layers; ++l) {
@@ -434,6 +434,7 @@ int build_model(nh_model* m, const nh::ArchiveSmall& sm) {
     m->head->m.out = D.out_rows;
     m->head->m.out_pad = (int)round_up(D.out_rows, nh::TILE_ROWS);
     m->head->d_codes = emb->d_codes;
+    m->head->d_w8 = emb->d_w8;
     m->head->d_norms = emb->d_norms;
     m->head->d_fsel = emb->d_fsel;
     m->head_bits = emb->m.bits;
@@ -614,14 +615,26 @@ int feed(nh_session* s, int t, int outputs, float* out, float* cells, hipStream_
         if (!cells || !last)
             NH_TRY(nh::fwd_layer(D, m->glob, S, last, nullptr, row0, rows, 0, m->head_bits, st), "head input");
         const bool logits = outputs == NH_OUT_LAST_LOGITS || outputs == NH_OUT_ALL_LOGITS;
-        for (int i = 0; i < rows && logits; ++i) {
+        if (logits) {
+            // every row's logits in one launch when they are asked for, else
+            // the last row's (head_logits: the decode combine either way)
+            const bool all = rows > 1 && out;
             nh_qact a = s->a_in;
-            a.d_xq += (size_t)i * Gd * nh::GROUP;
-            a.d_sx += (size_t)i * Gd;
-            float* y = (outputs == NH_OUT_ALL_LOGITS && out) ? out + (size_t)i * D.out_rows : S.logits;
-            NH_TRY(product(m->head, &a, 1, y, D.out_rows, nullptr, st), "head");
-            if (i == rows - 1 && y != S.logits)
-                NH_TRY(hipMemcpyAsync(S.logits, y, (size_t)D.out_rows * 4, hipMemcpyDeviceToDevice, st), "logits");
+            if (!all) {
+                a.d_xq += (size_t)(rows - 1) * Gd * nh::GROUP;
+                a.d_sx += (size_t)(rows - 1) * Gd;
+            }
+            float* y = (outputs == NH_OUT_ALL_LOGITS && out) ? out : S.logits;
+            if (all) {
+                a.rows = rows;
+                NH_TRY(nh::launch_gemm_decode(m->head, &a, y, D.out_rows, st), "head");
+            } else {
+                NH_TRY(product(m->head, &a, 1, y, D.out_rows, nullptr, st), "head");
+            }
+            if (y != S.logits)
+                NH_TRY(hipMemcpyAsync(S.logits, y + (size_t)(rows - 1) * D.out_rows, (size_t)D.out_rows * 4,
+                                      hipMemcpyDeviceToDevice, st),
+                       "logits");
         }
         if (out && !logits)
             NH_TRY(hipMemcpyAsync(out, S.hid, (size_t)rows * d * 4, hipMemcpyDeviceToDevice, st), "hidden");
