@@ -382,10 +382,8 @@ hipError_t fwd_engram_hist(const Dims& D, const Globals& G, const SessDev& S, in
 // handing it out.
 namespace {
 
-constexpr int BT_STRIDE = HADA_NB + 2;  // padded (even: 8-byte reads) row of a transposed mix8 output
-constexpr int MIX_T = 256;              // threads of one mix8 (a 2 x 2 output block each)
-constexpr int MIX_STEPS = 4;            // j steps per pipelined batch of a mix8 pass (one 16-byte factor read)
-constexpr int KP_PITCH = HADA_NB + 4;   // dwords per pair row of a staged factor (16-byte reads, 2-way banks)
+constexpr int MIX_T = 256;    // threads of one mix8: four wavefronts, a 16 x 16 tile of the output each
+constexpr int BT_PITCH = 36;  // floats per row of a first mix8's output (16-byte reads; rows 4 banks apart)
 // Transposed copies for the serial chains, so a chain lane reads its
 // operands as contiguous 16-byte vectors: a dot16 operand x[16 c + l] at
 // l * pitch + c (pitch TP_D for d-long vectors, TP_X for the 4 lanes);
@@ -404,8 +402,8 @@ struct LayerShared {
     union {
         struct {
             alignas(16) float A[HADA_N];
-            alignas(16) float B[HADA_NB * BT_STRIDE];
-            alignas(16) uint32_t kp[6][HADA_NB / 2 * KP_PITCH];  // Kronecker factors as f16 pairs, pair-major
+            alignas(16) float B[HADA_NB * BT_PITCH];
+            alignas(16) uint4 kf[6][HADA_N / 8];  // Kronecker factors as MFMA fragments (stage order)
         };
         alignas(16) float tX[16 * TP_X];
     };
@@ -459,76 +457,71 @@ __device__ __forceinline__ void chain_pipe_any(int nb, Load load, Chain chain) {
 }
 
 // mix8 (infer.rs:2343-2380), portable branch: out[r][c] =
-// sum_j ct[j][r] * rows[j][c], each output an fma chain from j = 0.  Thread
-// u < 256 computes the 2 x 2 block r = 2 (u / 16) + {0, 1}, c = 2 (u % 16) +
-// {0, 1}.  The factor operand is read from its pair-major f16 copy (kp[p]
-// [j] = the factor's elements [j][2p], [j][2p + 1], p = the thread's pair):
-// one 16-byte read per MIX_STEPS steps, beside one 8-byte read of the
-// vector operand per step, for four fmas a step.
-// Transposed (ct = a factor, rows = [32][32]): stored at out[c * BT_STRIDE + r].
-__device__ __forceinline__ void mix8_t(int u, const uint32_t* kp, const float* rows, float* out) {
-    const int r = (u >> 4) * 2, c = (u & 15) * 2;
-    const uint4* fr = reinterpret_cast<const uint4*>(kp + (u >> 4) * KP_PITCH);
-    float o00 = 0.0f, o01 = 0.0f, o10 = 0.0f, o11 = 0.0f;
-    struct Buf {
-        uint4 f;
-        float2 v[MIX_STEPS];
-    };
-    auto load = [&](Buf& d, int b) {
-        d.f = fr[b];
+// sum_j ct[j][r] * rows[j][c] over 32 x 32, each output an fma chain from
+// j = 0.  v_mfma_f32_16x16x4_f32 runs exactly that chain: its four products
+// of an output are added one after the other in k order with one rounding
+// each (on gfx950 bit-identical to the fmaf chain over random, wide-range,
+// signed-zero and subnormal operands, and over the reference's results in
+// the forward tests), so eight of them in j order are the reference's 32
+// steps.  Four wavefronts take a 16 x 16 tile of the output each.  A pass is
+// one chain of eight dependent MFMAs (34 cycles each) between two LDS round
+// trips, and a lane reads 8 + 8 operands for its 4 outputs; the same chains
+// on the vector ALU (2 x 2 outputs a thread, 64 + 64 operands read for 4
+// outputs) were bound by LDS bandwidth.  With cond_weights' conversions apart
+// from its chain: 32 greedy tokens after a 118-token prompt 16.93 -> 16.58
+// ms, a 512-token prefill 1.328 -> 1.313 ms.
+//
+// Lane (q, i) = (lane / 16, lane % 16) supplies factor element [4 s + q][16 tile + i]
+// of step s, f16 in the staged fragment order: kf[tile * 64 + lane] holds
+// s = 0..7 (the same element as operand A of the transposed pass, where
+// the tile is the output's row block, and as operand B of the plain one,
+// where it is its column block), and gets out[4 q + v][i] of its tile.
+__device__ __forceinline__ f32x4 mix_chain(const uint4& f, const float (&x)[8], bool factor_rows) {
+    const uint32_t fw[4] = {f.x, f.y, f.z, f.w};
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int i = 0; i < MIX_STEPS; ++i)
-            d.v[i] = *reinterpret_cast<const float2*>(rows + (b * MIX_STEPS + i) * HADA_NB + c);
-    };
-    auto chain = [&](const Buf& d, int) {
-        const uint32_t fw[4] = {d.f.x, d.f.y, d.f.z, d.f.w};
-#pragma unroll
-        for (int i = 0; i < MIX_STEPS; ++i) {
-            const float ax = h2f((uint16_t)(fw[i] & 0xffffu)), ay = h2f((uint16_t)(fw[i] >> 16));
-            const float2 b = d.v[i];
-            o00 = __builtin_fmaf(ax, b.x, o00);
-            o01 = __builtin_fmaf(ax, b.y, o01);
-            o10 = __builtin_fmaf(ay, b.x, o10);
-            o11 = __builtin_fmaf(ay, b.y, o11);
-        }
-    };
-    chain_pipe_n<HADA_NB / MIX_STEPS, 3, Buf>(load, chain);
-    *reinterpret_cast<float2*>(out + c * BT_STRIDE + r) = make_float2(o00, o10);
-    *reinterpret_cast<float2*>(out + (c + 1) * BT_STRIDE + r) = make_float2(o01, o11);
+    for (int s = 0; s < 8; ++s) {
+        const float k = h2f((uint16_t)(fw[s >> 1] >> (16 * (s & 1))));
+        acc = factor_rows ? __builtin_amdgcn_mfma_f32_16x16x4f32(k, x[s], acc, 0, 0, 0)
+                          : __builtin_amdgcn_mfma_f32_16x16x4f32(x[s], k, acc, 0, 0, 0);
+    }
+    return acc;
 }
 
-// Plain (ct = the output of mix8_t, rows = a factor): out[r][c], rows
-// r < rows_limit (a multiple of 2).
-__device__ __forceinline__ void mix8_n(int u, const float* ct, const uint32_t* kp, float* out, int rows_limit) {
-    const int r = (u >> 4) * 2, c = (u & 15) * 2;
-    if (r >= rows_limit) return;
-    const uint4* fr = reinterpret_cast<const uint4*>(kp + (u & 15) * KP_PITCH);
-    float o00 = 0.0f, o01 = 0.0f, o10 = 0.0f, o11 = 0.0f;
-    struct Buf {
-        uint4 f;
-        float2 v[MIX_STEPS];
-    };
-    auto load = [&](Buf& d, int b) {
-        d.f = fr[b];
+// Element t (row j = t / 32, column c = t % 32) of the transposed pass's
+// vector operand, column block major: a wavefront's reads of four rows x 16
+// columns are 64 consecutive floats.
+__device__ __forceinline__ int mix_in(int t) { return ((t >> 4) & 1) * (HADA_N / 2) + (t >> 5) * 16 + (t & 15); }
+
+// Transposed (ct = a factor, rows = the vector operand in mix_in order):
+// out[r][c] at out[r * BT_PITCH + 8 (c % 4) + c / 4], so that a lane of the
+// plain pass reads its eight k elements as two 16-byte vectors.
+__device__ __forceinline__ void mix8_t(int u, const uint4* kf, const float* rows, float* out) {
+    const int lane = u & 63, q = lane >> 4, i = lane & 15, rt = (u >> 6) & 1, ct = u >> 7;
+    const uint4 f = kf[rt * 64 + lane];
+    float x[8];
 #pragma unroll
-        for (int i = 0; i < MIX_STEPS; ++i)
-            d.v[i] = *reinterpret_cast<const float2*>(ct + (b * MIX_STEPS + i) * BT_STRIDE + r);
-    };
-    auto chain = [&](const Buf& d, int) {
-        const uint32_t fw[4] = {d.f.x, d.f.y, d.f.z, d.f.w};
+    for (int s = 0; s < 8; ++s) x[s] = rows[ct * (HADA_N / 2) + s * 64 + lane];
+    const f32x4 o = mix_chain(f, x, true);
+    const int c = ct * 16 + i;
 #pragma unroll
-        for (int i = 0; i < MIX_STEPS; ++i) {
-            const float2 a = d.v[i];
-            const float bx = h2f((uint16_t)(fw[i] & 0xffffu)), by = h2f((uint16_t)(fw[i] >> 16));
-            o00 = __builtin_fmaf(a.x, bx, o00);
-            o01 = __builtin_fmaf(a.x, by, o01);
-            o10 = __builtin_fmaf(a.y, bx, o10);
-            o11 = __builtin_fmaf(a.y, by, o11);
-        }
-    };
-    chain_pipe_n<HADA_NB / MIX_STEPS, 3, Buf>(load, chain);
-    *reinterpret_cast<float2*>(out + r * HADA_NB + c) = make_float2(o00, o01);
-    *reinterpret_cast<float2*>(out + (r + 1) * HADA_NB + c) = make_float2(o10, o11);
+    for (int v = 0; v < 4; ++v) out[(rt * 16 + 4 * q + v) * BT_PITCH + (c & 3) * 8 + (c >> 2)] = o[v];
+}
+
+// Plain (ct = the output of mix8_t, rows = a factor): out[r][c] row-major,
+// rows r < rows_limit (a multiple of 8).
+__device__ __forceinline__ void mix8_n(int u, const float* ct, const uint4* kf, float* out, int rows_limit) {
+    const int lane = u & 63, q = lane >> 4, i = lane & 15, rt = (u >> 6) & 1, cb = u >> 7;
+    const uint4 f = kf[cb * 64 + lane];
+    const float4* xr = reinterpret_cast<const float4*>(ct + (rt * 16 + i) * BT_PITCH + q * 8);
+    const float4 x0 = xr[0], x1 = xr[1];
+    const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+    const f32x4 o = mix_chain(f, x, false);
+    const int r = rt * 16 + 4 * q;
+    if (r < rows_limit) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) out[(r + v) * HADA_NB + cb * 16 + i] = o[v];
+    }
 }
 
 // Element i of a dot16 operand into its transposed copy.
@@ -722,12 +715,7 @@ __device__ __forceinline__ void store_out(int d, const OutRegs& q, LayerShared& 
     for (int r = 0; r < STAGE_PER; ++r) {
         const int e = t + r * LT;
         if (e < kron_n) {
-            // 8 f16 of factor row j: pairs 4 (e % 4) + k, stored pair-major
-            const int i = e / (HADA_N / 8), ee = e % (HADA_N / 8), j = ee >> 2, p0 = (ee & 3) * 4;
-            const uint4 v = q.st[r];
-            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int k = 0; k < 4; ++k) sh.kp[i][(p0 + k) * KP_PITCH + j] = w[k];
+            (&sh.kf[0][0])[e] = q.st[r];  // (already in fragment order)
         } else if (e < kron_n + cv_n) {
             // row j of cond_v (8 f16) into column j / 4 of rows 8 (j % 4) + k
             const int j = e - kron_n;
@@ -769,11 +757,16 @@ __device__ __forceinline__ void cond_weights(const LayerShared& sh, int d, int l
         auto chain = [&](const Buf& d) {
             const float hv[8] = {d.h[0].x, d.h[0].y, d.h[0].z, d.h[0].w, d.h[1].x, d.h[1].y, d.h[1].z, d.h[1].w};
             const uint32_t cw[4] = {d.c.x, d.c.y, d.c.z, d.c.w};
+            // (converted apart from the chain: folded into the fmas, the
+            // conversions make every dependent step a slower mixed one)
+            float cv[8];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                a = __builtin_fmaf(hv[2 * u], h2f((uint16_t)(cw[u] & 0xffffu)), a);
-                a = __builtin_fmaf(hv[2 * u + 1], h2f((uint16_t)(cw[u] >> 16)), a);
+            for (int u = 0; u < 8; ++u) {
+                cv[u] = h2f((uint16_t)(cw[u >> 1] >> (16 * (u & 1))));
+                asm("" : "+v"(cv[u]));
             }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) a = __builtin_fmaf(hv[u], cv[u], a);
         };
         if (nb > 0) chain_pipe_any<3, Buf>(nb, load, chain);
         for (int u = nb * 8; u < steps; ++u)
@@ -827,7 +820,7 @@ __device__ float layer_out(const Dims& D, const SessDev& S, const LayerDev& P, c
             h2 = __builtin_fmaf(tt, h2f_late(q.ph), tt);
             sh.hT[(t & 3) * TP_H + (t >> 2)] = h2;
         }
-        sh.A[t] = t < d ? h2 * h2f_late(q.d1) : 0.0f;
+        sh.A[mix_in(t)] = t < d ? h2 * h2f_late(q.d1) : 0.0f;
     }
     __syncthreads();
     // cond_weights (wavefront 0) spans both passes of the first mix8; the
@@ -835,9 +828,9 @@ __device__ float layer_out(const Dims& D, const SessDev& S, const LayerDev& P, c
     before_mix();
     if (wave == 0) cond_weights(sh, d, lane, sh.wk);
     if (mixer) {
-        mix8_t(mu, sh.kp[0], sh.A, sh.B);
+        mix8_t(mu, sh.kf[0], sh.A, sh.B);
         mixer_sync(&sh.mix_count, MIX_T / 64, D.spin_limit, S.status);
-        mix8_n(mu, sh.B, sh.kp[1], sh.C, HADA_NB);
+        mix8_n(mu, sh.B, sh.kf[1], sh.C, HADA_NB);
     }
     __syncthreads();
     {
@@ -848,18 +841,18 @@ __device__ float layer_out(const Dims& D, const SessDev& S, const LayerDev& P, c
             cond = __builtin_fmaf(h2f((uint16_t)(cw[k >> 1] >> (16 * (k & 1)))), sh.wk[k], cond);
         float zs = __builtin_fmaf(sh.C[q.p1], cond * h2f_late(q.d2), h2f_late(q.b2));
         zs = zs / (nexp(-zs) + 1.0f);
-        sh.A[t] = zs;
+        sh.A[mix_in(t)] = zs;
     }
     __syncthreads();
-    if (mixer) mix8_t(mu, sh.kp[2], sh.A, sh.B);
+    if (mixer) mix8_t(mu, sh.kf[2], sh.A, sh.B);
     __syncthreads();
-    if (mixer) mix8_n(mu, sh.B, sh.kp[3], sh.C, HADA_NB);
+    if (mixer) mix8_n(mu, sh.B, sh.kf[3], sh.C, HADA_NB);
     __syncthreads();
-    sh.A[t] = sh.C[q.p2] * h2f_late(q.d3);
+    sh.A[mix_in(t)] = sh.C[q.p2] * h2f_late(q.d3);
     __syncthreads();
-    if (mixer) mix8_t(mu, sh.kp[4], sh.A, sh.B);
+    if (mixer) mix8_t(mu, sh.kf[4], sh.A, sh.B);
     __syncthreads();
-    if (mixer) mix8_n(mu, sh.B, sh.kp[5], sh.C, d / HADA_NB / 8 * 8);
+    if (mixer) mix8_n(mu, sh.B, sh.kf[5], sh.C, d / HADA_NB / 8 * 8);
     __syncthreads();
     after_mlp();
     // The mHC write: y = (x2 + t3 * d4) - u; lane a = y hpost[a] + sum_b

@@ -322,7 +322,12 @@ int build_model(nh_model* m, const nh::ArchiveSmall& sm) {
         std::vector<float> blk;
         for (int k = 0; k < 6; ++k) {
             const auto& f = sm.layer[l][nh::S_KRON0 + k];
-            blk.insert(blk.end(), f.begin(), f.begin() + nh::HADA_N);
+            // (in the order the mix8 MFMAs read them: 16-wide column tile,
+            // lane 16 q + i, step s holds row 4 s + q, column i of the tile)
+            for (int tile = 0; tile < 2; ++tile)
+                for (int lane = 0; lane < 64; ++lane)
+                    for (int st = 0; st < 8; ++st)
+                        blk.push_back(f[(4 * st + lane / 16) * nh::HADA_NB + tile * 16 + lane % 16]);
         }
         const auto& cv = sm.layer[l][nh::S_COND_V];
         blk.insert(blk.end(), cv.begin(), cv.begin() + (size_t)D.d * nh::COND_RANK);
