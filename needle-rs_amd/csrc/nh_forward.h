@@ -47,7 +47,9 @@ struct Dims {
     int sites, ntab, eheads, seed_stride, slots, sub, dilation;
     int orders[4];
     int cap;    // session positions
-    int vcap;   // row stride of the transposed int8 values: cap + 4 rounded up to 16
+    int kslots; // KV slots of a layer: a slot per position, then from stage0 on one per row of a feed
+    int stage0; // cap rounded up to 16
+    int vcap;   // row stride of the transposed int8 values: kslots + 4 rounded up to 16
     int max_chunks;  // attention chunks a position can need
     int spin_limit;  // polls of an in-kernel wait before it gives up (SPIN_LIMIT)
     // per-feed state, set by the host before each feed
@@ -55,6 +57,8 @@ struct Dims {
                      // crates/needle-engine/src/infer.rs:968-980): older rows read as zero
     int rope_prev;   // 1: a single token right after the newest RoPE row (the recurrence)
     int sink, ring;  // Session::attend (model.rs:62-66); ring 0: no span
+    int staged;      // 1: a feed under a span whose keys and values go to the staging slots (row i at
+                     // stage0 + i) until its attention has read the ring's old ones (staged_range)
 };
 
 // The keys an attention span leaves a feed (key_ranges,
@@ -116,10 +120,10 @@ struct SessDev {
     float* pm;        // [rows][nh][max_chunks]
     float* psum;      // [rows][nh][max_chunks]
     float* hist;      // [layers][hist_slots][W] ring of pre-tap rows
-    int8_t* k8;       // [layers][cap][nkv][qk]
-    float* ks;        // [layers][cap][nkv]
+    int8_t* k8;       // [layers][kslots][nkv][qk]
+    float* ks;        // [layers][kslots][nkv]
     int8_t* v8t;      // [layers][nkv][vd][vcap]
-    float* vs;        // [layers][cap][nkv]
+    float* vs;        // [layers][kslots][nkv]
     int8_t* ev8;      // [sites][cap][d]
     float* evs;       // [sites][cap][d / 32]
     int8_t* xq_in;    // [ACT_ROWS][G(d)][128] the layer inputs (K = d)
@@ -171,7 +175,10 @@ hipError_t fwd_engram_hist(const Dims& D, const Globals& G, const SessDev& S, in
 hipError_t fwd_layer(const Dims& D, const Globals& G, const SessDev& S, const LayerDev* prev, const LayerDev* next,
                      int row0, int rows, int in_bits, int head_bits, hipStream_t s, int head_row0 = 0);
 hipError_t fwd_units(const Dims& D, const SessDev& S, const LayerDev& L, int layer, int p0, int t, hipStream_t s);
-// `span`: the keys of a session with an attention span (null: none).
+// Whether a feed under an attention span can take the staged form (D.staged):
+// the geometry of the grouped attention kernel.
+bool attend_staged_fits(const Dims& D, const LayerDev& L);
+// `span`: the keys of a session with an attention span (null: none, or staged).
 hipError_t fwd_attend(const Dims& D, const SessDev& S, const LayerDev& L, int layer, int p0, int t,
                       const KeySpan* span, hipStream_t s);
 // Also writes the tap history of a feed of several chunks (there the units

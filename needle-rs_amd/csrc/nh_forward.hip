@@ -1471,12 +1471,12 @@ __global__ __launch_bounds__(MAX_UNITS * 64) void k_units(Dims D, SessDev S, Lay
     } else {
         const float s = wave_quant_scale(i < len ? v : 0.0f);
         const int8_t q = quant_one(v, 1.0f / s);
-        const size_t lc = (size_t)layer * D.cap;
-        const int slot = slot_of(D, pos);
+        const size_t lc = (size_t)layer * D.kslots;
+        const int slot = D.staged ? D.stage0 + row : slot_of(D, pos);
         // A ring shorter than the feed gives two of its rows one slot: the
         // later position keeps it (the slot map says so; the reference's
         // members would race there).
-        const bool taken = D.ring > 0 && pos >= D.sink && pos + D.ring < p0 + t;
+        const bool taken = !D.staged && D.ring > 0 && pos >= D.sink && pos + D.ring < p0 + t;
         if (taken) return;
         if (unit < nh + nkv) {
             const int kh = unit - nh;
@@ -1572,6 +1572,55 @@ __device__ __forceinline__ int key_count(const Dims& D, const KeySpan& K, bool s
     return span_count(K, alo, ahi, blo, bhi);
 }
 
+// A staged feed's row (rows p0 .. p0 + rows - 1, row's window starts at lo):
+// its chunk's key ranges [lo, ahi) and [blo, pos + 1), every position of
+// them live; returns the number of keys.
+__host__ __device__ inline int staged_range(const Dims& D, int p0, int rows, int row, int lo, int& ahi, int& blo) {
+    const int pos = p0 + row, end = p0 + min(rows, (row / FWD_ROWS + 1) * FWD_ROWS);
+    ahi = max(lo, min(D.sink, pos + 1));
+    blo = min(max(end - D.ring, D.sink), pos + 1);
+    return ahi - lo + pos + 1 - blo;
+}
+
+// Keys k0 .. k1 - 1 of such a row as runs of consecutive slots in key order:
+// run r starts at key key[r] (past k0) in slot slot[r], its value columns at
+// col[r], a multiple of 16 (column col[r] + slot[r] % 16 for its first key);
+// cols columns in all.  Runs past the last start past every key.
+constexpr int AG_RUNS = 4;
+struct StagedRuns {
+    int key[AG_RUNS], slot[AG_RUNS], col[AG_RUNS], cols;
+};
+__host__ __device__ inline void staged_runs(const Dims& D, int p0, int pos, int lo, int ahi, int blo, int k0, int k1,
+                                            StagedRuns& R) {
+    int k = 0, ns = 0, c = 0;
+    auto run = [&](int a, int b, int slot) {  // positions a .. b - 1 from `slot` on
+        const int from = max(k, k0), to = min(k + b - a, k1);
+        if (b > a && from < to) {
+            R.key[ns] = from - k0;
+            R.slot[ns] = slot + from - k;
+            R.col[ns] = c;
+            c += ((R.slot[ns] & 15) + to - from + 15) & ~15;
+            ++ns;
+        }
+        k += max(b - a, 0);
+    };
+    // the sink's older positions, the feed's; the ring's older ones (cut
+    // where it wraps), the feed's
+    run(lo, min(ahi, p0), lo);
+    run(max(lo, p0), ahi, D.stage0 + max(lo, p0) - p0);
+    const int old = min(pos + 1, p0), s0 = D.sink + max(blo - D.sink, 0) % D.ring;
+    const int wrap = min(max(old, blo), blo + D.sink + D.ring - s0);
+    run(blo, wrap, s0);
+    run(wrap, old, D.sink);
+    run(max(blo, p0), pos + 1, D.stage0 + max(blo, p0) - p0);
+    R.cols = c;
+    for (; ns < AG_RUNS; ++ns) {
+        R.key[ns] = ATT_CHUNK_MAX;
+        R.slot[ns] = 0;
+        R.col[ns] = c;
+    }
+}
+
 constexpr int ATT_KPITCH = MAX_HEAD_DIM + 16;        // key row (80 bytes: 8 rows cover the 32 banks)
 constexpr int ATT_PITCH = ATT_CHUNK_MAX + 8;         // value / digit row: 3 alignment bytes + 256 keys + tail
 constexpr int ATT_VDW = (ATT_CHUNK_MAX + 3 + 3) / 4; // value dwords per column
@@ -1609,7 +1658,7 @@ __global__ __launch_bounds__(ATT_THREADS) void k_attend(Dims D, SessDev S, Layer
     __shared__ float red[ATT_THREADS / 64];
     __shared__ float s_qs, s_sum;
     __shared__ int kslot[SPAN ? ATT_CHUNK_MAX : 1];
-    const size_t lc = (size_t)layer * D.cap;
+    const size_t lc = (size_t)layer * D.kslots;
     // every load first (unconditional, at clamped in-range addresses)
     const float qv = S.qbuf[((size_t)row * D.nh + hh) * qk + min(lane, qk - 1)];
     constexpr int KR = ATT_CHUNK_MAX * 4 / ATT_THREADS, VR = (MAX_HEAD_DIM * ATT_VDW + ATT_THREADS - 1) / ATT_THREADS;
@@ -1844,9 +1893,21 @@ __device__ __forceinline__ void wave_lds_sync() {
 // Between them wavefront h runs query head h's float steps as the reference
 // orders them: the chunk max, chunk_exp with its sum order (lanes 0-7 run
 // the eight lane-class chains), the weights and the 21-bit digits.
+//
+// SPAN: a staged feed under an attention span.  A row's keys are its chunk's
+// two position ranges (staged_range), older positions in their ring slots and
+// the feed's own in the staging slots: at most four runs of consecutive
+// slots in key order (the sink's; the ring's older ones, cut where the ring
+// wraps; the feed's; or the sink's older and newer parts and the feed's
+// others).  Each run's value columns are staged from its first slot rounded
+// down to 16 at a column of its own, a multiple of 16, so the loads stay
+// whole 16-byte chunks; the digits between the runs are zero.  (The general
+// kernel gathers the values byte by byte, per query head.)
 constexpr int AG_WAVES = 8;   // query heads per kv head this kernel takes
 constexpr int AG_T = AG_WAVES * 64;
-constexpr int AG_COLS = 320;  // value / digit columns: 15 alignment + 256 keys, in whole 64-column steps
+// value / digit columns: 15 alignment + 256 keys, in whole 64-column steps;
+// four runs: 256 keys + 4 x (15 alignment + 15 rounding)
+constexpr int AG_COLS_1 = 320, AG_COLS_4 = 384;
 constexpr int AG_KPL = ATT_CHUNK_MAX / 64;  // keys per lane in the head steps
 constexpr int AG_TP = ATT_CHUNK_MAX / 8 + 4;  // a lane class's exps (16-byte rows, room for the trailing 4-block)
 
@@ -1856,7 +1917,7 @@ constexpr int AG_TP = ATT_CHUNK_MAX / 8 + 4;  // a lane class's exps (16-byte ro
 // (threads rr * 512 ...) run its scores, head steps and P.V over its own
 // keys, a prefix of the staged ones; a feed with an odd count of rows
 // leaves the last workgroup's second row empty.
-template <int RP>
+template <int RP, bool SPAN>
 __global__ __launch_bounds__(AG_T * RP) __attribute__((amdgpu_waves_per_eu(RP == 2 ? 8 : 1))) void k_attend_group(
     const float* qbuf, const int8_t* k8l, const float* ksl, const float* vsl, const int8_t* v8l, int p0, int rows,
     int wv, int geom, Dims D, SessDev S, LayerDev L, int layer) {
@@ -1867,7 +1928,7 @@ __global__ __launch_bounds__(AG_T * RP) __attribute__((amdgpu_waves_per_eu(RP ==
     // argument segment)
     const int g_nh = geom & 255, g_nkv = (geom >> 8) & 255, g_qk = (geom >> 16) & 255,
               g_vd = (int)((unsigned)geom >> 24), window = wv & 0xffff, vcap = (int)((unsigned)wv >> 16);
-    constexpr int NTT = AG_T * RP;
+    constexpr int NTT = AG_T * RP, AG_COLS = SPAN ? AG_COLS_4 : AG_COLS_1;
     // (the row half and the wavefront are wave-uniform: in scalar registers,
     // so the lengths and bounds derived from them are too)
     const int tb = threadIdx.x, rr = __builtin_amdgcn_readfirstlane(tb / AG_T), t = tb % AG_T;
@@ -1878,24 +1939,33 @@ __global__ __launch_bounds__(AG_T * RP) __attribute__((amdgpu_waves_per_eu(RP ==
     // longest rows first; the staged range is row A's (the block's rows
     // share lo and the chunking).
     __shared__ int prm[6];
+    __shared__ StagedRuns runs;
     if (tb < 64) {
         const int pr = (int)blockIdx.x / g_nkv, rA = rows - 1 - RP * pr, pA = p0 + rA;
         const int l0 = window_lo(window, pA);
-        int cnt, chk;
-        key_chunks(pA + 1 - l0, g_nkv, rows > 1, cnt, chk);
+        int cnt, chk, nk = pA + 1 - l0, ahi = 0, blo = 0;
+        if constexpr (SPAN) nk = staged_range(D, p0, rows, rA, l0, ahi, blo);
+        key_chunks(nk, g_nkv, rows > 1, cnt, chk);
+        if constexpr (SPAN) {
+            if (tb == 0) {
+                const int k0 = (int)blockIdx.y * chk;
+                staged_runs(D, p0, pA, l0, ahi, blo, k0, min(k0 + chk, nk), runs);
+            }
+        }
         if (tb == 0) {
             prm[0] = rA;
             prm[1] = (int)blockIdx.x - pr * g_nkv;
             prm[2] = l0;
             prm[3] = cnt;
             prm[4] = chk;
-            prm[5] = g_nh / g_nkv;
+            prm[5] = SPAN ? nk : g_nh / g_nkv;
         }
     }
     __syncthreads();
     const int rowA = __builtin_amdgcn_readfirstlane(prm[0]), kvh = __builtin_amdgcn_readfirstlane(prm[1]);
     const int lo = __builtin_amdgcn_readfirstlane(prm[2]), count = __builtin_amdgcn_readfirstlane(prm[3]);
-    const int chunk = __builtin_amdgcn_readfirstlane(prm[4]), hpg = __builtin_amdgcn_readfirstlane(prm[5]);
+    const int chunk = __builtin_amdgcn_readfirstlane(prm[4]), prm5 = __builtin_amdgcn_readfirstlane(prm[5]);
+    const int hpg = SPAN ? g_nh / g_nkv : prm5;
     const int ci = blockIdx.y;
     if (ci >= count) return;
     const int row = rowA - rr;
@@ -1903,12 +1973,44 @@ __global__ __launch_bounds__(AG_T * RP) __attribute__((amdgpu_waves_per_eu(RP ==
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, posA = p0 + rowA,
               pos = p0 + (live ? row : 0);
     const int nkv = g_nkv, qk = g_qk, vd = g_vd;
-    const int nA = posA + 1 - lo, n = pos + 1 - lo;
-    const int c0 = ci * chunk, lenA = min(chunk, nA - c0), slot0 = lo + c0;
+    // (SPAN: the earlier row's keys are the later one's without its last rr)
+    const int nA = SPAN ? prm5 : posA + 1 - lo, n = SPAN ? prm5 - rr : pos + 1 - lo;
+    const int c0 = ci * chunk, lenA = min(chunk, nA - c0), slot0 = SPAN ? 0 : lo + c0;
     const int len = live ? min(chunk, n - c0) : 0, blocked = len / 4 * 4;
     // value columns and digits from slot base = slot0 rounded down to 16
     // bytes (column j = key + sh)
-    const int sh = slot0 & 15, base = slot0 - sh, colsA = sh + lenA, cols = sh + len;
+    const int sh = slot0 & 15, base = slot0 - sh;
+    int rk[AG_RUNS] = {}, rs[AG_RUNS] = {}, rc[AG_RUNS] = {};
+    if constexpr (SPAN) {
+#pragma unroll
+        for (int r = 0; r < AG_RUNS; ++r) {
+            rk[r] = __builtin_amdgcn_readfirstlane(runs.key[r]);
+            rs[r] = __builtin_amdgcn_readfirstlane(runs.slot[r]);
+            rc[r] = __builtin_amdgcn_readfirstlane(runs.col[r]);
+        }
+    }
+    const int colsA = SPAN ? __builtin_amdgcn_readfirstlane(runs.cols) : sh + lenA, cols = SPAN ? colsA : sh + len;
+    // key i's slot (past slot0) and value / digit column
+    auto key_slot = [&](int i) __attribute__((always_inline)) {
+        if constexpr (!SPAN) return i;
+        return i + (i < rk[1] ? rs[0] - rk[0] : i < rk[2] ? rs[1] - rk[1] : i < rk[3] ? rs[2] - rk[2] : rs[3] - rk[3]);
+    };
+    auto key_col = [&](int i) __attribute__((always_inline)) {
+        if constexpr (!SPAN) return sh + i;
+        return i + (i < rk[1]   ? rc[0] + (rs[0] & 15) - rk[0]
+                    : i < rk[2] ? rc[1] + (rs[1] & 15) - rk[1]
+                    : i < rk[3] ? rc[2] + (rs[2] & 15) - rk[2]
+                                : rc[3] + (rs[3] & 15) - rk[3]);
+    };
+    // the first slot (past base) of 16-byte value chunk k
+    auto chunk_slot = [&](int k) __attribute__((always_inline)) {
+        if constexpr (!SPAN) return k * 16;
+        const int c = k * 16;
+        return c + (c < rc[1]   ? (rs[0] & ~15) - rc[0]
+                    : c < rc[2] ? (rs[1] & ~15) - rc[1]
+                    : c < rc[3] ? (rs[2] & ~15) - rc[2]
+                                : (rs[3] & ~15) - rc[3]);
+    };
     __shared__ alignas(16) int8_t vs8[MAX_HEAD_DIM][AG_COLS];
     __shared__ float kss[ATT_CHUNK_MAX], vss[ATT_CHUNK_MAX];
     __shared__ alignas(16) int8_t q8s[RP][AG_WAVES][MAX_HEAD_DIM];
@@ -1938,27 +2040,27 @@ __global__ __launch_bounds__(AG_T * RP) __attribute__((amdgpu_waves_per_eu(RP ==
     const int rq = qk / 16, vq = (colsA + 15) / 16;
     // buffer resources over the chunk's key rows (this kv head's, from
     // slot0), their scales and the value columns (from base)
-    const int kstride = nkv * qk;
-    const __amdgpu_buffer_rsrc_t rk = make_rsrc(k8l + (size_t)slot0 * kstride + kvh * qk, (size_t)lenA * kstride);
-    const __amdgpu_buffer_rsrc_t rks = make_rsrc(ksl + (size_t)slot0 * nkv + kvh, (size_t)lenA * nkv * 4);
-    const __amdgpu_buffer_rsrc_t rvs = make_rsrc(vsl + (size_t)slot0 * nkv + kvh, (size_t)lenA * nkv * 4);
+    const int kstride = nkv * qk, nslots = SPAN ? D.kslots : lenA;
+    const __amdgpu_buffer_rsrc_t rkb = make_rsrc(k8l + (size_t)slot0 * kstride + kvh * qk, (size_t)nslots * kstride);
+    const __amdgpu_buffer_rsrc_t rks = make_rsrc(ksl + (size_t)slot0 * nkv + kvh, (size_t)nslots * nkv * 4);
+    const __amdgpu_buffer_rsrc_t rvs = make_rsrc(vsl + (size_t)slot0 * nkv + kvh, (size_t)nslots * nkv * 4);
     const __amdgpu_buffer_rsrc_t rv = make_rsrc(v8l + (size_t)kvh * vd * vcap + base, (size_t)vd * vcap);
     u32x4 kr[KR], vw[VR];
 #pragma unroll
     for (int r = 0; r < KR; ++r) {
         const int e = tb + r * NTT, i = min(e >> 2, lenA - 1), c = min(e & 3, rq - 1);
-        kr[r] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, __mul24(i, kstride) + c * 16, 0, 0));
+        kr[r] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rkb, __mul24(key_slot(i), kstride) + c * 16, 0, 0));
     }
     float ksr, vsr;
     {
-        const int i = min(tb, lenA - 1);
+        const int i = key_slot(min(tb, lenA - 1));
         ksr = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rks, __mul24(i, nkv) * 4, 0, 0));
         vsr = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rvs, __mul24(i, nkv) * 4, 0, 0));
     }
 #pragma unroll
     for (int r = 0; r < VR; ++r) {
         const int e = tb + r * NTT, dm = min(e / VQ, vd - 1), k = min(e % VQ, vq - 1);
-        vw[r] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, __mul24(dm, vcap) + k * 16, 0, 0));
+        vw[r] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, __mul24(dm, vcap) + chunk_slot(k), 0, 0));
     }
     // the int8 query of this wavefront's head, zero past qk (the key rows'
     // bytes there are not staged)
@@ -2092,20 +2194,29 @@ __global__ __launch_bounds__(AG_T * RP) __attribute__((amdgpu_waves_per_eu(RP ==
         wmax = wave_max_nonneg(wmax);
         const float qwt = bits_f32(0x49fffff8u) / wmax;
         int8_t(*dg)[AG_COLS] = dig[wave];
+        if constexpr (SPAN) {
+            // zero digits everywhere first (a wavefront's LDS writes land in order)
+            for (int j = lane; j < (cols + 63) / 64 * 16; j += 64)
+                reinterpret_cast<int*>(dg[0])[j] = reinterpret_cast<int*>(dg[1])[j] = reinterpret_cast<int*>(dg[2])[j] = 0;
+            wave_lds_sync();
+        }
 #pragma unroll
         for (int j = 0; j < AG_KPL; ++j) {
             const int i = lane + 64 * j;
             if (i < len) {
                 const int32_t wq = (int32_t)roundf(e[j] * qwt);
-                dg[0][sh + i] = (int8_t)(wq >> 14);
-                dg[1][sh + i] = (int8_t)((wq >> 7) & 127);
-                dg[2][sh + i] = (int8_t)(wq & 127);
+                const int c = key_col(i);
+                dg[0][c] = (int8_t)(wq >> 14);
+                dg[1][c] = (int8_t)((wq >> 7) & 127);
+                dg[2][c] = (int8_t)(wq & 127);
             }
         }
-        // zero digits before the keys and from their end to the last step's
-        if (lane < sh) dg[0][lane] = dg[1][lane] = dg[2][lane] = 0;
-        const int j1 = cols + lane;
-        if (j1 < (cols + 63) / 64 * 64) dg[0][j1] = dg[1][j1] = dg[2][j1] = 0;
+        if constexpr (!SPAN) {
+            // zero digits before the keys and from their end to the last step's
+            if (lane < sh) dg[0][lane] = dg[1][lane] = dg[2][lane] = 0;
+            const int j1 = cols + lane;
+            if (j1 < (cols + 63) / 64 * 64) dg[0][j1] = dg[1][j1] = dg[2][j1] = 0;
+        }
         cw = wmax * bits_f32(0x35000004u);
     }
     __syncthreads();
@@ -2144,44 +2255,58 @@ __global__ __launch_bounds__(AG_T * RP) __attribute__((amdgpu_waves_per_eu(RP ==
     }
 }
 
+// The geometry k_attend_group takes (its packed arguments).
+static bool attend_group_fits(const Dims& D, const LayerDev& L) {
+    return D.nh / D.nkv <= AG_WAVES && D.nh < 256 && D.nkv < 256 && D.qk < 256 && D.vd < 256 && L.window >= 0 &&
+           L.window < 65536 && D.vcap < 65536;
+}
+
+bool attend_staged_fits(const Dims& D, const LayerDev& L) { return attend_group_fits(D, L); }
+
 hipError_t fwd_attend(const Dims& D, const SessDev& S, const LayerDev& L, int layer, int p0, int t,
                       const KeySpan* span, hipStream_t s) {
     if (span)
         hipLaunchKernelGGL(k_attend<true>, dim3(t * D.nh, D.max_chunks), dim3(ATT_THREADS), 0, s, D, S, L, layer, p0,
                            t, *span);
-    else if (D.nh / D.nkv <= AG_WAVES && D.nh < 256 && D.nkv < 256 && D.qk < 256 && D.vd < 256 &&
-             L.window >= 0 && L.window < 65536 && D.vcap < 65536) {
+    else if (attend_group_fits(D, L)) {
+        // row i's window start, first key past the sink's range (staged) and chunking
+        struct Row {
+            int lo, blo, count, chunk;
+        };
+        auto row = [&](int i) {
+            Row r{window_lo(L.window, p0 + i), 0, 0, 0};
+            int ahi, n = p0 + i + 1 - r.lo;
+            if (D.staged) n = staged_range(D, p0, t, i, r.lo, ahi, r.blo);
+            key_chunks(n, D.nkv, t > 1, r.count, r.chunk);
+            return r;
+        };
         // the most chunks a row of the feed needs
         int most = 1;
-        for (int i = 0; i < t; ++i) {
-            const int pos = p0 + i, n = pos + 1 - window_lo(L.window, pos);
-            int count, chunk;
-            key_chunks(n, D.nkv, t > 1, count, chunk);
-            most = count > most ? count : most;
-        }
+        for (int i = 0; i < t; ++i) most = std::max(most, row(i).count);
         // consecutive rows whose window start and chunking agree share a
         // workgroup (every pair of the feed, else none); rows of one chunk
-        // each agree whatever its length (the chunk is all their keys)
+        // each agree whatever its length (the chunk is all their keys);
+        // staged, the earlier row's keys must be the later one's but its last
         bool pairs = t > 1;
         for (int i = t - 1; i > 0 && pairs; i -= 2) {
-            const int pa = p0 + i, pb = pa - 1, la = window_lo(L.window, pa), lb = window_lo(L.window, pb);
-            int ca, sa, cb, sb;
-            key_chunks(pa + 1 - la, D.nkv, true, ca, sa);
-            key_chunks(pb + 1 - lb, D.nkv, true, cb, sb);
-            pairs = la == lb && ca == cb && (ca == 1 || sa == sb);
+            const Row a = row(i), b = row(i - 1);
+            pairs = a.lo == b.lo && a.count == b.count && (a.count == 1 || a.chunk == b.chunk);
+            if (D.staged) pairs = pairs && std::min(a.blo, p0 + i) == b.blo;
         }
-        const size_t lc = (size_t)layer * D.cap;
+        const size_t lc = (size_t)layer * D.kslots;
         const int8_t* k8l = S.k8 + lc * D.nkv * D.qk;
         const float* ksl = S.ks + lc * D.nkv;
         const float* vsl = S.vs + lc * D.nkv;
         const int8_t* v8l = S.v8t + (size_t)layer * D.nkv * D.vd * D.vcap;
         const int geom = D.nh | D.nkv << 8 | D.qk << 16 | D.vd << 24, wv = L.window | D.vcap << 16;
-        if (pairs)
-            hipLaunchKernelGGL(k_attend_group<2>, dim3((t + 1) / 2 * D.nkv, most), dim3(2 * AG_T), 0, s, S.qbuf, k8l,
-                               ksl, vsl, v8l, p0, t, wv, geom, D, S, L, layer);
+        auto go = [&](auto kern, int rp) {
+            hipLaunchKernelGGL(kern, dim3((t + rp - 1) / rp * D.nkv, most), dim3(rp * AG_T), 0, s, S.qbuf, k8l, ksl,
+                               vsl, v8l, p0, t, wv, geom, D, S, L, layer);
+        };
+        if (D.staged)
+            pairs ? go(k_attend_group<2, true>, 2) : go(k_attend_group<1, true>, 1);
         else
-            hipLaunchKernelGGL(k_attend_group<1>, dim3(t * D.nkv, most), dim3(AG_T), 0, s, S.qbuf, k8l, ksl, vsl,
-                               v8l, p0, t, wv, geom, D, S, L, layer);
+            pairs ? go(k_attend_group<2, false>, 2) : go(k_attend_group<1, false>, 1);
     }
     else
         hipLaunchKernelGGL(k_attend<false>, dim3(t * D.nh, D.max_chunks), dim3(ATT_THREADS), 0, s, D, S, L, layer,
@@ -2211,8 +2336,26 @@ __global__ __launch_bounds__(LT) void k_attn_out(Dims D, SessDev S, LayerDev L, 
         post_gates(S.p + (size_t)row * 64, L, lane);
         return;
     }
-    if (wave >= Ga) return;
-    const int n = key_count(D, KS, span != 0, L.window, pos);
+    if (wave >= Ga) {
+        // a staged feed's keys and values into their slots, now that every
+        // row has attended (a position whose slot a later row takes, not)
+        if (D.staged && (pos < D.sink || pos + D.ring >= p0 + rows)) {
+            const int slot = slot_of(D, pos), from = D.stage0 + row, nt = LT - 64 - Ga * 64, t0 = t - Ga * 64;
+            const size_t lc = (size_t)layer * D.kslots;
+            const int kq = D.nkv * D.qk;
+            for (int e = t0; e < kq; e += nt) S.k8[(lc + slot) * kq + e] = S.k8[(lc + from) * kq + e];
+            int8_t* v8 = S.v8t + (size_t)layer * D.nkv * vd * D.vcap;
+            for (int e = t0; e < D.nkv * vd; e += nt) v8[(size_t)e * D.vcap + slot] = v8[(size_t)e * D.vcap + from];
+            for (int e = t0; e < D.nkv; e += nt) {
+                S.ks[(lc + slot) * D.nkv + e] = S.ks[(lc + from) * D.nkv + e];
+                S.vs[(lc + slot) * D.nkv + e] = S.vs[(lc + from) * D.nkv + e];
+            }
+        }
+        return;
+    }
+    int ahi, blo;
+    const int lo = window_lo(L.window, pos);
+    const int n = D.staged ? staged_range(D, p0, rows, row, lo, ahi, blo) : key_count(D, KS, span != 0, L.window, pos);
     int count, chunk;
     key_chunks(n, D.nkv, rows > 1, count, chunk);
     auto merged = [&](int q) -> float {
@@ -2361,11 +2504,11 @@ __global__ __launch_bounds__(DG_THREADS) void k_dec_group(const int8_t* k8l, con
         const int8_t q = quant_one(v, 1.0f / s);
         if (lane < qk) {
             ks8[n - 1][lane] = q;
-            if (owner) S.k8[(((size_t)layer * D.cap + p0) * nkv + kvh) * qk + lane] = q;
+            if (owner) S.k8[(((size_t)layer * D.kslots + p0) * nkv + kvh) * qk + lane] = q;
         }
         if (lane == 0) {
             kss[n - 1] = s;
-            if (owner) S.ks[((size_t)layer * D.cap + p0) * nkv + kvh] = s;
+            if (owner) S.ks[((size_t)layer * D.kslots + p0) * nkv + kvh] = s;
         }
     } else if (wave == HP + 1) {
         const float v = unit_finish<TAPS, EXACT>(D, S, layer, p0, qd + kd + kvh * vd, vd, ui, false, lane, owner);
@@ -2377,7 +2520,7 @@ __global__ __launch_bounds__(DG_THREADS) void k_dec_group(const int8_t* k8l, con
         }
         if (lane == 0) {
             vss[n - 1] = s;
-            if (owner) S.vs[((size_t)layer * D.cap + p0) * nkv + kvh] = s;
+            if (owner) S.vs[((size_t)layer * D.kslots + p0) * nkv + kvh] = s;
         }
     } else {
 #pragma unroll
@@ -2584,7 +2727,7 @@ hipError_t fwd_dec_attn(const Dims& D, const SessDev& S, const LayerDev& L, int 
     // The staging loads' operands lead the arguments (scalars, preloaded
     // into SGPRs at wave launch): the layer's key rows, scales and value
     // columns, the window start and the geometry (nh, nkv, qk, vd < 256).
-    const size_t lc = (size_t)layer * D.cap;
+    const size_t lc = (size_t)layer * D.kslots;
     const int8_t* k8l = S.k8 + lc * D.nkv * D.qk;
     const float* ksl = S.ks + lc * D.nkv;
     const float* vsl = S.vs + lc * D.nkv;
@@ -2703,7 +2846,7 @@ __global__ __launch_bounds__(DG_THREADS) void k_dec_chunks(Dims D, SessDev S, La
     __shared__ float att[HP * MAX_HEAD_DIM];
     __shared__ float gden[HP * MAX_HEAD_DIM];
     __shared__ int s_merge;
-    const size_t lc = (size_t)layer * D.cap;
+    const size_t lc = (size_t)layer * D.kslots;
     const int role = __builtin_amdgcn_readfirstlane(wave < HP ? 0 : min(wave - HP + 1, 3));  // 0 q, 1 k, 2 v, 3 keys
     constexpr int NS = DG_THREADS - (HP + 2) * 64;  // staging threads
     constexpr int KR = (ATT_CHUNK_MAX * 4 + NS - 1) / NS, SR = (ATT_CHUNK_MAX + NS - 1) / NS;

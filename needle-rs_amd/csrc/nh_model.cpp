@@ -520,6 +520,27 @@ int span_keys(const nh_session* s, const nh::Dims& D, const std::vector<nh::Laye
     return NH_OK;
 }
 
+// Whether the tokens from s->len on, of which the first chunk holds `first`,
+// can be fed under the span as chunks together (or one chunk of two tokens
+// or more) in the staged form: their keys and values go to staging slots, so
+// no chunk overwrites a ring slot an earlier one still reads, and every row
+// takes its chunk's key ranges (chunk end e: [0, sink) and [max(e - ring,
+// sink), e)) without a slot map.  That needs every older position of the
+// first chunk's ranges to be live (later chunks see no other older ones, and
+// a feed's own positions within a ring of its end are never overwritten by
+// it), a ring no shorter than a chunk, and the grouped kernel's geometry.
+bool span_staged(const nh_session* s, int first) {
+    if (first < 2 || s->ring < nh::FWD_ROWS) return false;
+    for (const auto& L : s->m->layers)
+        if (!nh::attend_staged_fits(s->dims, L)) return false;
+    const int p0 = s->len;
+    for (int p = 0; p < std::min(s->sink, p0); ++p)
+        if (!live(s, p)) return false;
+    for (int p = std::max(p0 + first - s->ring, s->sink); p < p0; ++p)
+        if (!live(s, p)) return false;
+    return true;
+}
+
 // Rows an output mode returns for a feed of t tokens (chunk.rs:331-335).
 int out_rows_of(int outputs, int t) {
     return outputs == NH_OUT_NONE ? 0 : (outputs == NH_OUT_ALL_LOGITS || outputs == NH_OUT_HIDDEN) ? t : 1;
@@ -540,9 +561,11 @@ int out_width(const nh_session* s, int outputs) {
 // session's copies); for several chunks the Last* modes mean the last
 // chunk's last row, All* every row.  `cells` (device, or null): the rows'
 // cells [t][layers + 1][d] (step.rs:240-243,672-714, chunk.rs:69-70,310).
+// staged: under an attention span, the staged form (span_staged held).
 // pick: the greedy loop's step, whose token is the argmax of the previous
 // step's logits, taken by the feed's first kernel.
-int feed(nh_session* s, int t, int outputs, float* out, float* cells, hipStream_t st, bool pick = false) {
+int feed(nh_session* s, int t, int outputs, float* out, float* cells, hipStream_t st, bool pick = false,
+         bool staged = false) {
     const nh_model* m = s->m;
     nh::SessDev S = s->S;
     S.cells = cells;
@@ -558,7 +581,9 @@ int feed(nh_session* s, int t, int outputs, float* out, float* cells, hipStream_
         return fail(NH_EDEVICE, "a feed failed on purpose (nh_session_debug_fail_feed)");
     nh::KeySpan span{};
     const nh::KeySpan* sp = nullptr;
-    if (s->ring > 0) {
+    if (s->ring > 0 && staged) {
+        D.staged = 1;
+    } else if (s->ring > 0) {
         if (int rc = span_keys(s, D, m->layers, p0, p0 + t, &span)) return rc;
         sp = &span;
     }
@@ -746,10 +771,12 @@ int forward_ids(nh_session* s, const uint32_t* toks, int n, int outputs, float* 
     int rows = 0;
     for (int i = 0; i < n;) {
         // whole chunks of 32 together while every chunk has two tokens or
-        // more (a one-token chunk is a step) and no attention span (a span's
-        // slot map changes chunk by chunk)
+        // more (a one-token chunk is a step); under an attention span when
+        // the staged form holds, else chunk by chunk (the slot map changes
+        // with each)
         int t = std::min(nh::FWD_ROWS, n - i);
-        if (s->ring == 0 && t > 1)
+        const bool staged = s->ring > 0 && span_staged(s, t);
+        if ((s->ring == 0 || staged) && t > 1)
             while (t < nh::BATCH_ROWS && i + t < n && n - (i + t) > 1) t += std::min(nh::FWD_ROWS, n - (i + t));
         const bool last = i + t == n;
         const int want =
@@ -757,7 +784,7 @@ int forward_ids(nh_session* s, const uint32_t* toks, int n, int outputs, float* 
         const size_t cw = s->cell_floats();
         float* cdst = nullptr;
         if (want_cells) cdst = s->track_cells ? s->d_cells + (size_t)s->ncells * cw : cells ? cells + i * cw : nullptr;
-        const int r = feed(s, t, want, out ? out + (size_t)rows * width : nullptr, cdst, st);
+        const int r = feed(s, t, want, out ? out + (size_t)rows * width : nullptr, cdst, st, false, staged);
         if (r < 0) return reset_after(s, r);
         if (cdst && s->track_cells) {
             if (cells)
@@ -848,7 +875,9 @@ int nh_session_new(const nh_model* m, int cap, nh_session** out) {
     nh::Dims& D = s->dims;
     D = m->dims;
     D.cap = cap;
-    D.vcap = (int)round_up((size_t)cap + 4, 16);
+    D.stage0 = (int)round_up((size_t)cap, 16);
+    D.kslots = D.stage0 + nh::BATCH_ROWS;
+    D.vcap = (int)round_up((size_t)D.kslots + 4, 16);
     int mc = 1;
     for (int n = 1; n <= cap; ++n) mc = std::max(mc, key_chunk_count(n, D.nkv));
     D.max_chunks = mc;
@@ -866,8 +895,9 @@ int nh_session_new(const nh_model* m, int cap, nh_session** out) {
     const size_t o_po = Y.take(R * D.nh * mc * D.vd * 4), o_pm = Y.take(R * D.nh * mc * 4),
                  o_ps = Y.take(R * D.nh * mc * 4);
     const size_t o_hist = Y.take(L * D.hist_slots * D.W * 4);
-    const size_t o_k8 = Y.take(L * c * D.nkv * D.qk), o_ks = Y.take(L * c * D.nkv * 4);
-    const size_t o_v8 = Y.take(L * D.nkv * D.vd * D.vcap), o_vs = Y.take(L * c * D.nkv * 4);
+    const size_t ksl = D.kslots;
+    const size_t o_k8 = Y.take(L * ksl * D.nkv * D.qk), o_ks = Y.take(L * ksl * D.nkv * 4);
+    const size_t o_v8 = Y.take(L * D.nkv * D.vd * D.vcap), o_vs = Y.take(L * ksl * D.nkv * 4);
     const size_t o_e8 = Y.take(E * c * d), o_es = Y.take(E * c * (d / 32) * 4);
     const size_t o_xi = Y.take(AR * Gd * nh::GROUP), o_si = Y.take(AR * Gd * 4);
     const size_t o_xa = Y.take(AR * Ga * nh::GROUP), o_sa = Y.take(AR * Ga * 4);
