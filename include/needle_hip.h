@@ -115,8 +115,17 @@ int nh_matmul(const nh_qmat* w, const nh_qact* a, float* y, int ldy, int col0, v
 /* QLinear::apply (qlinear.rs:555-557): y[rows][out] = the products of w
  * with QAct::new(x, rows, in_dim, act_bits) (DEVICE x[rows][in_dim] f32,
  * DEVICE y), the decode combine for one row, the prefill combine for more.
- * The activation staging is allocated and released on `stream` by the call. */
+ * One row of a small matrix runs as one launch without staging; otherwise the
+ * activation staging is allocated and released on `stream` by the call. */
 int nh_qlinear_apply(const nh_qmat* w, const float* x, int rows, float* y, void* stream);
+/* nh_qlinear_apply with the caller's staging (an allocator of its own keeps
+ * the call to its launches): DEVICE ws, 16-byte aligned, of at least
+ * nh_qlinear_apply_ws_bytes(w, rows) bytes, used by the work queued on
+ * `stream` only.  0 bytes (one row of a small matrix): ws may be null, if x
+ * and y do not overlap. */
+int64_t nh_qlinear_apply_ws_bytes(const nh_qmat* w, int rows);
+int nh_qlinear_apply_ws(const nh_qmat* w, const float* x, int rows, float* y, void* ws, uint64_t ws_bytes,
+                        void* stream);
 /* No counterpart in the reference: nh_qlinear_apply for callers that cannot
  * allocate (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  It allocates nothing: the activation staging is a

@@ -654,9 +654,44 @@ static int check_apply(const nh_qmat* w, const float* x, int rows, const float* 
     return NH_OK;
 }
 
+// One row whose A8 runs inside the product: no staging.  Its workgroups read
+// x while others store y, so an overlapping pair (an in-place call) takes the
+// two steps.
+static bool apply_fused(const nh_qmat* w, const float* x, int rows, const float* y) {
+    return rows == 1 && gemv_f32_fits(w) && (x + w->m.in_dim <= y || y + w->m.out <= x);
+}
+
+static size_t apply_ws_bytes(const nh_qmat* w, int rows) {
+    const size_t cap = ((size_t)rows + ACT_PAD - 1) / ACT_PAD * ACT_PAD;
+    return cap * w->m.groups * (GROUP + 4);
+}
+
+int64_t nh_qlinear_apply_ws_bytes(const nh_qmat* w, int rows) {
+    if (!w || rows <= 0) return fail(NH_EINVAL, "bad arguments");
+    return rows == 1 && gemv_f32_fits(w) ? 0 : (int64_t)apply_ws_bytes(w, rows);
+}
+
+int nh_qlinear_apply_ws(const nh_qmat* w, const float* x, int rows, float* y, void* ws, uint64_t ws_bytes,
+                        void* stream) {
+    if (int rc = check_apply(w, x, rows, y)) return rc;
+    hipStream_t st = (hipStream_t)stream;
+    if (apply_fused(w, x, rows, y)) {
+        NH_HIP(launch_gemv_f32(w, x, y, st), "apply");
+        return NH_OK;
+    }
+    if (!ws || (uintptr_t)ws % 16 != 0) return fail(NH_EINVAL, "apply: no 16-byte aligned workspace");
+    if (ws_bytes < apply_ws_bytes(w, rows)) return fail(NH_ESMALL, "apply: the workspace is too small");
+    const int cap = (rows + ACT_PAD - 1) / ACT_PAD * ACT_PAD;
+    return apply_into(w, x, rows, y, (int8_t*)ws, (float*)((uint8_t*)ws + (size_t)cap * w->m.groups * GROUP), cap, st);
+}
+
 int nh_qlinear_apply(const nh_qmat* w, const float* x, int rows, float* y, void* stream) {
     if (int rc = check_apply(w, x, rows, y)) return rc;
     hipStream_t st = (hipStream_t)stream;
+    if (apply_fused(w, x, rows, y)) {
+        NH_HIP(launch_gemv_f32(w, x, y, st), "apply");
+        return NH_OK;
+    }
     const int cap = (rows + ACT_PAD - 1) / ACT_PAD * ACT_PAD;
     const size_t nx = (size_t)cap * w->m.groups * GROUP, ns = (size_t)cap * w->m.groups;
     void* buf = nullptr;
@@ -675,6 +710,10 @@ int nh_qlinear_apply_static(const nh_qmat* w, const float* x, int rows, float* y
     NH_HIP(hipGetDevice(&dev), "hipGetDevice");
     void* p = dev >= 0 && dev < MAX_DEVICES ? g_scratch[dev] : nullptr;
     if (!p) return fail(NH_ESTATE, "nh_init has not been called for the current device");
+    if (apply_fused(w, x, rows, y)) {
+        NH_HIP(launch_gemv_f32(w, x, y, (hipStream_t)stream), "apply");
+        return NH_OK;
+    }
     // Nothing in the staging needs to start at zero: act_prep writes the
     // rows' codes and scales, and the products store no padding row.
     return apply_into(w, x, rows, y, (int8_t*)p, (float*)((uint8_t*)p + SCRATCH_XQ), STATIC_ROWS,

@@ -175,6 +175,40 @@ hipError_t launch_gemv_batch(const nh_qmat* const* w, const nh_qact* const* a, f
     return w[0]->m.bits == 2 ? dispatch_batch<2>(w[0], b, n, s) : dispatch_batch<4>(w[0], b, n, s);
 }
 
+// One f32 token against a matrix, its A8 done by the product's own
+// workgroups (gemv_tile's XF form): one launch and no activation buffer for
+// QLinear::apply of a token.  Every tile repeats the A8 of every group, so
+// this is for matrices of up to 64 tile-groups a CU (gemv_f32_fits: 8192 x
+// 4096); larger ones do the A8 once, in a launch before.  Graph replay, us,
+// one launch against two: 1568 x 768 2.55 / 4.80, 3072 x 2048 3.33 / 6.30,
+// 8192 x 2048 4.60 / 6.83, 8192 x 4096 7.10 / 10.37 (2-bit 6.37 / 9.84).  The
+// whole call on 1568 x 768, with the staging's release gone from it: 28.3 ->
+// 7.1 us.
+template <int GPS, int S, int BITS, bool NT>
+__global__ __launch_bounds__(S * 64) void k_gemv_f32(const void* __restrict__ codes, const uint16_t* __restrict__ norms,
+                                                     const float* __restrict__ x, float* __restrict__ y, int in_dim,
+                                                     int out, int G, float cbs, Lut lut) {
+    gemv_tile<GPS, S, BITS, false, NT, true>(codes, norms, nullptr, nullptr, y, nullptr, out, G, cbs, lut, blockIdx.x,
+                                             x, in_dim);
+}
+
+bool gemv_f32_fits(const nh_qmat* w) {
+    return (long)w->m.out_pad / TILE_ROWS * w->m.groups <= 64L * device_cus() && w->m.groups <= 32;
+}
+
+hipError_t launch_gemv_f32(const nh_qmat* w, const float* x, float* y, hipStream_t s) {
+    const QMatMeta& m = w->m;
+    const Lut lut{m.lut.a_hi, m.lut.a_lo, m.lut.b_hi, m.lut.b_lo};
+    return gemv_shape(m.groups, [&](auto sh) {
+        constexpr int GPS = decltype(sh)::GPS, S = decltype(sh)::S;
+        auto kern = m.bits == 2 ? (w->resident ? k_gemv_f32<GPS, S, 2, false> : k_gemv_f32<GPS, S, 2, true>)
+                                : (w->resident ? k_gemv_f32<GPS, S, 4, false> : k_gemv_f32<GPS, S, 4, true>);
+        hipLaunchKernelGGL(kern, dim3(m.out_pad / TILE_ROWS), dim3(S * 64), 0, s, w->d_codes, w->d_norms, x, y,
+                           m.in_dim, m.out, m.groups, m.cbs, lut);
+        return hipGetLastError();
+    });
+}
+
 // Read floors of the decode product, for measurement only.  The tile form
 // issues exactly the loads k_gemv<GPS, S, 4> issues (codes with the
 // streaming hint, norms, activations, scales) in its grid, and no

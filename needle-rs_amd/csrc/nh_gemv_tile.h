@@ -16,11 +16,16 @@ namespace nh {
 // NT: the code loads carry the non-temporal hint (a matrix read once per
 // sweep of more than the caches hold); without it (a resident matrix, read
 // again at every token) their lines stay cached.
-template <int GPS, int S, int BITS, bool DBG, bool NT>
+// XF: the token comes as f32 (xf, in_dim values) and each wavefront A8s its
+// own groups into its part of the LDS activations (prep_group's arithmetic,
+// the same in every tile), so the product needs no activation buffer and no
+// launch of its own for them.
+template <int GPS, int S, int BITS, bool DBG, bool NT, bool XF = false>
 __device__ __forceinline__ void gemv_tile(const void* __restrict__ codes, const uint16_t* __restrict__ norms,
                                           const uint4* __restrict__ xq, const float* __restrict__ sx,
                                           float* __restrict__ y, int32_t* __restrict__ dbg, int out, int G, float cbs,
-                                          Lut lut, int tile) {
+                                          Lut lut, int tile, const float* __restrict__ xf = nullptr,
+                                          int in_dim = 0) {
     const int wave = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
     const int r = lane >> 2, l = lane & 3;
@@ -33,11 +38,19 @@ __device__ __forceinline__ void gemv_tile(const void* __restrict__ codes, const 
     // wavefront, an L2 hit after the first workgroup) and no barrier waits
     // for the slowest wavefront; with more, the G * 128 bytes go to LDS once
     // per workgroup (two direct reads per group measured slower there).
-    constexpr bool DIRECT = GPS == 1;
-    static_assert(DIRECT || S * 64 >= GPS * S * 8, "one thread per activation uint4");
+    constexpr bool DIRECT = GPS == 1 && !XF;
+    static_assert(DIRECT || XF || S * 64 >= GPS * S * 8, "one thread per activation uint4");
     __shared__ uint4 xs[DIRECT ? 1 : GPS * S * 8];
     uint4 xa[GPS], xb[GPS], xv = make_uint4(0, 0, 0, 0);
-    if constexpr (DIRECT) {
+    float x0f[GPS], x1f[GPS];
+    if constexpr (XF) {
+#pragma unroll
+        for (int j = 0; j < GPS; ++j) {
+            const int p0 = (g0 + j) * GROUP + lane, p1 = p0 + 64;
+            x0f[j] = p0 < in_dim ? xf[p0] : 0.0f;
+            x1f[j] = p1 < in_dim ? xf[p1] : 0.0f;
+        }
+    } else if constexpr (DIRECT) {
         const int g = g0 < G ? g0 : 0;
         xa[0] = xq[(g * 4 + l) * 2];
         xb[0] = xq[(g * 4 + l) * 2 + 1];
@@ -59,9 +72,20 @@ __device__ __forceinline__ void gemv_tile(const void* __restrict__ codes, const 
         } else
             c[j] = reinterpret_cast<const uint2*>(codes)[(size_t)(tile * G + g) * 64 + lane];
         nb[j] = norms[(size_t)n * G + g];
-        sxv[j] = sx[g];
+        if constexpr (!XF) sxv[j] = sx[g];
     }
-    if constexpr (!DIRECT) {
+    if constexpr (XF) {
+        // (groups past G are zeros and never used)
+        __shared__ float xsc[GPS * S];
+#pragma unroll
+        for (int j = 0; j < GPS; ++j)
+            a8_group(x0f[j], x1f[j], lane, BITS, reinterpret_cast<int8_t*>(xs + (g0 + j) * 8), &xsc[g0 + j]);
+        // the wavefront reads back only what it wrote
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < GPS; ++j) sxv[j] = xsc[g0 + j];
+    } else if constexpr (!DIRECT) {
         if (threadIdx.x < G * 8) xs[threadIdx.x] = xv;
         __syncthreads();
     }
@@ -73,7 +97,7 @@ __device__ __forceinline__ void gemv_tile(const void* __restrict__ codes, const 
             x0 = xa[j];
             x1 = xb[j];
         } else {
-            const int g = g0 + j < G ? g0 + j : 0;
+            const int g = XF || g0 + j < G ? g0 + j : 0;
             const uint4* xp = xs + (g * 4 + l) * 2;
             x0 = xp[0];
             x1 = xp[1];

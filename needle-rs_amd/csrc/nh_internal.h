@@ -145,6 +145,11 @@ hipError_t launch_gemv_batch(const nh_qmat* const* w, const nh_qact* const* a, f
 hipError_t launch_act_prep(const float* x, int rows, int in_dim, int groups, int bits, const uint16_t* norm_scale,
                            int8_t* xq, float* sx, hipStream_t s);
 hipError_t launch_gemv(const nh_qmat* w, const nh_qact* a, float* y, int col0, int32_t* dbg_lanes, hipStream_t s);
+// A8 of one f32 token and the decode product in one launch, for matrices
+// small enough that every tile repeating the A8 costs less than a launch
+// (x and y must not overlap).
+bool gemv_f32_fits(const nh_qmat* w);
+hipError_t launch_gemv_f32(const nh_qmat* w, const float* x, float* y, hipStream_t s);
 // The decode product's read floors (0: its loads in its grid, 1: a plain stream of its bytes).
 hipError_t launch_read_floor(const nh_qmat* w, const nh_qact* a, int mode, float* y, hipStream_t s);
 hipError_t launch_expand_w8(const nh_qmat* w, hipStream_t s);

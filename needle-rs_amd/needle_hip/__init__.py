@@ -46,6 +46,8 @@ SIGNATURES = {
     "nh_qact_download": (I, [P, P, C.c_uint64, P, C.c_uint64]),
     "nh_matmul": (I, [P, P, P, I, I, P]),
     "nh_qlinear_apply": (I, [P, P, I, P, P]),
+    "nh_qlinear_apply_ws_bytes": (C.c_int64, [P, I]),
+    "nh_qlinear_apply_ws": (I, [P, P, I, P, P, C.c_uint64, P]),
     "nh_qlinear_apply_static": (I, [P, P, I, P, P]),
     "nh_matmul_flags": (I, [P, P, P, P, I, I, P]),
     "nh_single_rows": (I, [P, P, P, I, P, P]),
@@ -129,6 +131,7 @@ def init(device: int = 0):
     if not _ready:
         if not torch.cuda.is_available():
             raise NeedleHipError(-3, "no HIP device visible")
+        torch.cuda.init()
         torch.cuda.set_device(device)
         _check(lib.nh_init(device))
         _ready = True
@@ -136,13 +139,15 @@ def init(device: int = 0):
 
 
 def _stream(stream=None):
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return C.c_void_p(s.cuda_stream)
+    if stream is not None:
+        return stream.cuda_stream
+    # (the current stream's handle without building a Stream object)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _dptr(t: torch.Tensor):
     assert t.is_cuda and t.is_contiguous()
-    return C.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _hptr(a: np.ndarray):
@@ -340,8 +345,18 @@ class QLinear:
     def apply(self, x: torch.Tensor, rows: int, stream=None) -> torch.Tensor:
         """QLinear::apply (qlinear.rs:555-557): A8 of x [rows][in_dim] and the
         products, in one call (nh_qlinear_apply)."""
+        rows = int(rows)
         y = torch.empty((rows, self.out), dtype=torch.float32, device="cuda")
-        _check(_lib.nh_qlinear_apply(self.fused.h, _dptr(x), int(rows), _dptr(y), _stream(stream)))
+        if stream is not None:
+            # (the call's own stream-ordered staging: torch would hand a
+            # workspace of the current stream on before that stream is done)
+            _check(_lib.nh_qlinear_apply(self.fused.h, _dptr(x), rows, _dptr(y), _stream(stream)))
+            return y
+        # the staging from torch's caching allocator, on the current stream
+        n = _lib.nh_qlinear_apply_ws_bytes(self.fused.h, rows)
+        ws = torch.empty(n, dtype=torch.uint8, device="cuda") if n > 0 else None
+        _check(_lib.nh_qlinear_apply_ws(self.fused.h, _dptr(x), rows, _dptr(y), ws.data_ptr() if n > 0 else None,
+                                        max(n, 0), _stream()))
         return y
 
     def apply_static(self, x: torch.Tensor, rows: int, y: torch.Tensor, stream=None) -> torch.Tensor:
