@@ -73,7 +73,7 @@ struct KeySpan {
 };
 
 struct LayerDev {
-    const uint16_t* stage;  // the six Kronecker factors (MFMA fragments), cond_v [d][8], cond_u [1024][8]
+    const uint16_t* stage;  // the six Kronecker factors (MFMA fragments), cond_v by chain (f32), cond_u [1024][8]
     const uint16_t *d1, *d2, *b2, *d3, *d4;
     const uint16_t *norm_in, *post_norm, *pre_hada, *q_taps, *k_taps, *v_taps, *q_norm, *k_norm;
     const int8_t* phi_q;  // [24][lanes * d]

@@ -123,6 +123,11 @@ __host__ __device__ inline void key_chunks(int n, int nkv, bool nested, int& cou
 }
 
 // The attended range of position p0: keys lo..p0.
+// roundf of a value >= 0 as an integer (the attention weights' 21-bit
+// digits): truncating v + the float below 1/2 gives the same for every float
+// in [0, 2^22) (checked over all of them), in two instructions.
+__device__ __forceinline__ int32_t round_digits(float v) { return (int32_t)(v + 0x1.fffffep-2f); }
+
 // slot_of (infer.rs:1749-1756): the KV slot of position p; the sink keeps
 // its positions, the rest share the ring.
 __device__ __forceinline__ int slot_of(const Dims& D, int p) {
@@ -392,9 +397,10 @@ constexpr int BT_PITCH = 36;  // floats per row of a first mix8's output (16-byt
 constexpr int TP_D = FWD_MAX_D / 16 + 4;
 constexpr int TP_X = MHC_LANES * FWD_MAX_D / 16 + 4;
 constexpr int TP_H = FWD_MAX_D / 4 + 4;
-constexpr int TP_C = FWD_MAX_D / 4 + 8;
+constexpr int TP_C = FWD_MAX_D / 4 + 4;
 
-struct LayerShared {
+// One row's LDS.
+struct LayerRow {
     float x2[FWD_MAX_D];
     float h[FWD_MAX_D];
     // The MLP's buffers are dead once its last pass is read; the mHC write
@@ -403,13 +409,11 @@ struct LayerShared {
         struct {
             alignas(16) float A[HADA_N];
             alignas(16) float B[HADA_NB * BT_PITCH];
-            alignas(16) uint4 kf[6][HADA_N / 8];  // Kronecker factors as MFMA fragments (stage order)
         };
         alignas(16) float tX[16 * TP_X];
     };
     alignas(16) float C[HADA_N];
     alignas(16) int8_t nx8[MHC_LANES * FWD_MAX_D];
-    alignas(16) uint16_t cvT[4 * COND_RANK * TP_C];
     alignas(16) float tA[16 * TP_D];
     alignas(16) float tB[16 * TP_D];
     alignas(16) float hT[4 * TP_H];
@@ -417,7 +421,15 @@ struct LayerShared {
     float p[64];
     float wk[COND_RANK];
     float r_sx, r_a, r_b, r_c;
-    int mix_count;  // the mixer wavefronts' arrivals (mixer_sync)
+    int mix_count;  // the row's mixer wavefronts' arrivals (mixer_sync)
+};
+
+// RP rows of a workgroup and the previous layer's tables they share.
+template <int RP>
+struct LayerShared {
+    alignas(16) uint4 kf[6][HADA_N / 8];  // Kronecker factors as MFMA fragments (stage order)
+    alignas(16) float cvT[4 * COND_RANK * TP_C];
+    LayerRow row[RP];
 };
 
 // chain_pipe for a fixed batch count, fully unrolled (batch indices are
@@ -625,27 +637,31 @@ __device__ __forceinline__ void mixer_sync(int* count, int target, int limit, in
     __builtin_amdgcn_wave_barrier();
 }
 
-// rinv(dot16(x, x)) over a transposed operand by wavefront 0, handed to
-// the block through LDS.
-__device__ __forceinline__ float block_rinv_t(const float* xT, int pitch, int n, float* slot) {
-    if ((threadIdx.x >> 6) == 0) {
-        const float r = rinv(dot16_t<true>(xT, xT, pitch, n, threadIdx.x & 63), n);
-        if (threadIdx.x == 0) *slot = r;
+// rinv(dot16(x, x)) of every row's transposed operand xT(row), row rr's by
+// wavefront rr, handed to the block through LDS (slot(row)).
+//
+// (Every wavefront running the chain itself saves the hand-over's barrier:
+// block_rinv_all.  With one row that is faster for the MLP's h2 norm, 0.5 k
+// cycles; the other d-long norms measured slower that way, decode 501.6 ->
+// 507.5 us per token, and for the 4d-long mHC operand the sixteen copies' LDS
+// reads cost more than the barrier, 0.7 k cycles.)
+template <int RP, typename Op, typename Slot>
+__device__ __forceinline__ void block_rinv_t(LayerShared<RP>& sh, Op xT, int pitch, int n, Slot slot, float (&r)[RP]) {
+    const int wave = RP == 1 ? threadIdx.x >> 6 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (wave < RP) {
+        LayerRow& R = sh.row[RP == 1 ? 0 : wave];
+        const float v = rinv(dot16_t<true>(xT(R), xT(R), pitch, n, threadIdx.x & 63), n);
+        if ((threadIdx.x & 63) == 0) slot(R) = v;
     }
     __syncthreads();
-    return *slot;
+#pragma unroll
+    for (int rr = 0; rr < RP; ++rr) r[rr] = slot(sh.row[rr]);
 }
 
-// The same value computed by every wavefront (each runs the 16-lane chain;
-// the result is wavefront-uniform and identical in all of them), so no
-// barrier hands it over.  The chain is latency-bound (~13 cycles a step),
-// so four wavefronts on a SIMD run their copies side by side at about the
-// cost of one for d-long operands: the MLP's h2 norm (measured: 0.5 k cycles
-// saved).  The other d-long norms (post norm, input norm, the head's norm)
-// measured slower this way (decode 501.6 -> 507.5 us per token, prefill
-// 1.303 -> 1.332 ms), and for the 4d-long mHC operand the sixteen copies'
-// LDS reads cost more than the barrier (0.7 k cycles lost), so those stay on
-// wavefront 0.  The phase that follows must not write the operand.
+// The same value of one row computed by every wavefront (each runs the
+// 16-lane chain; the result is wavefront-uniform and identical in all of
+// them), so no barrier hands it over.  The phase that follows must not write
+// the operand.
 __device__ __forceinline__ float block_rinv_all(const float* xT, int pitch, int n) {
     return rinv(dot16_t<true>(xT, xT, pitch, n, threadIdx.x & 63), n);
 }
@@ -653,39 +669,43 @@ __device__ __forceinline__ float block_rinv_all(const float* xT, int pitch, int 
 
 // The previous layer's inputs and weights a thread needs, read up front.
 // The LDS tables go out as one list of 16-byte chunks, up to STAGE_PER per
-// thread: [0, 768) the six Kronecker factors (128 each), then cond_v
-// (d chunks); cond_u follows them, one 16-byte column per thread.
-constexpr int STAGE_PER = 2;
+// thread, in the order of their LDS copies: [0, 768) the six Kronecker
+// factors (f16, 128 each), then cond_v (f32) by chain, COND_CHUNKS for each
+// of the 32 chains (the first d / 16 of them used); cond_u follows them, one
+// 16-byte column per thread.
+constexpr int KRON_CHUNKS = 6 * HADA_N / 8, COND_CHUNKS = FWD_MAX_D / 16;
+constexpr int STAGE_CHUNKS = KRON_CHUNKS + 4 * COND_RANK * COND_CHUNKS;
+constexpr int STAGE_PER = (STAGE_CHUNKS + LT - 1) / LT;
 
 // f16 weights stay raw bits (one per register) until their use:
 // converting or packing them on arrival would make the wave wait for each
 // load before issuing the next.
+template <int RP>
 struct OutRegs {
-    float o, x1, u, pv;
+    float o[RP], x1[RP], u[RP], pv[RP];
     uint32_t pn, ph, d1, d2, b2, d3, d4;
     int p1, p2;
-    uint4 st[STAGE_PER];
+    u32x4 st[STAGE_PER];
     uint4 cu;  // cond_u [k][t], k < 8, as f16 pairs
 };
 
-__device__ __forceinline__ OutRegs load_out(int d, const uint4* stage, const uint16_t* pn, const Globals& G,
-                                            const SessDev& S, const LayerDev& P) {
+template <int RP>
+__device__ __forceinline__ OutRegs<RP> load_out(int d, const uint4* stage, const uint16_t* pn, const Globals& G,
+                                                const SessDev (&S)[RP], const LayerDev& P) {
     const int t = threadIdx.x;
-    OutRegs q{};
-    const int kron_n = 6 * HADA_N / 8, cv_n = d * COND_RANK / 8;
-    static_assert(STAGE_PER * LT >= 6 * HADA_N / 8 + FWD_MAX_D * COND_RANK / 8, "the stage loads cover the tables");
+    OutRegs<RP> q{};
 #pragma unroll
-    for (int r = 0; r < STAGE_PER; ++r) {
-        const int e = min(t + r * LT, kron_n + cv_n - 1);
-        q.st[r] = stage[e];
-    }
-    q.cu = stage[kron_n + cv_n + t];
+    for (int r = 0; r < STAGE_PER; ++r) q.st[r] = reinterpret_cast<const u32x4*>(stage)[min(t + r * LT, STAGE_CHUNKS - 1)];
+    q.cu = stage[STAGE_CHUNKS + t];
     // (unconditional loads: threads past d read element d - 1 and ignore it)
     const int td = min(t, d - 1);
-    q.o = S.o[td];
-    q.pv = S.p[t & 63];
-    q.x1 = S.x1[td];
-    q.u = S.u[td];
+#pragma unroll
+    for (int rr = 0; rr < RP; ++rr) {
+        q.o[rr] = S[rr].o[td];
+        q.pv[rr] = S[rr].p[t & 63];
+        q.x1[rr] = S[rr].x1[td];
+        q.u[rr] = S[rr].u[td];
+    }
     // (the loads above take preloaded operands only: none waits for the
     // argument segment, which those below need)
     __builtin_amdgcn_sched_barrier(0);
@@ -708,69 +728,56 @@ __device__ __forceinline__ float h2f_late(uint32_t b) {
     return h2f((uint16_t)b);
 }
 
-__device__ __forceinline__ void store_out(int d, const OutRegs& q, LayerShared& sh) {
+template <int RP>
+__device__ __forceinline__ void store_out(int d, const OutRegs<RP>& q, LayerShared<RP>& sh) {
     const int t = threadIdx.x;
-    const int kron_n = 6 * HADA_N / 8, cv_n = d * COND_RANK / 8;
 #pragma unroll
     for (int r = 0; r < STAGE_PER; ++r) {
-        const int e = t + r * LT;
-        if (e < kron_n) {
-            (&sh.kf[0][0])[e] = q.st[r];  // (already in fragment order)
-        } else if (e < kron_n + cv_n) {
-            // row j of cond_v (8 f16) into column j / 4 of rows 8 (j % 4) + k
-            const int j = e - kron_n;
-            const uint4 v = q.st[r];
-            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-            uint16_t* dst = sh.cvT + (j & 3) * COND_RANK * TP_C + (j >> 2);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                dst[(2 * k) * TP_C] = (uint16_t)(w[k] & 0xffffu);
-                dst[(2 * k + 1) * TP_C] = (uint16_t)(w[k] >> 16);
-            }
-        }
+        const int e = t + r * LT, c = e - KRON_CHUNKS;
+        u32x4* dst = e < KRON_CHUNKS ? reinterpret_cast<u32x4*>(&sh.kf[0][0]) + e  // (already in fragment order)
+                                     : reinterpret_cast<u32x4*>(sh.cvT + c / COND_CHUNKS * TP_C + c % COND_CHUNKS * 4);
+        if (e < STAGE_CHUNKS) *dst = q.st[r];
     }
-    if (t < d) put_t(sh.tA, TP_D, t, q.o);
-    if (t < 64) sh.p[t] = q.pv;
+#pragma unroll
+    for (int rr = 0; rr < RP; ++rr) {
+        if (t < d) put_t(sh.row[rr].tA, TP_D, t, q.o[rr]);
+        if (t < 64) sh.row[rr].p[t] = q.pv[rr];
+    }
 }
 
-// cond_weights (infer.rs:1640-1656) by wavefront 0: lane 8 jm + k carries
+// cond_weights (infer.rs:1640-1656) by one wavefront: lane 8 jm + k carries
 // acc[jm][k] = fma(h2[j], cond_v[j][k], .) over j = jm, jm + 4, ...
 // (u = j / 4 in order), reading h2 and cond_v from their transposed copies
 // in 8-step batches on chain_pipe; then the softmax of the
 // combined logits.
-__device__ __forceinline__ void cond_weights(const LayerShared& sh, int d, int lane, float* wk) {
+__device__ __forceinline__ void cond_weights(const float* hT, const float* cvT, int d, int lane, float* wk) {
     const int k = lane & 7, jm = lane >> 3;
     float a = 0.0f;
     if (lane < 32) {
         const int steps = d / 4, nb = steps / 8;
-        const float4* hr = reinterpret_cast<const float4*>(sh.hT + jm * TP_H);
-        const uint4* cr = reinterpret_cast<const uint4*>(sh.cvT + (jm * COND_RANK + k) * TP_C);
+        const float4* hr = reinterpret_cast<const float4*>(hT + jm * TP_H);
+        const float4* cr = reinterpret_cast<const float4*>(cvT + (jm * COND_RANK + k) * TP_C);
         struct Buf {
-            float4 h[2];
-            uint4 c;
+            float4 h[2], c[2];
         };
         auto load = [&](Buf& d, int b) {
             d.h[0] = hr[2 * b];
             d.h[1] = hr[2 * b + 1];
-            d.c = cr[b];
+            d.c[0] = cr[2 * b];
+            d.c[1] = cr[2 * b + 1];
         };
         auto chain = [&](const Buf& d) {
-            const float hv[8] = {d.h[0].x, d.h[0].y, d.h[0].z, d.h[0].w, d.h[1].x, d.h[1].y, d.h[1].z, d.h[1].w};
-            const uint32_t cw[4] = {d.c.x, d.c.y, d.c.z, d.c.w};
-            // (converted apart from the chain: folded into the fmas, the
-            // conversions make every dependent step a slower mixed one)
-            float cv[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                cv[u] = h2f((uint16_t)(cw[u >> 1] >> (16 * (u & 1))));
-                asm("" : "+v"(cv[u]));
+            for (int u = 0; u < 2; ++u) {
+                a = __builtin_fmaf(d.h[u].x, d.c[u].x, a);
+                a = __builtin_fmaf(d.h[u].y, d.c[u].y, a);
+                a = __builtin_fmaf(d.h[u].z, d.c[u].z, a);
+                a = __builtin_fmaf(d.h[u].w, d.c[u].w, a);
             }
-#pragma unroll
-            for (int u = 0; u < 8; ++u) a = __builtin_fmaf(hv[u], cv[u], a);
         };
         if (nb > 0) chain_pipe_any<3, Buf>(nb, load, chain);
         for (int u = nb * 8; u < steps; ++u)
-            a = __builtin_fmaf(sh.hT[jm * TP_H + u], h2f(sh.cvT[(jm * COND_RANK + k) * TP_C + u]), a);
+            a = __builtin_fmaf(hT[jm * TP_H + u], cvT[(jm * COND_RANK + k) * TP_C + u], a);
     }
     const float a0 = __shfl(a, k, 64), a1 = __shfl(a, 8 + k, 64), a2 = __shfl(a, 16 + k, 64),
                 a3 = __shfl(a, 24 + k, 64);
@@ -790,92 +797,118 @@ __device__ __forceinline__ void cond_weights(const LayerShared& sh, int d, int l
 }
 
 // The Hadamard MLP and mHC write of layer P (step.rs:600-705): xl holds the
-// thread's element of the 4 lanes (t < d) and gets the new ones; returns
-// this thread's max |new lane value| (for the next layer's mHC read).
-template <typename BeforeMix, typename AfterMlp>
-__device__ float layer_out(const Dims& D, const SessDev& S, const LayerDev& P, const OutRegs& q, LayerShared& sh,
-                           float (&xl)[MHC_LANES], BeforeMix before_mix, AfterMlp after_mlp) {
+// thread's element of the rows' 4 lanes (t < d) and gets the new ones; m gets
+// this thread's max |new lane value| of each row (for the next layer's mHC
+// read).
+template <int RP, typename BeforeMix, typename AfterMlp>
+__device__ void layer_out(const Dims& D, const SessDev& S, const LayerDev& P, const OutRegs<RP>& q, LayerShared<RP>& sh,
+                          float (&xl)[RP][MHC_LANES], float (&m)[RP], BeforeMix before_mix, AfterMlp after_mlp) {
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63, d = D.d;
-    // mix8 runs on waves 4..7 (threads 256..511), beside cond_weights on wave 0
-    const bool mixer = t >= MIX_T && t < 2 * MIX_T;
-    const int mu = t - MIX_T;
+    // mix8 runs on waves 4..7 (threads 256..511; row 1: 8..11), beside
+    // cond_weights on wave 0 (row 1: wave 1)
+    const bool mixer = t >= MIX_T && t < (1 + RP) * MIX_T;
+    const int mu = RP == 1 ? t - MIX_T : t & (MIX_T - 1);
+    LayerRow& M = sh.row[RP == 1 ? 0 : __builtin_amdgcn_readfirstlane(mixer ? t / MIX_T - 1 : 0)];
     // on = zcn16(o, post_norm); x2 = fma(on, sigmoid(attn_gate), x1)
-    float x2 = 0.0f;
+    float x2[RP] = {};
     {
-        const float r = block_rinv_t(sh.tA, TP_D, d, &sh.r_a);
+        float r[RP];
+        block_rinv_t<RP>(sh, [](LayerRow& R) { return R.tA; }, TP_D, d, [](LayerRow& R) -> float& { return R.r_a; }, r);
         if (t < d) {
-            const float tt = q.o * r;
-            const float on = __builtin_fmaf(tt, h2f_late(q.pn), tt);
-            x2 = __builtin_fmaf(on, P.ga, q.x1);
-            put_t(sh.tB, TP_D, t, x2);
+#pragma unroll
+            for (int rr = 0; rr < RP; ++rr) {
+                const float tt = q.o[rr] * r[rr];
+                const float on = __builtin_fmaf(tt, h2f_late(q.pn), tt);
+                x2[rr] = __builtin_fmaf(on, P.ga, q.x1[rr]);
+                put_t(sh.row[rr].tB, TP_D, t, x2[rr]);
+            }
         }
     }
     __syncthreads();
     // h2 = zcn16(x2, pre_hada); z = h2 * d1 zero-padded to hada_n
-    float h2 = 0.0f;
     {
-        const float r = block_rinv_all(sh.tB, TP_D, d);
-        if (t < d) {
-            const float tt = x2 * r;
-            h2 = __builtin_fmaf(tt, h2f_late(q.ph), tt);
-            sh.hT[(t & 3) * TP_H + (t >> 2)] = h2;
+        float r[RP];
+        if constexpr (RP == 1)
+            r[0] = block_rinv_all(sh.row[0].tB, TP_D, d);
+        else
+            block_rinv_t<RP>(sh, [](LayerRow& R) { return R.tB; }, TP_D, d, [](LayerRow& R) -> float& { return R.r_b; },
+                             r);
+#pragma unroll
+        for (int rr = 0; rr < RP; ++rr) {
+            float h2 = 0.0f;
+            if (t < d) {
+                const float tt = x2[rr] * r[rr];
+                h2 = __builtin_fmaf(tt, h2f_late(q.ph), tt);
+                sh.row[rr].hT[(t & 3) * TP_H + (t >> 2)] = h2;
+            }
+            sh.row[rr].A[mix_in(t)] = t < d ? h2 * h2f_late(q.d1) : 0.0f;
         }
-        sh.A[mix_in(t)] = t < d ? h2 * h2f_late(q.d1) : 0.0f;
     }
     __syncthreads();
-    // cond_weights (wavefront 0) spans both passes of the first mix8; the
-    // mixers meet between their passes on their own
+    // cond_weights spans both passes of the first mix8; the mixers of a row
+    // meet between their passes on their own
     before_mix();
-    if (wave == 0) cond_weights(sh, d, lane, sh.wk);
+    if (RP == 1 ? wave == 0 : wave < RP) {
+        LayerRow& R = sh.row[RP == 1 ? 0 : __builtin_amdgcn_readfirstlane(wave)];
+        cond_weights(R.hT, sh.cvT, d, lane, R.wk);
+    }
     if (mixer) {
-        mix8_t(mu, sh.kf[0], sh.A, sh.B);
-        mixer_sync(&sh.mix_count, MIX_T / 64, D.spin_limit, S.status);
-        mix8_n(mu, sh.B, sh.kf[1], sh.C, HADA_NB);
+        mix8_t(mu, sh.kf[0], M.A, M.B);
+        mixer_sync(&M.mix_count, MIX_T / 64, D.spin_limit, S.status);
+        mix8_n(mu, M.B, sh.kf[1], M.C, HADA_NB);
     }
     __syncthreads();
     {
-        float cond = 1.0f;
         const uint32_t cw[4] = {q.cu.x, q.cu.y, q.cu.z, q.cu.w};
 #pragma unroll
-        for (int k = 0; k < COND_RANK; ++k)
-            cond = __builtin_fmaf(h2f((uint16_t)(cw[k >> 1] >> (16 * (k & 1)))), sh.wk[k], cond);
-        float zs = __builtin_fmaf(sh.C[q.p1], cond * h2f_late(q.d2), h2f_late(q.b2));
-        zs = zs / (nexp(-zs) + 1.0f);
-        sh.A[mix_in(t)] = zs;
+        for (int rr = 0; rr < RP; ++rr) {
+            LayerRow& R = sh.row[rr];
+            float cond = 1.0f;
+#pragma unroll
+            for (int k = 0; k < COND_RANK; ++k)
+                cond = __builtin_fmaf(h2f((uint16_t)(cw[k >> 1] >> (16 * (k & 1)))), R.wk[k], cond);
+            float zs = __builtin_fmaf(R.C[q.p1], cond * h2f_late(q.d2), h2f_late(q.b2));
+            zs = zs / (nexp(-zs) + 1.0f);
+            R.A[mix_in(t)] = zs;
+        }
     }
     __syncthreads();
-    if (mixer) mix8_t(mu, sh.kf[2], sh.A, sh.B);
+    if (mixer) mix8_t(mu, sh.kf[2], M.A, M.B);
     __syncthreads();
-    if (mixer) mix8_n(mu, sh.B, sh.kf[3], sh.C, HADA_NB);
+    if (mixer) mix8_n(mu, M.B, sh.kf[3], M.C, HADA_NB);
     __syncthreads();
-    sh.A[mix_in(t)] = sh.C[q.p2] * h2f_late(q.d3);
+#pragma unroll
+    for (int rr = 0; rr < RP; ++rr) sh.row[rr].A[mix_in(t)] = sh.row[rr].C[q.p2] * h2f_late(q.d3);
     __syncthreads();
-    if (mixer) mix8_t(mu, sh.kf[4], sh.A, sh.B);
+    if (mixer) mix8_t(mu, sh.kf[4], M.A, M.B);
     __syncthreads();
-    if (mixer) mix8_n(mu, sh.B, sh.kf[5], sh.C, d / HADA_NB / 8 * 8);
+    if (mixer) mix8_n(mu, M.B, sh.kf[5], M.C, d / HADA_NB / 8 * 8);
     __syncthreads();
     after_mlp();
     // The mHC write: y = (x2 + t3 * d4) - u; lane a = y hpost[a] + sum_b
     // hres[a][b] old[b] as an fma chain over b.
-    float m = 0.0f;
-    if (t < d) {
-        const float* hpost = sh.p + MHC_COLS;
-        const float* hres = sh.p + MHC_COLS + MHC_LANES;
-        const float y = (x2 + sh.C[t] * h2f_late(q.d4)) - q.u;
-        float old[MHC_LANES];
 #pragma unroll
-        for (int b = 0; b < MHC_LANES; ++b) old[b] = xl[b];
+    for (int rr = 0; rr < RP; ++rr) {
+        LayerRow& R = sh.row[rr];
+        m[rr] = 0.0f;
+        if (t < d) {
+            const float* hpost = R.p + MHC_COLS;
+            const float* hres = R.p + MHC_COLS + MHC_LANES;
+            const float y = (x2[rr] + R.C[t] * h2f_late(q.d4)) - q.u[rr];
+            float old[MHC_LANES];
 #pragma unroll
-        for (int a = 0; a < MHC_LANES; ++a) {
-            float v = y * hpost[a];
+            for (int b = 0; b < MHC_LANES; ++b) old[b] = xl[rr][b];
 #pragma unroll
-            for (int b = 0; b < MHC_LANES; ++b) v = __builtin_fmaf(old[b], hres[a * MHC_LANES + b], v);
-            xl[a] = v;
-            put_t(sh.tX, TP_X, a * d + t, v);
-            m = fmaxf(m, fabsf(v));
+            for (int a = 0; a < MHC_LANES; ++a) {
+                float v = y * hpost[a];
+#pragma unroll
+                for (int b = 0; b < MHC_LANES; ++b) v = __builtin_fmaf(old[b], hres[a * MHC_LANES + b], v);
+                xl[rr][a] = v;
+                put_t(R.tX, TP_X, a * d + t, v);
+                m[rr] = fmaxf(m[rr], fabsf(v));
+            }
         }
     }
-    return m;
 }
 
 // The next layer's weights a thread needs, read up front: its norm scale,
@@ -892,39 +925,42 @@ static_assert(3 * PHI_MF >= MHC_COLS && 2 * PHI_MF < MHC_COLS, "holders 0 and 1 
 __device__ __forceinline__ int phi_holder(int wave) { return wave >= 1 && wave <= 3 ? wave - 1 : wave >= 8 ? wave - 5 : -1; }
 // PC: the 1 KB chunks a Phi8 row has (its 4 d int8 / 1024), fixed at compile
 // time so a narrower model holds no registers for chunks it never reads (3
-// at d = 768: 24 VGPRs instead of 32, which the 64-VGPR batched kernel needs).
-template <int PC>
+// at d = 768).
+template <int PC, int RP>
 struct InRegs {
     uint32_t norm;
-    float kr, ev, ps0, ps1, ps2;
+    float kr[RP], ev[RP], ps0, ps1, ps2;
     uint4 r0[PC], r1[PC], r2[PC];
 };
 
-template <int PC, bool MF>
-__device__ __forceinline__ void load_phi(const Dims& D, const LayerDev& N, InRegs<PC>& q);
+template <int PC, int RP, bool MF>
+__device__ __forceinline__ void load_phi(const Dims& D, const LayerDev& N, InRegs<PC, RP>& q);
 
 // PHI: the Phi8 rows too (else layer_in reads them itself).
-template <bool PHI, int PC, bool MF>
-__device__ __forceinline__ InRegs<PC> load_in(const Dims& D, const SessDev& S, const LayerDev& N) {
+template <bool PHI, int PC, bool MF, int RP>
+__device__ __forceinline__ InRegs<PC, RP> load_in(const Dims& D, const SessDev (&S)[RP], const LayerDev& N) {
     const int t = threadIdx.x, d = D.d;
     // Unconditional loads at clamped addresses (threads, rows and chunks
     // past the ranges read an in-range element and ignore it; a layer
     // without an engram site reads the projection row instead, which
     // nothing else here reads).
-    InRegs<PC> q;
+    InRegs<PC, RP> q;
     const int td = min(t, d - 1);
     q.norm = N.norm_in[td];
     const bool site = N.site >= 0;
-    const float* kp = site ? S.ekv + (size_t)N.site * BATCH_ROWS * 2 * d : S.proj;
-    const float* ep = site ? S.evals + (size_t)N.site * BATCH_ROWS * d : S.proj + d;
-    q.kr = kp[td];
-    q.ev = ep[td];
-    if constexpr (PHI) load_phi<PC, MF>(D, N, q);
+#pragma unroll
+    for (int rr = 0; rr < RP; ++rr) {
+        const float* kp = site ? S[rr].ekv + (size_t)N.site * BATCH_ROWS * 2 * d : S[rr].proj;
+        const float* ep = site ? S[rr].evals + (size_t)N.site * BATCH_ROWS * d : S[rr].proj + d;
+        q.kr[rr] = kp[td];
+        q.ev[rr] = ep[td];
+    }
+    if constexpr (PHI) load_phi<PC, RP, MF>(D, N, q);
     return q;
 }
 
-template <int PC, bool MF>
-__device__ __forceinline__ void load_phi(const Dims& D, const LayerDev& N, InRegs<PC>& q) {
+template <int PC, int RP, bool MF>
+__device__ __forceinline__ void load_phi(const Dims& D, const LayerDev& N, InRegs<PC, RP>& q) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nc = MHC_LANES * D.d;
     if constexpr (MF) {
         const int h = phi_holder(__builtin_amdgcn_readfirstlane(wave));
@@ -1001,271 +1037,356 @@ __device__ __forceinline__ int dot_row(const uint4* r, const int8_t* x8, int per
 }
 
 // The mHC read, engram gate, input norm and A8 of layer N
-// (step.rs:400-479).  xl holds the thread's element of the 4 lanes (t < d);
-// their transposed copy and the wavefronts' maxima of |xs| are in LDS
-// behind a barrier.  The post and residual
-// gates of the layer (hpost, the Sinkhorn hres) are computed beside its
-// units, off this kernel's path.
-template <bool LATE_PHI, int PC, bool MF>
-__device__ void layer_in(const Dims& D, const SessDev& S, const LayerDev& N, InRegs<PC> q, int in_bits,
-                         LayerShared& sh, const float (&xl)[MHC_LANES]) {
+// (step.rs:400-479).  xl holds the thread's element of the rows' 4 lanes
+// (t < d); their transposed copies and the wavefronts' maxima of |xs| are in
+// LDS behind a barrier.  live[rr]: row rr exists (else nothing of it is
+// stored).  The post and residual gates of the layer (hpost, the Sinkhorn
+// hres) are computed beside its units, off this kernel's path.
+template <bool LATE_PHI, int PC, bool MF, int RP>
+__device__ void layer_in(const Dims& D, const SessDev (&S)[RP], const LayerDev& N, InRegs<PC, RP> q, int in_bits,
+                         LayerShared<RP>& sh, const float (&xl)[RP][MHC_LANES], const bool (&live)[RP]) {
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63, d = D.d, nc = MHC_LANES * d;
-    // (the Phi8 rows read now land while wavefront 0 runs the norm chain)
-    if constexpr (LATE_PHI) load_phi<PC, MF>(D, N, q);
+    // (the Phi8 rows read now land while the norm chain runs)
+    if constexpr (LATE_PHI) load_phi<PC, RP, MF>(D, N, q);
     // every wavefront: r = rinv(dot16(xs)), the amax over the wavefronts'
     // maxima of |xs| (rounding is monotonic, so max_i |xs_i r| =
     // max_i |xs_i| r for r > 0), then the int8 lanes
     {
-        const float r = block_rinv_t(sh.tX, TP_X, nc, &sh.r_a);
-        float m = sh.red[0];
+        float r[RP];
+        block_rinv_t<RP>(sh, [](LayerRow& R) { return R.tX; }, TP_X, nc, [](LayerRow& R) -> float& { return R.r_a; }, r);
 #pragma unroll
-        for (int i = 1; i < LT / 64; ++i) m = fmaxf(m, sh.red[i]);
-        m = m * r;
-        const float sx = m > 0.0f ? m * bits_f32(0x3c010204u) : 1.0f;
-        const float inv = 1.0f / sx;
-        if (t < d) {
+        for (int rr = 0; rr < RP; ++rr) {
+            LayerRow& R = sh.row[rr];
+            float m = R.red[0];
 #pragma unroll
-            for (int b = 0; b < MHC_LANES; ++b) sh.nx8[b * d + t] = quant_one(xl[b] * r, inv);
+            for (int i = 1; i < LT / 64; ++i) m = fmaxf(m, R.red[i]);
+            m = m * r[rr];
+            const float sx = m > 0.0f ? m * bits_f32(0x3c010204u) : 1.0f;
+            const float inv = 1.0f / sx;
+            if (t < d) {
+#pragma unroll
+                for (int b = 0; b < MHC_LANES; ++b) R.nx8[b * d + t] = quant_one(xl[rr][b] * r[rr], inv);
+            }
+            if (t == 0) R.r_sx = sx;
         }
-        if (t == 0) sh.r_sx = sx;
     }
     __syncthreads();
     // Phi8 rows: p[k] = (sx * s_k) * idot(phi_q[k], nx8)
-    {
-        const float sx = sh.r_sx;
+#pragma unroll
+    for (int rr = 0; rr < RP; ++rr) {
+        LayerRow& R = sh.row[rr];
+        const float sx = R.r_sx;
         const int per = nc / 16;
         if constexpr (MF) {
             const int h = phi_holder(wave);
             if (h >= 0) {
-                const int acc = dot_row<PC>(q.r0, sh.nx8, per, lane);
-                const int acc1 = dot_row<PC>(q.r1, sh.nx8, per, lane);
+                const int acc = dot_row<PC>(q.r0, R.nx8, per, lane);
+                const int acc1 = dot_row<PC>(q.r1, R.nx8, per, lane);
                 if (lane == 0) {
-                    sh.p[h] = (sx * q.ps0) * (float)acc;
-                    sh.p[h + PHI_MF] = (sx * q.ps1) * (float)acc1;
+                    R.p[h] = (sx * q.ps0) * (float)acc;
+                    R.p[h + PHI_MF] = (sx * q.ps1) * (float)acc1;
                 }
                 if (h + 2 * PHI_MF < MHC_COLS) {
-                    const int acc2 = dot_row<PC>(q.r2, sh.nx8, per, lane);
-                    if (lane == 0) sh.p[h + 2 * PHI_MF] = (sx * q.ps2) * (float)acc2;
+                    const int acc2 = dot_row<PC>(q.r2, R.nx8, per, lane);
+                    if (lane == 0) R.p[h + 2 * PHI_MF] = (sx * q.ps2) * (float)acc2;
                 }
             }
         } else if (wave >= 1) {
-            const int acc = dot_row<PC>(q.r0, sh.nx8, per, lane);
-            if (lane == 0) sh.p[wave - 1] = (sx * q.ps0) * (float)acc;
+            const int acc = dot_row<PC>(q.r0, R.nx8, per, lane);
+            if (lane == 0) R.p[wave - 1] = (sx * q.ps0) * (float)acc;
             if (wave - 1 + PHI_B < MHC_COLS) {
-                const int acc1 = dot_row<PC>(q.r1, sh.nx8, per, lane);
-                if (lane == 0) sh.p[wave - 1 + PHI_B] = (sx * q.ps1) * (float)acc1;
+                const int acc1 = dot_row<PC>(q.r1, R.nx8, per, lane);
+                if (lane == 0) R.p[wave - 1 + PHI_B] = (sx * q.ps1) * (float)acc1;
             }
         }
     }
     __syncthreads();
-    // The pre gate hp (sigmoid) in every wavefront, then u and x1.
-    float hp[MHC_LANES];
+    // The pre gate hp (sigmoid) in every wavefront (lane 4 rr + b: row rr,
+    // lane b), then u and x1.
+    float hp[RP][MHC_LANES];
     {
         float g = 0.0f;
-        if (lane < MHC_LANES) {
-            const float off = lane == N.lane ? 4.0f : -4.0f;
-            const float zz = ((sh.p[lane] * N.a_pre) + off) + N.b_pre[lane];
+        if (lane < RP * MHC_LANES) {
+            const int b = lane & (MHC_LANES - 1);
+            const float off = b == N.lane ? 4.0f : -4.0f;
+            const float zz = ((sh.row[RP == 1 ? 0 : lane / MHC_LANES].p[b] * N.a_pre) + off) + N.b_pre[b];
             g = 1.0f / (lexpf(-zz) + 1.0f);
         }
 #pragma unroll
-        for (int b = 0; b < MHC_LANES; ++b)
-            hp[b] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, g), b));
-    }
-    float u = 0.0f, x1 = 0.0f;
-    if (t < d) {
-        u = xl[0] * hp[0];
+        for (int rr = 0; rr < RP; ++rr)
 #pragma unroll
-        for (int b = 1; b < MHC_LANES; ++b) u = __builtin_fmaf(xl[b], hp[b], u);
-        x1 = u;
-        put_t(sh.tA, TP_D, t, x1);
-        if (N.site >= 0) put_t(sh.tB, TP_D, t, q.kr);
+            for (int b = 0; b < MHC_LANES; ++b)
+                hp[rr][b] = __builtin_bit_cast(
+                    float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, g), rr * MHC_LANES + b));
+    }
+    float u[RP] = {}, x1[RP] = {};
+    if (t < d) {
+#pragma unroll
+        for (int rr = 0; rr < RP; ++rr) {
+            u[rr] = xl[rr][0] * hp[rr][0];
+#pragma unroll
+            for (int b = 1; b < MHC_LANES; ++b) u[rr] = __builtin_fmaf(xl[rr][b], hp[rr][b], u[rr]);
+            x1[rr] = u[rr];
+            put_t(sh.row[rr].tA, TP_D, t, x1[rr]);
+            if (N.site >= 0) put_t(sh.row[rr].tB, TP_D, t, q.kr[rr]);
+        }
     }
     __syncthreads();
     if (N.site >= 0) {
         // alpha = sigmoid(dot16(x1 / |x1|, k / |k|) / sqrt(d)); x1 += alpha * conv
-        if (wave == 1) {
-            const float rk = rinv(dot16_t<true>(sh.tB, sh.tB, TP_D, d, lane), d);
-            if (lane == 0) sh.r_b = rk;
+        if (wave >= RP && wave < 2 * RP) {
+            LayerRow& R = sh.row[RP == 1 ? 0 : __builtin_amdgcn_readfirstlane(wave - RP)];
+            const float rk = rinv(dot16_t<true>(R.tB, R.tB, TP_D, d, lane), d);
+            if (lane == 0) R.r_b = rk;
         }
-        const float rx = block_rinv_t(sh.tA, TP_D, d, &sh.r_a);
-        const float rk = sh.r_b;
+        float rx[RP];
+        block_rinv_t<RP>(sh, [](LayerRow& R) { return R.tA; }, TP_D, d, [](LayerRow& R) -> float& { return R.r_a; }, rx);
         if (t < d) {
-            put_t(sh.tA, TP_D, t, x1 * rx);
-            put_t(sh.tB, TP_D, t, q.kr * rk);
+#pragma unroll
+            for (int rr = 0; rr < RP; ++rr) {
+                const float rk = sh.row[rr].r_b;
+                put_t(sh.row[rr].tA, TP_D, t, x1[rr] * rx[rr]);
+                put_t(sh.row[rr].tB, TP_D, t, q.kr[rr] * rk);
+            }
         }
         __syncthreads();
-        if (wave == 0) {
-            const float dd = dot16_t<false>(sh.tA, sh.tB, TP_D, d, lane);
-            if (lane == 0) sh.r_c = 1.0f / (lexpf((-dd) / __builtin_sqrtf((float)d)) + 1.0f);
+        if (wave < RP) {
+            LayerRow& R = sh.row[RP == 1 ? 0 : __builtin_amdgcn_readfirstlane(wave)];
+            const float dd = dot16_t<false>(R.tA, R.tB, TP_D, d, lane);
+            if (lane == 0) R.r_c = 1.0f / (lexpf((-dd) / __builtin_sqrtf((float)d)) + 1.0f);
         }
         __syncthreads();
-        const float alpha = sh.r_c;
         if (t < d) {
-            x1 = __builtin_fmaf(q.ev, alpha, x1);
-            put_t(sh.tA, TP_D, t, x1);
+#pragma unroll
+            for (int rr = 0; rr < RP; ++rr) {
+                x1[rr] = __builtin_fmaf(q.ev[rr], sh.row[rr].r_c, x1[rr]);
+                put_t(sh.row[rr].tA, TP_D, t, x1[rr]);
+            }
         }
         __syncthreads();
     }
     // hloc = norm_apply16(x1, rinv(dot16(x1)), norm_in), then A8.
     {
-        const float r = block_rinv_t(sh.tA, TP_D, d, &sh.r_b);
+        float r[RP];
+        block_rinv_t<RP>(sh, [](LayerRow& R) { return R.tA; }, TP_D, d, [](LayerRow& R) -> float& { return R.r_b; }, r);
         if (t < d) {
-            const float tt = x1 * r;
-            sh.h[t] = __builtin_fmaf(tt, h2f_late(q.norm), tt);
-            S.u[t] = u;
-            S.x1[t] = x1;
+#pragma unroll
+            for (int rr = 0; rr < RP; ++rr) {
+                const float tt = x1[rr] * r[rr];
+                sh.row[rr].h[t] = __builtin_fmaf(tt, h2f_late(q.norm), tt);
+                if (RP == 1 || live[rr]) {
+                    S[rr].u[t] = u[rr];
+                    S[rr].x1[t] = x1[rr];
+                }
+            }
         }
     }
-    if (t < MHC_COLS) S.p[t] = sh.p[t];
+    if (t < MHC_COLS) {
+#pragma unroll
+        for (int rr = 0; rr < RP; ++rr)
+            if (RP == 1 || live[rr]) S[rr].p[t] = sh.row[rr].p[t];
+    }
     __syncthreads();
     const int groups = (d + GROUP - 1) / GROUP;
-    for (int g = wave; g < groups; g += LT / 64) {
-        const int p0 = g * GROUP + lane, p1 = p0 + 64;
-        a8_group(p0 < d ? sh.h[p0] : 0.0f, p1 < d ? sh.h[p1] : 0.0f, lane, in_bits, S.xq_in + (size_t)g * GROUP,
-                 S.sx_in + g);
+#pragma unroll
+    for (int rr = 0; rr < RP; ++rr) {
+        if (RP > 1 && !live[rr]) continue;
+        // (row 1 on wavefronts 8 up, then 0 up)
+        for (int g = (wave + LT / 64 - rr * 8) % (LT / 64); g < groups; g += LT / 64) {
+            const int p0 = g * GROUP + lane, p1 = p0 + 64;
+            a8_group(p0 < d ? sh.row[rr].h[p0] : 0.0f, p1 < d ? sh.row[rr].h[p1] : 0.0f, lane, in_bits,
+                     S[rr].xq_in + (size_t)g * GROUP, S[rr].sx_in + g);
+        }
     }
 }
 
 // The head's input (step.rs:706-728, chunk.rs:331-347): lane mean, zcn with
-// the f32 final norm into `hid`, A8 into activation row `arow`.
-__device__ void head_in(const Dims& D, const SessDev& S, float fnorm, int head_bits, int arow, LayerShared& sh,
-                        const float (&xl)[MHC_LANES]) {
+// the f32 final norm into `hid`, A8 into activation row `arow`; rows not
+// wanted (want[rr]) store nothing; the launch's last row (last[rr]) is
+// NatState::last_hidden too.
+template <int RP>
+__device__ void head_in(const Dims& D, const SessDev& S, float fnorm, int head_bits, const int (&arow)[RP],
+                        const bool (&want)[RP], const bool (&last)[RP], LayerShared<RP>& sh,
+                        const float (&xl)[RP][MHC_LANES]) {
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63, d = D.d;
-    float mean = 0.0f;
+    float mean[RP] = {};
     if (t < d) {
-        mean = (((xl[0] + xl[1]) + xl[2]) + xl[3]) * 0.25f;
-        put_t(sh.tA, TP_D, t, mean);
+#pragma unroll
+        for (int rr = 0; rr < RP; ++rr) {
+            mean[rr] = (((xl[rr][0] + xl[rr][1]) + xl[rr][2]) + xl[rr][3]) * 0.25f;
+            put_t(sh.row[rr].tA, TP_D, t, mean[rr]);
+        }
     }
     __syncthreads();
     {
-        const float r = block_rinv_t(sh.tA, TP_D, d, &sh.r_a);
+        float r[RP];
+        block_rinv_t<RP>(sh, [](LayerRow& R) { return R.tA; }, TP_D, d, [](LayerRow& R) -> float& { return R.r_a; }, r);
         if (t < d) {
-            const float tt = mean * r;
-            const float h = __builtin_fmaf(tt, fnorm, tt);
-            sh.x2[t] = h;
-            S.hid[(size_t)arow * d + t] = h;
-            // NatState::last_hidden: the last row returned (the launch's last block)
-            if (blockIdx.x == gridDim.x - 1) S.last_hid[t] = h;
+#pragma unroll
+            for (int rr = 0; rr < RP; ++rr) {
+                const float tt = mean[rr] * r[rr];
+                const float h = __builtin_fmaf(tt, fnorm, tt);
+                sh.row[rr].x2[t] = h;
+                if (want[rr]) S.hid[(size_t)arow[rr] * d + t] = h;
+                if (want[rr] && last[rr]) S.last_hid[t] = h;
+            }
         }
     }
     __syncthreads();
     const int groups = (d + GROUP - 1) / GROUP;
-    for (int g = wave; g < groups; g += LT / 64) {
-        const int p0 = g * GROUP + lane, p1 = p0 + 64;
-        a8_group(p0 < d ? sh.x2[p0] : 0.0f, p1 < d ? sh.x2[p1] : 0.0f, lane, head_bits,
-                 S.xq_in + ((size_t)arow * groups + g) * GROUP, S.sx_in + (size_t)arow * groups + g);
+#pragma unroll
+    for (int rr = 0; rr < RP; ++rr) {
+        if (!want[rr]) continue;
+        for (int g = (wave + LT / 64 - rr * 8) % (LT / 64); g < groups; g += LT / 64) {
+            const int p0 = g * GROUP + lane, p1 = p0 + 64;
+            a8_group(p0 < d ? sh.row[rr].x2[p0] : 0.0f, p1 < d ? sh.row[rr].x2[p1] : 0.0f, lane, head_bits,
+                     S.xq_in + ((size_t)arow[rr] * groups + g) * GROUP, S.sx_in + (size_t)arow[rr] * groups + g);
+        }
     }
 }
 
 }  // namespace
 
-// BATCH (a feed of several rows): two rows per CU (at most 64 VGPRs), so
-// the next layer's Phi8 rows are read at the start of the mHC read instead
-// of beside the MLP.
+// RP rows per workgroup, one workgroup a CU.  Almost every phase is a short
+// serial chain or a barrier, so a second row costs little beside the first:
+// its chains run on other wavefronts, its elementwise work on the same
+// threads, and the tables and Phi8 rows are read once for both.
 //
 // The operands of everything the first barrier waits for lead the arguments
 // as scalars (the previous layer's staged tables and post norm, the row
 // buffers, d and row0), so they are preloaded into SGPRs at wave launch.
-template <bool PREV, bool NEXT, bool BATCH, int PC>
-__global__ __launch_bounds__(LT) __attribute__((amdgpu_waves_per_eu(BATCH ? 8 : 1))) void k_layer(
+template <bool PREV, bool NEXT, int RP, int PC>
+__global__ __launch_bounds__(LT) void k_layer(
     const uint4* stage, const float* o, const float* p, float* xs, const float* x1, const float* u, int d, int row0,
-    Dims D, Globals G, SessDev S, LayerDev P, LayerDev N, int in_bits, int head_bits, int head_row0) {
-    constexpr bool has_prev = PREV, has_next = NEXT;
-    __shared__ LayerShared sh;
+    int rows, Dims D, Globals G, SessDev S, LayerDev P, LayerDev N, int in_bits, int head_bits, int head_row0) {
+    constexpr bool has_prev = PREV, has_next = NEXT, MF = RP == 1;
+    __shared__ LayerShared<RP> sh;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nc = MHC_LANES * d;
     const int Gd = (d + GROUP - 1) / GROUP;
-    // this block's row of every row buffer
-    const int row = row0 + blockIdx.x;
-    SessDev R = S;
-    R.xs = xs + (size_t)row * nc;
-    R.u = const_cast<float*>(u) + (size_t)row * d;
-    R.x1 = const_cast<float*>(x1) + (size_t)row * d;
-    R.p = const_cast<float*>(p) + (size_t)row * 64;
-    R.o = const_cast<float*>(o) + (size_t)row * d;
-    R.ekv += (size_t)row * 2 * d;
-    R.evals += (size_t)row * d;
-    R.xq_in += (size_t)row * Gd * GROUP;
-    R.sx_in += (size_t)row * Gd;
+    // this block's rows of every row buffer (a row past the last one reads
+    // the last and stores nothing)
+    SessDev R[RP];
+    bool live[RP];
+    int rix[RP];
+#pragma unroll
+    for (int rr = 0; rr < RP; ++rr) {
+        const int i = (int)blockIdx.x * RP + rr;
+        live[rr] = RP == 1 || i < rows;
+        rix[rr] = RP == 1 ? i : min(i, rows - 1);
+        const int row = row0 + rix[rr];
+        R[rr] = S;
+        R[rr].xs = xs + (size_t)row * nc;
+        R[rr].u = const_cast<float*>(u) + (size_t)row * d;
+        R[rr].x1 = const_cast<float*>(x1) + (size_t)row * d;
+        R[rr].p = const_cast<float*>(p) + (size_t)row * 64;
+        R[rr].o = const_cast<float*>(o) + (size_t)row * d;
+        R[rr].ekv += (size_t)row * 2 * d;
+        R[rr].evals += (size_t)row * d;
+        R[rr].xq_in += (size_t)row * Gd * GROUP;
+        R[rr].sx_in += (size_t)row * Gd;
+    }
     // every global read first, then the LDS stores; thread t < d holds
     // element t of each lane
     const int td = min(t, d - 1);
-    float xl[MHC_LANES];
+    float xl[RP][MHC_LANES];
 #pragma unroll
-    for (int k = 0; k < MHC_LANES; ++k) xl[k] = R.xs[k * d + td];
-    OutRegs qo;
-    if constexpr (has_prev) qo = load_out(d, stage, P.post_norm, G, R, P);
-    InRegs<PC> qi;
+    for (int rr = 0; rr < RP; ++rr)
+#pragma unroll
+        for (int k = 0; k < MHC_LANES; ++k) xl[rr][k] = R[rr].xs[k * d + td];
+    OutRegs<RP> qo;
+    if constexpr (has_prev) qo = load_out<RP>(d, stage, P.post_norm, G, R, P);
+    InRegs<PC, RP> qi;
     float fnorm = 0.0f;
     // Without a previous layer nothing else loads: the next layer's reads
     // go now.  With one they go after the first barrier: the Phi8 rows are
     // half the kernel's bytes and are not needed before the mHC read, so
     // they stay out of the way of the tables the MLP waits for.
-    if constexpr (has_next && !has_prev) qi = load_in<!BATCH, PC, !BATCH>(D, R, N);
+    if constexpr (has_next && !has_prev) qi = load_in<MF, PC, MF, RP>(D, R, N);
     if constexpr (!has_next) fnorm = G.final_norm[min(t, d - 1)];
-    float m = 0.0f;
-    if (t == 0) sh.mix_count = 0;
+    float m[RP] = {};
+    if (t < RP) sh.row[t].mix_count = 0;
     // With a previous layer the lanes' transposed copy is written by its
-    // mHC write (over the MLP's buffers, which store_out fills now).
+    // mHC write (over the MLP's buffers).
     if constexpr (!has_prev) {
         if (t < d) {
 #pragma unroll
-            for (int k = 0; k < MHC_LANES; ++k) {
-                put_t(sh.tX, TP_X, k * d + t, xl[k]);
-                m = fmaxf(m, fabsf(xl[k]));
-            }
+            for (int rr = 0; rr < RP; ++rr)
+#pragma unroll
+                for (int k = 0; k < MHC_LANES; ++k) {
+                    put_t(sh.row[rr].tX, TP_X, k * d + t, xl[rr][k]);
+                    m[rr] = fmaxf(m[rr], fabsf(xl[rr][k]));
+                }
         }
     }
-    if constexpr (has_prev) store_out(d, qo, sh);
+    if constexpr (has_prev) store_out<RP>(d, qo, sh);
     __syncthreads();
-    if constexpr (has_next && has_prev) qi = load_in<false, PC, !BATCH>(D, R, N);
+    if constexpr (has_next && has_prev) qi = load_in<false, PC, MF, RP>(D, R, N);
     // The Phi8 rows (72 KB at d = 768, ~16 cycles of the CU's address unit
     // per 1 KB wavefront load): one row alone issues them where wavefront 0
     // runs cond_weights, the longest chain of the MLP, and the other
     // wavefronts wait for it anyway (issued right after the first barrier
-    // they held the post norm's barrier back); batched, once the MLP's
-    // registers are free.
+    // they held the post norm's barrier back); two rows, whose mixers are
+    // eight wavefronts, once the MLP is done.
     if constexpr (has_prev)
-        m = layer_out(
-            D, S, P, qo, sh, xl,
+        layer_out<RP>(
+            D, S, P, qo, sh, xl, m,
             [&]() __attribute__((always_inline)) {
-                if constexpr (has_next && !BATCH) load_phi<PC, true>(D, N, qi);
+                if constexpr (has_next && MF) load_phi<PC, RP, true>(D, N, qi);
             },
             [&]() __attribute__((always_inline)) {
-                if constexpr (has_next && BATCH) load_phi<PC, false>(D, N, qi);
+                if constexpr (has_next && !MF) load_phi<PC, RP, false>(D, N, qi);
             });
     // the wavefronts' maxima of |xs| for the mHC read
-    m = wave_max_nonneg(m);
-    if (lane == 0) sh.red[wave] = m;
+#pragma unroll
+    for (int rr = 0; rr < RP; ++rr) {
+        const float mw = wave_max_nonneg(m[rr]);
+        if (lane == 0) sh.row[rr].red[wave] = mw;
+    }
     __syncthreads();
     // (the new lanes go back to HBM last: nothing here reads them there, and
     // stores issued earlier would sit in the memory counter ahead of loads
     // that are waited for)
-    if constexpr (has_next)
-        layer_in<BATCH && !has_prev, PC, !BATCH>(D, R, N, qi, in_bits, sh, xl);
-    else if ((int)blockIdx.x >= head_row0)  // (uniform over the block)
-        head_in(D, S, fnorm, head_bits, blockIdx.x - head_row0, sh, xl);  // row i - row0 - head_row0
+    if constexpr (has_next) {
+        layer_in<!MF && !has_prev, PC, MF, RP>(D, R, N, qi, in_bits, sh, xl, live);
+    } else {
+        // rows i >= head_row0 into activation row i - head_row0 (block-uniform)
+        int arow[RP];
+        bool want[RP], last[RP], any = false;
+#pragma unroll
+        for (int rr = 0; rr < RP; ++rr) {
+            arow[rr] = rix[rr] - head_row0;
+            want[rr] = live[rr] && arow[rr] >= 0;
+            last[rr] = rix[rr] == rows - 1;
+            any |= want[rr];
+        }
+        if (any) head_in<RP>(D, S, fnorm, head_bits, arow, want, last, sh, xl);
+    }
     if constexpr (has_prev) {
         if (t < d) {
 #pragma unroll
-            for (int k = 0; k < MHC_LANES; ++k) R.xs[k * d + t] = xl[k];
-            // the cell of layer P: the lane mean after its mHC write
-            // (step.rs:672-694, chunk.rs:310, lane_mean infer.rs:1707-1711)
-            if (S.cells)
-                S.cells[((size_t)row * (D.layers + 1) + P.index + 1) * d + t] =
-                    (((xl[0] + xl[1]) + xl[2]) + xl[3]) * 0.25f;
+            for (int rr = 0; rr < RP; ++rr) {
+                if (RP > 1 && !live[rr]) continue;
+#pragma unroll
+                for (int k = 0; k < MHC_LANES; ++k) R[rr].xs[k * d + t] = xl[rr][k];
+                // the cell of layer P: the lane mean after its mHC write
+                // (step.rs:672-694, chunk.rs:310, lane_mean infer.rs:1707-1711)
+                if (S.cells)
+                    S.cells[((size_t)(row0 + rix[rr]) * (D.layers + 1) + P.index + 1) * d + t] =
+                        (((xl[rr][0] + xl[rr][1]) + xl[rr][2]) + xl[rr][3]) * 0.25f;
+            }
         }
     }
 }
 
-template <bool BATCH, int PC>
+template <int RP, int PC>
 static void launch_layer(const Dims& D, const Globals& G, const SessDev& S, const LayerDev* prev,
                          const LayerDev* next, int row0, int rows, int in_bits, int head_bits, int head_row0,
                          hipStream_t s) {
     const LayerDev none{};
     const uint4* stage = prev ? reinterpret_cast<const uint4*>(prev->stage) : nullptr;
 #define NH_LAYER(HP, HN, PV, NX)                                                                                  \
-    hipLaunchKernelGGL((k_layer<HP, HN, BATCH, PC>), dim3(rows), dim3(LT), 0, s, stage, S.o, S.p, S.xs, S.x1,     \
-                       S.u, D.d, row0, D, G, S, PV, NX, in_bits, head_bits, head_row0)
+    hipLaunchKernelGGL((k_layer<HP, HN, RP, PC>), dim3((rows + RP - 1) / RP), dim3(LT), 0, s, stage, S.o, S.p,    \
+                       S.xs, S.x1, S.u, D.d, row0, rows, D, G, S, PV, NX, in_bits, head_bits, head_row0)
     if (prev && next)
         NH_LAYER(true, true, *prev, *next);
     else if (next)
@@ -1279,18 +1400,13 @@ static void launch_layer(const Dims& D, const Globals& G, const SessDev& S, cons
 
 hipError_t fwd_layer(const Dims& D, const Globals& G, const SessDev& S, const LayerDev* prev, const LayerDev* next,
                      int row0, int rows, int in_bits, int head_bits, hipStream_t s, int head_row0) {
-    // A feed's 64-VGPR kernel sized for a Phi8 row of at most three 1 KB
-    // chunks (d <= 768: no spills) or of four.  The one-row kernel has no
-    // register cap and keeps the four-chunk form (measured no faster with
-    // three).
-    if (rows > 1) {
-        if (MHC_LANES * D.d <= 3 * 1024)
-            launch_layer<true, 3>(D, G, S, prev, next, row0, rows, in_bits, head_bits, head_row0, s);
-        else
-            launch_layer<true, PHI_CHUNKS>(D, G, S, prev, next, row0, rows, in_bits, head_bits, head_row0, s);
-    } else {
-        launch_layer<false, PHI_CHUNKS>(D, G, S, prev, next, row0, rows, in_bits, head_bits, head_row0, s);
-    }
+    // One row per workgroup while that leaves no CU with two, else two.
+    const bool narrow = MHC_LANES * D.d <= 3 * 1024;
+    auto go = [&](auto launch) { launch(D, G, S, prev, next, row0, rows, in_bits, head_bits, head_row0, s); };
+    if (rows <= device_cus())
+        narrow ? go(launch_layer<1, 3>) : go(launch_layer<1, PHI_CHUNKS>);
+    else
+        narrow ? go(launch_layer<2, 3>) : go(launch_layer<2, PHI_CHUNKS>);
     return hipGetLastError();
 }
 
@@ -1817,7 +1933,7 @@ __global__ __launch_bounds__(ATT_THREADS) void k_attend(Dims D, SessDev S, Layer
     wmax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     const float qw = bits_f32(0x49fffff8u) / wmax;
     for (int i = t; i < len; i += ATT_THREADS) {
-        const int32_t wq = (int32_t)roundf(sc[i] * qw);
+        const int32_t wq = round_digits(sc[i] * qw);
         dig[0][sh + i] = (int8_t)(wq >> 14);
         dig[1][sh + i] = (int8_t)((wq >> 7) & 127);
         dig[2][sh + i] = (int8_t)(wq & 127);
@@ -2204,7 +2320,7 @@ __global__ __launch_bounds__(AG_T * RP) __attribute__((amdgpu_waves_per_eu(RP ==
         for (int j = 0; j < AG_KPL; ++j) {
             const int i = lane + 64 * j;
             if (i < len) {
-                const int32_t wq = (int32_t)roundf(e[j] * qwt);
+                const int32_t wq = round_digits(e[j] * qwt);
                 const int c = key_col(i);
                 dg[0][c] = (int8_t)(wq >> 14);
                 dg[1][c] = (int8_t)((wq >> 7) & 127);
@@ -2643,7 +2759,7 @@ __global__ __launch_bounds__(DG_THREADS) void k_dec_group(const int8_t* k8l, con
         const float qw = bits_f32(0x49fffff8u) / wmax;
         for (int i = u; i < n; i += DG_HEAD_T) {
             const float w = sc[h][i] * vss[i];
-            const int32_t wq = (int32_t)roundf(w * qw);
+            const int32_t wq = round_digits(w * qw);
             dig[h][0][sh + i] = (int8_t)(wq >> 14);
             dig[h][1][sh + i] = (int8_t)((wq >> 7) & 127);
             dig[h][2][sh + i] = (int8_t)(wq & 127);
@@ -3112,7 +3228,7 @@ __global__ __launch_bounds__(DG_THREADS) void k_dec_chunks(Dims D, SessDev S, La
         const float qw = bits_f32(0x49fffff8u) / wmax;
         for (int i = u; i < len; i += DG_HEAD_T) {
             const float w = sc[h][i] * vss[i];
-            const int32_t wq = (int32_t)roundf(w * qw);
+            const int32_t wq = round_digits(w * qw);
             dig[h][0][sh + i] = (int8_t)(wq >> 14);
             dig[h][1][sh + i] = (int8_t)((wq >> 7) & 127);
             dig[h][2][sh + i] = (int8_t)(wq & 127);

@@ -314,8 +314,8 @@ int build_model(nh_model* m, const nh::ArchiveSmall& sm) {
         return A.put(b.data(), b.size() * 2);
     };
     // The tables of the layer kernel, as one block per layer: the six
-    // Kronecker factors (MFMA fragments) and cond_v [d][8] (staged into LDS), then cond_u
-    // by column, [hada_n][8] (f16; thread t reads its column's 16 bytes).
+    // Kronecker factors (f16 MFMA fragments) and cond_v by chain (f32), staged
+    // into LDS, then cond_u by column, [hada_n][8] (f16; thread t reads its column's 16 bytes).
     std::vector<size_t> stage(D.layers);
     for (int l = 0; l < D.layers; ++l) {
         for (int k = 0; k < nh::SMALL_KINDS; ++k) off[l].t[k] = put16(sm.layer[l][k]);
@@ -329,12 +329,25 @@ int build_model(nh_model* m, const nh::ArchiveSmall& sm) {
                     for (int st = 0; st < 8; ++st)
                         blk.push_back(f[(4 * st + lane / 16) * nh::HADA_NB + tile * 16 + lane % 16]);
         }
+        std::vector<uint16_t> st(blk.size());
+        for (size_t i = 0; i < blk.size(); ++i) st[i] = f32_to_f16(blk[i]);
+        // (f32 of the f16 values the reference holds, so the chains need no
+        // conversions; chain 8 jm + k holds elements [4 u + jm][k], u in order)
         const auto& cv = sm.layer[l][nh::S_COND_V];
-        blk.insert(blk.end(), cv.begin(), cv.begin() + (size_t)D.d * nh::COND_RANK);
+        for (int jm = 0; jm < 4; ++jm)
+            for (int k = 0; k < nh::COND_RANK; ++k)
+                for (int u = 0; u < nh::FWD_MAX_D / 4; ++u) {
+                    const int j = 4 * u + jm;
+                    const _Float16 f = (_Float16)(j < D.d ? cv[(size_t)j * nh::COND_RANK + k] : 0.0f);
+                    const float v = (float)f;
+                    uint16_t h[2];
+                    memcpy(h, &v, 4);
+                    st.insert(st.end(), h, h + 2);
+                }
         const auto& cu = sm.layer[l][nh::S_COND_U];
         for (int t = 0; t < nh::HADA_N; ++t)
-            for (int k = 0; k < nh::COND_RANK; ++k) blk.push_back(cu[(size_t)k * nh::HADA_N + t]);
-        stage[l] = put16(blk);
+            for (int k = 0; k < nh::COND_RANK; ++k) st.push_back(f32_to_f16(cu[(size_t)k * nh::HADA_N + t]));
+        stage[l] = A.put(st.data(), st.size() * 2);
         off[l].phi_q = A.reserve((size_t)nh::MHC_COLS * nc);
         off[l].phi_s = A.reserve(nh::MHC_COLS * 4);
     }
