@@ -76,7 +76,7 @@ struct LayerDev {
     const uint16_t* stage;  // the six Kronecker factors (MFMA fragments), cond_v by chain (f32), cond_u [1024][8]
     const uint16_t *d1, *d2, *b2, *d3, *d4;
     const uint16_t *norm_in, *post_norm, *pre_hada, *q_taps, *k_taps, *v_taps, *q_norm, *k_norm;
-    const int8_t* phi_q;  // [24][lanes * d]
+    const int8_t* phi_q;  // [24 x lanes * d], in MFMA fragment order (phi_at)
     const float* phi_s;   // [24]
     float a_pre, a_post, a_res;
     float ga;             // sigmoid(attn_gate), f32 expf on the host
@@ -197,6 +197,7 @@ bool dec_chunks_fits(const Dims& D);
 hipError_t fwd_dec_chunks(const Dims& D, const SessDev& S, const LayerDev& L, int layer, int p0, int out_bits,
                           const KeySpan* span, hipStream_t s);
 hipError_t fwd_argmax(const float* logits, int n, uint32_t* dst, hipStream_t s);
+// (nrows at most 24; q in phi_at's order)
 hipError_t fwd_phi8(const float* rows, int nrows, int width, int8_t* q, float* scale, hipStream_t s);
 
 }  // namespace nh

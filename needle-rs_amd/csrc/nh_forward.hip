@@ -419,6 +419,7 @@ struct LayerRow {
     alignas(16) float hT[4 * TP_H];
     float red[LT / 64];
     float p[64];
+    int psum[MHC_COLS];  // the Phi8 dots' partial sums
     float wk[COND_RANK];
     float r_sx, r_a, r_b, r_c;
     int mix_count;  // the row's mixer wavefronts' arrivals (mixer_sync)
@@ -721,6 +722,17 @@ __device__ __forceinline__ OutRegs<RP> load_out(int d, const uint4* stage, const
     return q;
 }
 
+// The wait for the weights read so far, before the Phi8 rows are issued: the
+// compiler counts loads issued in a branch as possibly none, so a later use
+// of an earlier load would wait for the rows as well.
+template <int RP>
+__device__ __forceinline__ void settle(OutRegs<RP>& q) {
+    asm volatile("" : "+v"(q.d2), "+v"(q.b2), "+v"(q.d3), "+v"(q.d4), "+v"(q.p1), "+v"(q.p2), "+v"(q.cu.x), "+v"(q.cu.y),
+                      "+v"(q.cu.z), "+v"(q.cu.w));
+#pragma unroll
+    for (int rr = 0; rr < RP; ++rr) asm volatile("" : "+v"(q.u[rr]));
+}
+
 // A raw f16 weight as f32 at its use: the empty asm keeps the conversion
 // (and so the wait for the load) from being hoisted up to the load.
 __device__ __forceinline__ float h2f_late(uint32_t b) {
@@ -800,9 +812,9 @@ __device__ __forceinline__ void cond_weights(const float* hT, const float* cvT, 
 // thread's element of the rows' 4 lanes (t < d) and gets the new ones; m gets
 // this thread's max |new lane value| of each row (for the next layer's mHC
 // read).
-template <int RP, typename BeforeMix, typename AfterMlp>
-__device__ void layer_out(const Dims& D, const SessDev& S, const LayerDev& P, const OutRegs<RP>& q, LayerShared<RP>& sh,
-                          float (&xl)[RP][MHC_LANES], float (&m)[RP], BeforeMix before_mix, AfterMlp after_mlp) {
+template <int RP, typename BeforeMix, typename Late>
+__device__ void layer_out(const Dims& D, const SessDev& S, const LayerDev& P, OutRegs<RP>& q, LayerShared<RP>& sh,
+                          float (&xl)[RP][MHC_LANES], float (&m)[RP], BeforeMix before_mix, Late late) {
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63, d = D.d;
     // mix8 runs on waves 4..7 (threads 256..511; row 1: 8..11), beside
     // cond_weights on wave 0 (row 1: wave 1)
@@ -847,6 +859,7 @@ __device__ void layer_out(const Dims& D, const SessDev& S, const LayerDev& P, co
     __syncthreads();
     // cond_weights spans both passes of the first mix8; the mixers of a row
     // meet between their passes on their own
+    settle<RP>(q);
     before_mix();
     if (RP == 1 ? wave == 0 : wave < RP) {
         LayerRow& R = sh.row[RP == 1 ? 0 : __builtin_amdgcn_readfirstlane(wave)];
@@ -884,7 +897,7 @@ __device__ void layer_out(const Dims& D, const SessDev& S, const LayerDev& P, co
     __syncthreads();
     if (mixer) mix8_n(mu, M.B, sh.kf[5], M.C, d / HADA_NB / 8 * 8);
     __syncthreads();
-    after_mlp();
+    if constexpr (RP > 1) late();
     // The mHC write: y = (x2 + t3 * d4) - u; lane a = y hpost[a] + sum_b
     // hres[a][b] old[b] as an fma chain over b.
 #pragma unroll
@@ -911,42 +924,67 @@ __device__ void layer_out(const Dims& D, const SessDev& S, const LayerDev& P, co
     }
 }
 
+// Byte of element i of Phi8 row r (the order of the MFMA fragments): per 64
+// elements, rows 0-15's fragment (lane 16 q + r: elements 16 q ..), then rows
+// 16-23's half of one (16 bytes at 8 q + r - 16).
+constexpr int PHI_STEP = MHC_COLS * 64;
+__device__ __forceinline__ size_t phi_at(int r, int i) {
+    const int q = (i >> 4) & 3;
+    return (size_t)(i >> 6) * PHI_STEP + (r < 16 ? q * 16 + r : 64 + q * 8 + r - 16) * 16 + (i & 15);
+}
+
 // The next layer's weights a thread needs, read up front: its norm scale,
-// engram key / conv element, and its wavefront's Phi8 rows (16 bytes at
-// lane + 64 j of each, j < 4: rows of up to 4096).
-constexpr int PHI_CHUNKS = MHC_LANES * FWD_MAX_D / 16 / 64;
-constexpr int PHI_B = LT / 64 - 1;  // wavefronts holding Phi8 rows
-static_assert(2 * PHI_B >= MHC_COLS, "two Phi8 rows per wavefront cover the 24 rows");
-// The one-row kernel issues the rows beside cond_weights, where the mix8
-// wavefronts (4-7) are busy: there they are held by the other eleven (MF,
-// mixer-free), rows h, h + 11 and, for h < 2, h + 22 on holder h.
-constexpr int PHI_MF = PHI_B - MIX_T / 64;
-static_assert(3 * PHI_MF >= MHC_COLS && 2 * PHI_MF < MHC_COLS, "holders 0 and 1 take a third row");
-__device__ __forceinline__ int phi_holder(int wave) { return wave >= 1 && wave <= 3 ? wave - 1 : wave >= 8 ? wave - 5 : -1; }
-// PC: the 1 KB chunks a Phi8 row has (its 4 d int8 / 1024), fixed at compile
-// time so a narrower model holds no registers for chunks it never reads (3
-// at d = 768).
+// engram key / conv element, and its wavefront's part of the Phi8 rows as
+// MFMA fragments.
+//
+// The 24 projections are int8 dots of length 4 d, exact in any order:
+// v_mfma_i32_16x16x64_i8 with the Phi8 rows as operand A (rows 0-15; rows
+// 16-23 of two k-steps, each half with its own sums) and the rows' int8 lanes
+// as operand B, the k-steps of 64 spread over the holder wavefronts, whose
+// partial sums meet in LDS.  A wavefront reads
+// its 64 bytes of the lanes once a k-step, for all the projections (row by
+// row on the vector ALU every wavefront read all 4 d of them, twice, and ended in
+// a 64-lane reduction a row).
+//
+// Holders: every wavefront of the two-row kernel; of the one-row kernel all
+// but the mixers, which run the MLP's passes when most of the rows are
+// issued.  PC: 1 KB chunks of a Phi8 row (4 d / 1024, rounded up), fixed at
+// compile time so a narrower model holds no registers for k-steps it has not.
+constexpr int PHI_CHUNKS = MHC_LANES * FWD_MAX_D / 1024;
+template <int RP>
+struct Phi {
+    static constexpr int HOLDERS = RP == 1 ? LT / 64 - MIX_T / 64 : LT / 64;
+    static __device__ __forceinline__ int holder(int wave) {
+        if constexpr (RP == 1) return wave < 4 ? wave : wave >= 8 ? wave - 4 : -1;
+        return wave;
+    }
+    // issues its rows beside cond_weights, on the chain's wavefronts too
+    // (issuing wavefront 0's after its chain cost the one-row kernel 2 %: the
+    // MLP's later reads wait behind them); with two rows the mixers and
+    // the chains' wavefronts issue theirs after the MLP
+    static __device__ __forceinline__ bool early(int wave) {
+        if constexpr (RP == 1) return true;
+        return wave == 2 || wave == 3 || wave >= 12;
+    }
+};
 template <int PC, int RP>
 struct InRegs {
+    static constexpr int KS = (PC * 16 + Phi<RP>::HOLDERS - 1) / Phi<RP>::HOLDERS;  // k-steps of a holder
     uint32_t norm;
-    float kr[RP], ev[RP], ps0, ps1, ps2;
-    uint4 r0[PC], r1[PC], r2[PC];
+    float kr[RP], ev[RP], ps;
+    u32x4 f0[KS], f1[(KS + 1) / 2];
 };
 
-template <int PC, int RP, bool MF>
-__device__ __forceinline__ void load_phi(const Dims& D, const LayerDev& N, InRegs<PC, RP>& q);
-
-// PHI: the Phi8 rows too (else layer_in reads them itself).
-template <bool PHI, int PC, bool MF, int RP>
+template <int PC, int RP>
 __device__ __forceinline__ InRegs<PC, RP> load_in(const Dims& D, const SessDev (&S)[RP], const LayerDev& N) {
     const int t = threadIdx.x, d = D.d;
-    // Unconditional loads at clamped addresses (threads, rows and chunks
-    // past the ranges read an in-range element and ignore it; a layer
-    // without an engram site reads the projection row instead, which
-    // nothing else here reads).
+    // Unconditional loads at clamped addresses (threads past the ranges read
+    // an in-range element and ignore it; a layer without an engram site reads
+    // the projection row instead, which nothing else here reads).
     InRegs<PC, RP> q;
     const int td = min(t, d - 1);
     q.norm = N.norm_in[td];
+    q.ps = N.phi_s[min(t & 31, MHC_COLS - 1)];
     const bool site = N.site >= 0;
 #pragma unroll
     for (int rr = 0; rr < RP; ++rr) {
@@ -955,85 +993,28 @@ __device__ __forceinline__ InRegs<PC, RP> load_in(const Dims& D, const SessDev (
         q.kr[rr] = kp[td];
         q.ev[rr] = ep[td];
     }
-    if constexpr (PHI) load_phi<PC, RP, MF>(D, N, q);
     return q;
 }
 
-template <int PC, int RP, bool MF>
+// The wavefront's Phi8 fragments: k-steps h, h + HOLDERS, ... (none that the
+// rows have not: issuing a load takes the CU's address unit ~16 cycles;
+// registers of skipped steps stay unset and unread).
+template <int PC, int RP>
 __device__ __forceinline__ void load_phi(const Dims& D, const LayerDev& N, InRegs<PC, RP>& q) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nc = MHC_LANES * D.d;
-    if constexpr (MF) {
-        const int h = phi_holder(__builtin_amdgcn_readfirstlane(wave));
-        if (h >= 0) {
-            const int per = nc / 16;
-            const bool three = h + 2 * PHI_MF < MHC_COLS;
-            const int k2 = min(h + 2 * PHI_MF, MHC_COLS - 1);
-            const uint4* row0 = reinterpret_cast<const uint4*>(N.phi_q + (size_t)h * nc);
-            const uint4* row1 = reinterpret_cast<const uint4*>(N.phi_q + (size_t)(h + PHI_MF) * nc);
-            const uint4* row2 = reinterpret_cast<const uint4*>(N.phi_q + (size_t)k2 * nc);
+    const int h = Phi<RP>::holder(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, r = lane & 15, steps = MHC_LANES * D.d / 64;
+    if (h < 0) return;
+    const int8_t* p0 = N.phi_q + lane * 16;
+    const int8_t* p1 = N.phi_q + (64 + (lane >> 4) * 8 + (r & 7)) * 16;
 #pragma unroll
-            for (int j = 0; j < PC; ++j) {
-                if (64 * j < per) {
-                    const int c = min(lane + 64 * j, per - 1);
-                    q.r0[j] = row0[c];
-                    q.r1[j] = row1[c];
-                    if (three) q.r2[j] = row2[c];
-                }
-            }
-            q.ps0 = N.phi_s[h];
-            q.ps1 = N.phi_s[h + PHI_MF];
-            q.ps2 = N.phi_s[k2];
-        }
-        return;
-    }
-    // Phi8 rows: wavefront w >= 1 holds row w - 1, and row w + PHI_B - 1
-    // while that is below 24; wavefront 0, which runs the first chain of the
-    // MLP right after these loads are issued, holds none, so it never waits
-    // behind them in the CU's load queue.  Issuing them takes the CU's
-    // address unit ~16 cycles per 1 KB load, so none is issued that is not
-    // used: chunk j only while the row has one (a wavefront-uniform test;
-    // registers of skipped chunks stay unset and unread).
-    const int wu = __builtin_amdgcn_readfirstlane(wave);
-    if (wu != 0) {
-        const int per = nc / 16;  // uint4 per row
-        const int w0 = wu - 1, w1 = min(wu - 1 + PHI_B, MHC_COLS - 1);
-        const bool two = wu - 1 + PHI_B < MHC_COLS;
-        const uint4* row0 = reinterpret_cast<const uint4*>(N.phi_q + (size_t)w0 * nc);
-        const uint4* row1 = reinterpret_cast<const uint4*>(N.phi_q + (size_t)w1 * nc);
-#pragma unroll
-        for (int j = 0; j < PC; ++j) {
-            if (64 * j < per) {
-                const int c = min(lane + 64 * j, per - 1);
-                q.r0[j] = row0[c];
-                if (two) q.r1[j] = row1[c];
-            }
-        }
-        q.ps0 = N.phi_s[w0];
-        q.ps1 = N.phi_s[w1];
-    }
-}
-
-// (The device library's wavefront sum: the DPP form of wave_sum_i32
-// measured no faster in the one-row kernel and spilled 8 more bytes in the
-// 64-VGPR batched one.)
-extern "C" __device__ __attribute__((const)) int __ockl_wfred_add_i32(int);
-
-template <int PC>
-__device__ __forceinline__ int dot_row(const uint4* r, const int8_t* x8, int per, int lane) {
-    const uint4* xv = reinterpret_cast<const uint4*>(x8);
-    int acc = 0;
-#pragma unroll
-    for (int j = 0; j < PC; ++j) {
-        const int i = lane + 64 * j;
-        if (i < per) {
-            const uint4 b = xv[i];
-            acc = __builtin_amdgcn_sdot4((int)r[j].x, (int)b.x, acc, false);
-            acc = __builtin_amdgcn_sdot4((int)r[j].y, (int)b.y, acc, false);
-            acc = __builtin_amdgcn_sdot4((int)r[j].z, (int)b.z, acc, false);
-            acc = __builtin_amdgcn_sdot4((int)r[j].w, (int)b.w, acc, false);
+    for (int s = 0; s < InRegs<PC, RP>::KS; ++s) {
+        const int k = h + s * Phi<RP>::HOLDERS, k1 = k + Phi<RP>::HOLDERS;
+        if (k < steps) {
+            q.f0[s] = *reinterpret_cast<const u32x4*>(p0 + k * PHI_STEP);
+            if (s % 2 == 0)
+                q.f1[s / 2] = *reinterpret_cast<const u32x4*>(p1 + (r < 8 || k1 >= steps ? k : k1) * PHI_STEP);
         }
     }
-    return __ockl_wfred_add_i32(acc);
 }
 
 // The mHC read, engram gate, input norm and A8 of layer N
@@ -1042,12 +1023,10 @@ __device__ __forceinline__ int dot_row(const uint4* r, const int8_t* x8, int per
 // LDS behind a barrier.  live[rr]: row rr exists (else nothing of it is
 // stored).  The post and residual gates of the layer (hpost, the Sinkhorn
 // hres) are computed beside its units, off this kernel's path.
-template <bool LATE_PHI, int PC, bool MF, int RP>
-__device__ void layer_in(const Dims& D, const SessDev (&S)[RP], const LayerDev& N, InRegs<PC, RP> q, int in_bits,
+template <int PC, int RP>
+__device__ void layer_in(const Dims& D, const SessDev (&S)[RP], const LayerDev& N, const InRegs<PC, RP>& q, int in_bits,
                          LayerShared<RP>& sh, const float (&xl)[RP][MHC_LANES], const bool (&live)[RP]) {
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63, d = D.d, nc = MHC_LANES * d;
-    // (the Phi8 rows read now land while the norm chain runs)
-    if constexpr (LATE_PHI) load_phi<PC, RP, MF>(D, N, q);
     // every wavefront: r = rinv(dot16(xs)), the amax over the wavefronts'
     // maxima of |xs| (rounding is monotonic, so max_i |xs_i r| =
     // max_i |xs_i| r for r > 0), then the int8 lanes
@@ -1071,53 +1050,50 @@ __device__ void layer_in(const Dims& D, const SessDev (&S)[RP], const LayerDev& 
         }
     }
     __syncthreads();
-    // Phi8 rows: p[k] = (sx * s_k) * idot(phi_q[k], nx8)
+    // the Phi8 dots: lane (q, i) gets rows 4 q + v against row i's lanes
+    {
+        const int h = Phi<RP>::holder(__builtin_amdgcn_readfirstlane(wave)), i = lane & 15, kq = (lane >> 4) * 16;
+        if (h >= 0) {
+            const int8_t* x8 = sh.row[RP == 1 ? 0 : i & (RP - 1)].nx8 + kq;
+            v4i a0 = {0, 0, 0, 0}, a1[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
 #pragma unroll
-    for (int rr = 0; rr < RP; ++rr) {
-        LayerRow& R = sh.row[rr];
-        const float sx = R.r_sx;
-        const int per = nc / 16;
-        if constexpr (MF) {
-            const int h = phi_holder(wave);
-            if (h >= 0) {
-                const int acc = dot_row<PC>(q.r0, R.nx8, per, lane);
-                const int acc1 = dot_row<PC>(q.r1, R.nx8, per, lane);
-                if (lane == 0) {
-                    R.p[h] = (sx * q.ps0) * (float)acc;
-                    R.p[h + PHI_MF] = (sx * q.ps1) * (float)acc1;
-                }
-                if (h + 2 * PHI_MF < MHC_COLS) {
-                    const int acc2 = dot_row<PC>(q.r2, R.nx8, per, lane);
-                    if (lane == 0) R.p[h + 2 * PHI_MF] = (sx * q.ps2) * (float)acc2;
+            for (int s = 0; s < InRegs<PC, RP>::KS; ++s) {
+                const int k = h + s * Phi<RP>::HOLDERS;
+                if (k < nc / 64) {
+                    const v4i b = *reinterpret_cast<const v4i*>(x8 + k * 64);
+                    a0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i, q.f0[s]), b, a0, 0, 0, 0);
+                    a1[s & 1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i, q.f1[s / 2]), b, a1[s & 1], 0,
+                                                                      0, 0);
                 }
             }
-        } else if (wave >= 1) {
-            const int acc = dot_row<PC>(q.r0, R.nx8, per, lane);
-            if (lane == 0) R.p[wave - 1] = (sx * q.ps0) * (float)acc;
-            if (wave - 1 + PHI_B < MHC_COLS) {
-                const int acc1 = dot_row<PC>(q.r1, R.nx8, per, lane);
-                if (lane == 0) R.p[wave - 1 + PHI_B] = (sx * q.ps1) * (float)acc1;
+            if (i < RP) {
+                // (rows 16-23: fragment rows 0-7 of the first sums, 8-15 of the second)
+                int* ps = sh.row[RP == 1 ? 0 : i].psum;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    __hip_atomic_fetch_add(ps + (lane >> 4) * 4 + v, a0[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    __hip_atomic_fetch_add(ps + 16 + ((lane >> 4) & 1) * 4 + v, lane < 32 ? a1[0][v] : a1[1][v],
+                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                }
             }
         }
     }
     __syncthreads();
-    // The pre gate hp (sigmoid) in every wavefront (lane 4 rr + b: row rr,
-    // lane b), then u and x1.
+    // p[k] = (sx * s_k) * idot(phi_q[k], nx8), lane 32 rr + k: row rr's; the
+    // pre gate hp (sigmoid of its first four) in every wavefront, then u and x1.
+    const int prow = RP == 1 ? 0 : lane >> 5, pk = min(lane & 31, MHC_COLS - 1);
+    const float pv = (sh.row[prow].r_sx * q.ps) * (float)sh.row[prow].psum[pk];
     float hp[RP][MHC_LANES];
     {
-        float g = 0.0f;
-        if (lane < RP * MHC_LANES) {
-            const int b = lane & (MHC_LANES - 1);
-            const float off = b == N.lane ? 4.0f : -4.0f;
-            const float zz = ((sh.row[RP == 1 ? 0 : lane / MHC_LANES].p[b] * N.a_pre) + off) + N.b_pre[b];
-            g = 1.0f / (lexpf(-zz) + 1.0f);
-        }
+        const int b = lane & (MHC_LANES - 1);
+        const float off = b == N.lane ? 4.0f : -4.0f;
+        const float zz = ((pv * N.a_pre) + off) + N.b_pre[b];
+        const float g = 1.0f / (lexpf(-zz) + 1.0f);
 #pragma unroll
         for (int rr = 0; rr < RP; ++rr)
 #pragma unroll
-            for (int b = 0; b < MHC_LANES; ++b)
-                hp[rr][b] = __builtin_bit_cast(
-                    float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, g), rr * MHC_LANES + b));
+            for (int b2 = 0; b2 < MHC_LANES; ++b2)
+                hp[rr][b2] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, g), rr * 32 + b2));
     }
     float u[RP] = {}, x1[RP] = {};
     if (t < d) {
@@ -1181,11 +1157,9 @@ __device__ void layer_in(const Dims& D, const SessDev (&S)[RP], const LayerDev& 
             }
         }
     }
-    if (t < MHC_COLS) {
 #pragma unroll
-        for (int rr = 0; rr < RP; ++rr)
-            if (RP == 1 || live[rr]) S[rr].p[t] = sh.row[rr].p[t];
-    }
+    for (int rr = 0; rr < RP; ++rr)
+        if (t >= rr * 32 && t < rr * 32 + MHC_COLS && (RP == 1 || live[rr])) S[rr].p[t - rr * 32] = pv;
     __syncthreads();
     const int groups = (d + GROUP - 1) / GROUP;
 #pragma unroll
@@ -1259,7 +1233,7 @@ template <bool PREV, bool NEXT, int RP, int PC>
 __global__ __launch_bounds__(LT) void k_layer(
     const uint4* stage, const float* o, const float* p, float* xs, const float* x1, const float* u, int d, int row0,
     int rows, Dims D, Globals G, SessDev S, LayerDev P, LayerDev N, int in_bits, int head_bits, int head_row0) {
-    constexpr bool has_prev = PREV, has_next = NEXT, MF = RP == 1;
+    constexpr bool has_prev = PREV, has_next = NEXT;
     __shared__ LayerShared<RP> sh;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nc = MHC_LANES * d;
     const int Gd = (d + GROUP - 1) / GROUP;
@@ -1301,10 +1275,17 @@ __global__ __launch_bounds__(LT) void k_layer(
     // go now.  With one they go after the first barrier: the Phi8 rows are
     // half the kernel's bytes and are not needed before the mHC read, so
     // they stay out of the way of the tables the MLP waits for.
-    if constexpr (has_next && !has_prev) qi = load_in<MF, PC, MF, RP>(D, R, N);
+    if constexpr (has_next && !has_prev) {
+        qi = load_in<PC, RP>(D, R, N);
+        load_phi<PC, RP>(D, N, qi);
+    }
     if constexpr (!has_next) fnorm = G.final_norm[min(t, d - 1)];
     float m[RP] = {};
     if (t < RP) sh.row[t].mix_count = 0;
+    if (t < MHC_COLS) {
+#pragma unroll
+        for (int rr = 0; rr < RP; ++rr) sh.row[rr].psum[t] = 0;
+    }
     // With a previous layer the lanes' transposed copy is written by its
     // mHC write (over the MLP's buffers).
     if constexpr (!has_prev) {
@@ -1320,21 +1301,26 @@ __global__ __launch_bounds__(LT) void k_layer(
     }
     if constexpr (has_prev) store_out<RP>(d, qo, sh);
     __syncthreads();
-    if constexpr (has_next && has_prev) qi = load_in<false, PC, MF, RP>(D, R, N);
+    if constexpr (has_next && has_prev) qi = load_in<PC, RP>(D, R, N);
     // The Phi8 rows (72 KB at d = 768, ~16 cycles of the CU's address unit
-    // per 1 KB wavefront load): one row alone issues them where wavefront 0
-    // runs cond_weights, the longest chain of the MLP, and the other
-    // wavefronts wait for it anyway (issued right after the first barrier
-    // they held the post norm's barrier back); two rows, whose mixers are
-    // eight wavefronts, once the MLP is done.
+    // per 1 KB wavefront load) go out where cond_weights, the longest chain of
+    // the MLP, keeps the other wavefronts waiting anyway (issued right after
+    // the first barrier they held the post norm's barrier back).
+    const bool early = Phi<RP>::early(__builtin_amdgcn_readfirstlane(wave));
     if constexpr (has_prev)
         layer_out<RP>(
             D, S, P, qo, sh, xl, m,
             [&]() __attribute__((always_inline)) {
-                if constexpr (has_next && MF) load_phi<PC, RP, true>(D, N, qi);
+                if constexpr (has_next) {
+                    asm volatile("" : "+v"(qi.norm), "+v"(qi.ps));
+#pragma unroll
+                    for (int rr = 0; rr < RP; ++rr) asm volatile("" : "+v"(qi.kr[rr]), "+v"(qi.ev[rr]));
+                    if (early) load_phi<PC, RP>(D, N, qi);
+                }
             },
             [&]() __attribute__((always_inline)) {
-                if constexpr (has_next && !MF) load_phi<PC, RP, false>(D, N, qi);
+                if constexpr (has_next)
+                    if (!early) load_phi<PC, RP>(D, N, qi);
             });
     // the wavefronts' maxima of |xs| for the mHC read
 #pragma unroll
@@ -1347,7 +1333,7 @@ __global__ __launch_bounds__(LT) void k_layer(
     // stores issued earlier would sit in the memory counter ahead of loads
     // that are waited for)
     if constexpr (has_next) {
-        layer_in<!MF && !has_prev, PC, MF, RP>(D, R, N, qi, in_bits, sh, xl, live);
+        layer_in<PC, RP>(D, R, N, qi, in_bits, sh, xl, live);
     } else {
         // rows i >= head_row0 into activation row i - head_row0 (block-uniform)
         int arow[RP];
@@ -3484,7 +3470,7 @@ __global__ __launch_bounds__(256) void k_phi8(const float* __restrict__ rows, in
     m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     const float s = m > 0.0f ? m * bits_f32(0x3c010204u) : 1.0f;
     const float inv = 1.0f / s;
-    for (int i = t; i < width; i += 256) q[(size_t)r * width + i] = quant_one(x[i], inv);
+    for (int i = t; i < width; i += 256) q[phi_at(r, i)] = quant_one(x[i], inv);
     if (t == 0) scale[r] = s;
 }
 
