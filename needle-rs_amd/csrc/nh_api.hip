@@ -254,6 +254,37 @@ static void relayout2(const uint8_t* packed, int out, int out_pad, int groups, s
         }
 }
 
+// A 4-bit matrix's handle and device buffers (the selectors' f32 codebook
+// filled in, codes, int8 copy and norms not).
+static int new_qmat4(int out, int in_dim, nh_qmat** h) {
+    const int groups = (in_dim + GROUP - 1) / GROUP, alloc = (out + PANEL_ROWS - 1) / PANEL_ROWS * PANEL_ROWS;
+    nh_qmat* q = new nh_qmat();
+    QMatMeta& m = q->m;
+    m.out = out;
+    m.out_pad = (out + TILE_ROWS - 1) / TILE_ROWS * TILE_ROWS;
+    m.in_dim = in_dim;
+    m.groups = groups;
+    m.bits = 4;
+    m.ternary = false;
+    m.cbs = g_cbs4;
+    memcpy(m.vals, g_cb8, 16);
+    memcpy(m.fvals, g_cb4, sizeof g_cb4);
+    m.lut = g_lut4;
+    float fsel[16];
+    for (int s = 0; s < 16; ++s) fsel[s] = m.fvals[m.lut.code_of_sel[s]];
+    hipError_t e = hipMalloc(&q->d_codes, (size_t)alloc * groups * 64);
+    if (e == hipSuccess) e = hipMalloc(&q->d_w8, (size_t)alloc * groups * 128);
+    if (e == hipSuccess) e = hipMalloc(&q->d_norms, (size_t)alloc * groups * 2);
+    if (e == hipSuccess) e = hipMalloc(&q->d_fsel, 64);
+    if (e == hipSuccess) e = hipMemcpy(q->d_fsel, fsel, 64, hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        nh_qmat_free(q);
+        return fail(NH_ENOMEM, std::string("matrix allocation: ") + hipGetErrorString(e));
+    }
+    *h = q;
+    return NH_OK;
+}
+
 // QMat::build (qlinear.rs:244-265) for the code width `bits` (2 or 4), with
 // from_cq's ternary remap (qlinear.rs:222-227): code 3 is the first level,
 // codes 0..2 the rest; codes without a level are 0.
@@ -446,28 +477,41 @@ int nh_qmat_from_f32(const float* w, int out, int in_dim, nh_qmat** h) {
     if (out <= 0 || in_dim <= 0) return fail(NH_EINVAL, "empty matrix");
     const int groups = (in_dim + GROUP - 1) / GROUP;
     if (groups > 32) return fail(NH_EINVAL, "in_dim above 4096 is not supported");
-    float* dw = nullptr;
-    float* dcb = nullptr;
-    uint8_t* dp = nullptr;
-    uint16_t* dn = nullptr;
+    // One temporary block: the weights, the codebook, the packed codes and the
+    // norms, stream-ordered.  The codes are tiled on the device, so they cross
+    // to the host once, for the matrix's archive-layout copy.
     const size_t nw = (size_t)out * in_dim, np = (size_t)out * groups * 64, nn = (size_t)out * groups;
-    hipError_t e = hipMalloc(&dw, nw * 4);
-    if (e == hipSuccess) e = hipMalloc(&dcb, 64);
-    if (e == hipSuccess) e = hipMalloc(&dp, np);
-    if (e == hipSuccess) e = hipMalloc(&dn, nn * 2);
-    std::vector<uint8_t> packed(np);
-    std::vector<uint16_t> norms(nn);
-    if (e == hipSuccess) e = hipMemcpy(dw, w, nw * 4, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(dcb, g_cb4, 64, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = launch_cq_pack(dw, out, in_dim, groups, dcb, dp, dn, nullptr);
-    if (e == hipSuccess) e = hipMemcpy(packed.data(), dp, np, hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = hipMemcpy(norms.data(), dn, nn * 2, hipMemcpyDeviceToHost);
-    hipFree(dw);
-    hipFree(dcb);
-    hipFree(dp);
-    hipFree(dn);
-    if (e != hipSuccess) return hip_fail(e, "cq_pack");
-    return upload(std::move(packed), std::move(norms), out, in_dim, 4, false, h);
+    const auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+    uint8_t* buf = nullptr;
+    hipError_t e = hipMallocAsync((void**)&buf, up(nw * 4) + 256 + up(np) + up(nn * 2), nullptr);
+    if (e != hipSuccess) return fail(NH_ENOMEM, std::string("hipMallocAsync: ") + hipGetErrorString(e));
+    float* dw = (float*)buf;
+    float* dcb = (float*)(buf + up(nw * 4));
+    uint8_t* dp = buf + up(nw * 4) + 256;
+    uint16_t* dn = (uint16_t*)(dp + up(np));
+    nh_qmat* q = nullptr;
+    int rc = new_qmat4(out, in_dim, &q);
+    if (rc == NH_OK) {
+        e = hipMemcpy(dw, w, nw * 4, hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = hipMemcpy(dcb, g_cb4, 64, hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = launch_cq_pack(dw, out, in_dim, groups, dcb, dp, dn, nullptr);
+        const int alloc = (out + PANEL_ROWS - 1) / PANEL_ROWS * PANEL_ROWS;
+        if (e == hipSuccess) e = launch_tile4(dp, dn, out, alloc, groups, q->m.lut, q->d_codes, q->d_norms, nullptr);
+        if (e == hipSuccess) e = launch_expand_w8(q, nullptr);
+        q->h_packed.resize(np);
+        q->h_norms.resize(nn);
+        if (e == hipSuccess) e = hipMemcpy(q->h_packed.data(), dp, np, hipMemcpyDeviceToHost);
+        if (e == hipSuccess) e = hipMemcpy(q->h_norms.data(), dn, nn * 2, hipMemcpyDeviceToHost);
+        if (e == hipSuccess) e = hipDeviceSynchronize();
+        if (e != hipSuccess) {
+            nh_qmat_free(q);
+            rc = hip_fail(e, "cq_pack");
+        }
+    }
+    hipFreeAsync(buf, nullptr);
+    if (rc != NH_OK) return rc;
+    *h = q;
+    return NH_OK;
 }
 
 int nh_qlinear_new(nh_qmat* const* parts, int n, nh_qmat** h) {

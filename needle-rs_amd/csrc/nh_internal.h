@@ -167,6 +167,10 @@ hipError_t launch_single_rows(const nh_qmat* w, const nh_qact* a, const uint32_t
                               float* scatter_logits, int scatter_n, hipStream_t s);
 hipError_t launch_fill(float* p, float v, int n, hipStream_t s);
 hipError_t launch_rows(const nh_qmat* w, const uint32_t* ids, int n, float* out, hipStream_t s);
+// Archive-layout 4-bit codes and norms on the device into a matrix's tiled
+// codes and padded norms (`alloc` rows).
+hipError_t launch_tile4(const uint8_t* packed, const uint16_t* norms, int out, int alloc, int G, const LutTables& lut,
+                        uint4* tiled, uint16_t* dnorms, hipStream_t s);
 hipError_t launch_cq_pack(const float* w, int rows, int d, int groups, const float* cb, uint8_t* packed,
                           uint16_t* norms, hipStream_t s);
 
