@@ -812,9 +812,9 @@ __device__ __forceinline__ void cond_weights(const float* hT, const float* cvT, 
 // thread's element of the rows' 4 lanes (t < d) and gets the new ones; m gets
 // this thread's max |new lane value| of each row (for the next layer's mHC
 // read).
-template <int RP, typename BeforeMix, typename Late>
+template <int RP, typename BeforeMix>
 __device__ void layer_out(const Dims& D, const SessDev& S, const LayerDev& P, OutRegs<RP>& q, LayerShared<RP>& sh,
-                          float (&xl)[RP][MHC_LANES], float (&m)[RP], BeforeMix before_mix, Late late) {
+                          float (&xl)[RP][MHC_LANES], float (&m)[RP], BeforeMix before_mix) {
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63, d = D.d;
     // mix8 runs on waves 4..7 (threads 256..511; row 1: 8..11), beside
     // cond_weights on wave 0 (row 1: wave 1)
@@ -897,7 +897,6 @@ __device__ void layer_out(const Dims& D, const SessDev& S, const LayerDev& P, Ou
     __syncthreads();
     if (mixer) mix8_n(mu, M.B, sh.kf[5], M.C, d / HADA_NB / 8 * 8);
     __syncthreads();
-    if constexpr (RP > 1) late();
     // The mHC write: y = (x2 + t3 * d4) - u; lane a = y hpost[a] + sum_b
     // hres[a][b] old[b] as an fma chain over b.
 #pragma unroll
@@ -957,14 +956,6 @@ struct Phi {
     static __device__ __forceinline__ int holder(int wave) {
         if constexpr (RP == 1) return wave < 4 ? wave : wave >= 8 ? wave - 4 : -1;
         return wave;
-    }
-    // issues its rows beside cond_weights, on the chain's wavefronts too
-    // (issuing wavefront 0's after its chain cost the one-row kernel 2 %: the
-    // MLP's later reads wait behind them); with two rows the mixers and
-    // the chains' wavefronts issue theirs after the MLP
-    static __device__ __forceinline__ bool early(int wave) {
-        if constexpr (RP == 1) return true;
-        return wave == 2 || wave == 3 || wave >= 12;
     }
 };
 template <int PC, int RP>
@@ -1305,23 +1296,18 @@ __global__ __launch_bounds__(LT) void k_layer(
     // The Phi8 rows (72 KB at d = 768, ~16 cycles of the CU's address unit
     // per 1 KB wavefront load) go out where cond_weights, the longest chain of
     // the MLP, keeps the other wavefronts waiting anyway (issued right after
-    // the first barrier they held the post norm's barrier back).
-    const bool early = Phi<RP>::early(__builtin_amdgcn_readfirstlane(wave));
+    // the first barrier they held the post norm's barrier back; after the MLP,
+    // or wavefront 0's after its chain, they hold the mHC read or later
+    // reads back: 2 % of a prefill, 2 % of a decode step).
     if constexpr (has_prev)
-        layer_out<RP>(
-            D, S, P, qo, sh, xl, m,
-            [&]() __attribute__((always_inline)) {
-                if constexpr (has_next) {
-                    asm volatile("" : "+v"(qi.norm), "+v"(qi.ps));
+        layer_out<RP>(D, S, P, qo, sh, xl, m, [&]() __attribute__((always_inline)) {
+            if constexpr (has_next) {
+                asm volatile("" : "+v"(qi.norm), "+v"(qi.ps));
 #pragma unroll
-                    for (int rr = 0; rr < RP; ++rr) asm volatile("" : "+v"(qi.kr[rr]), "+v"(qi.ev[rr]));
-                    if (early) load_phi<PC, RP>(D, N, qi);
-                }
-            },
-            [&]() __attribute__((always_inline)) {
-                if constexpr (has_next)
-                    if (!early) load_phi<PC, RP>(D, N, qi);
-            });
+                for (int rr = 0; rr < RP; ++rr) asm volatile("" : "+v"(qi.kr[rr]), "+v"(qi.ev[rr]));
+                load_phi<PC, RP>(D, N, qi);
+            }
+        });
     // the wavefronts' maxima of |xs| for the mHC read
 #pragma unroll
     for (int rr = 0; rr < RP; ++rr) {
