@@ -261,7 +261,7 @@ __global__ __launch_bounds__(256) void k_begin(Dims D, Globals G, SessDev S, Beg
                         row_group<4>(tb.codes, tb.norms, tb.fsel, tb.groups, row, 0, lane, v0, v1);
                 }
             }
-            const size_t unit = ((size_t)e * ACT_ROWS + i) * Gd + g;
+            const size_t unit = ((size_t)e * D.batch + i) * Gd + g;
             a8_group(v0, v1, lane, B.eng_bits[e], S.xq_eng + unit * GROUP, S.sx_eng + unit);
         }
     } else if (wave < t * per_row + t) {
@@ -322,7 +322,7 @@ __global__ __launch_bounds__(1024) void k_engram_hist(Dims D, Globals G, SessDev
     const int e = blockIdx.x, i = blockIdx.y, k = threadIdx.x, d = D.d, pos = p0 + i;
     const bool on = k < d;
     const int kc = on ? k : 0;
-    const float* kv = S.ekv + (size_t)e * BATCH_ROWS * 2 * d;
+    const float* kv = S.ekv + (size_t)e * D.batch * 2 * d;
     const int gs = d / 32;
     int8_t* ev8 = S.ev8 + (size_t)e * D.cap * d;
     float* evs = S.evs + (size_t)e * D.cap * gs;
@@ -365,7 +365,7 @@ __global__ __launch_bounds__(1024) void k_engram_hist(Dims D, Globals G, SessDev
         const float tw = on ? twj[j] : 0.0f;
         dst = __builtin_fmaf(tw, qs * (float)q8, dst);
     }
-    if (on) S.evals[((size_t)e * BATCH_ROWS + i) * d + k] = dst;
+    if (on) S.evals[((size_t)e * D.batch + i) * d + k] = dst;
 }
 
 hipError_t fwd_engram_hist(const Dims& D, const Globals& G, const SessDev& S, int p0, int t, hipStream_t s) {
@@ -979,8 +979,8 @@ __device__ __forceinline__ InRegs<PC, RP> load_in(const Dims& D, const SessDev (
     const bool site = N.site >= 0;
 #pragma unroll
     for (int rr = 0; rr < RP; ++rr) {
-        const float* kp = site ? S[rr].ekv + (size_t)N.site * BATCH_ROWS * 2 * d : S[rr].proj;
-        const float* ep = site ? S[rr].evals + (size_t)N.site * BATCH_ROWS * d : S[rr].proj + d;
+        const float* kp = site ? S[rr].ekv + (size_t)N.site * D.batch * 2 * d : S[rr].proj;
+        const float* ep = site ? S[rr].evals + (size_t)N.site * D.batch * d : S[rr].proj + d;
         q.kr[rr] = kp[td];
         q.ev[rr] = ep[td];
     }

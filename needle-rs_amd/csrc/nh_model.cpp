@@ -127,7 +127,7 @@ struct nh_model {
 struct nh_session {
     const nh_model* m = nullptr;
     nh::Dims dims{};
-    nh::SessDev S{};
+    nh::SessDev S{};  // (with the row buffers of `many`)
     void* d_buf = nullptr;
     size_t bytes = 0;
     int len = 0;
@@ -142,8 +142,17 @@ struct nh_session {
     int sink = 0, ring = 0;
     std::vector<int64_t> slot_pos;
     std::vector<uint32_t> toks;
-    nh_qact a_in{}, a_att{};
-    std::vector<nh_qact> a_eng;
+    // The row buffers of a feed of `rows` rows, and the A8 views of them.
+    struct Rows {
+        nh::SessDev S{};
+        nh_qact a_in{}, a_att{};
+        std::vector<nh_qact> a_eng;
+        int rows = 0;
+    };
+    // A step's are a set of their own, one row each, side by side: row 0 of
+    // buffers of Dims::batch rows would be a page each (eight steps at 2,900
+    // keys, 2048 rows: 4.50 ms so, 4.47 with the set).
+    Rows step, many;
     // The status word as the stream last copied it (pinned), behind
     // ev_status; pending while that copy has not been read.
     int32_t* h_status = nullptr;
@@ -565,7 +574,7 @@ int out_width(const nh_session* s, int outputs) {
 
 // One feed at positions s->len ..: step_native for one token, chunk_job for
 // a chunk of up to 32 (forward_native, infer.rs:1105-1132), or several whole
-// chunks of at least two tokens each (t <= BATCH_ROWS) as one pass through
+// chunks of at least two tokens each (t <= Dims::batch) as one pass through
 // the layers with each row keeping its chunk's arithmetic (chunk c = rows
 // 32c ..: its rows' block flags, nested key chunks and sincosf RoPE rows;
 // the causal keys of a row do not depend on how the prompt was cut).
@@ -580,11 +589,13 @@ int out_width(const nh_session* s, int outputs) {
 int feed(nh_session* s, int t, int outputs, float* out, float* cells, hipStream_t st, bool pick = false,
          bool staged = false) {
     const nh_model* m = s->m;
-    nh::SessDev S = s->S;
+    nh_session::Rows& B = t == 1 ? s->step : s->many;
+    nh::SessDev S = B.S;
     S.cells = cells;
     const int p0 = s->len;
     const uint8_t* flags = t > nh::FWD_ROWS ? S.flags : nullptr;
     nh::Dims D = s->dims;
+    D.batch = B.rows;
     D.hist_lo = p0 - s->hrows;
     D.rope_prev = t == 1 && s->rope_n > 0;
     D.sink = s->sink;
@@ -606,9 +617,9 @@ int feed(nh_session* s, int t, int outputs, float* out, float* cells, hipStream_
         const nh_qact* acts[nh::GEMV_BATCH_MAX];
         float* ys[nh::GEMV_BATCH_MAX];
         for (int e = 0; e < D.sites; ++e) {
-            s->a_eng[e].rows = 1;
-            acts[e] = &s->a_eng[e];
-            ys[e] = S.ekv + (size_t)e * nh::BATCH_ROWS * 2 * D.d;
+            B.a_eng[e].rows = 1;
+            acts[e] = &B.a_eng[e];
+            ys[e] = S.ekv + (size_t)e * D.batch * 2 * D.d;
         }
         NH_TRY(nh::launch_gemv_batch(m->ekv.data(), acts, ys, D.sites, st), "engram kv");
     } else {
@@ -617,22 +628,22 @@ int feed(nh_session* s, int t, int outputs, float* out, float* cells, hipStream_
         const nh_qact* acts[nh::MAX_SITES];
         float* ys[nh::MAX_SITES];
         for (int e = 0; e < D.sites; ++e) {
-            s->a_eng[e].rows = t;
-            acts[e] = &s->a_eng[e];
-            ys[e] = S.ekv + (size_t)e * nh::BATCH_ROWS * 2 * D.d;
+            B.a_eng[e].rows = t;
+            acts[e] = &B.a_eng[e];
+            ys[e] = S.ekv + (size_t)e * D.batch * 2 * D.d;
         }
         if (t > 1 && D.sites > 1 && nh::gemm_batchable(m->ekv.data(), acts, D.sites)) {
             NH_TRY(nh::launch_gemm_batch(m->ekv.data(), acts, ys, D.sites, flags, 2 * D.d, st), "engram kv");
         } else {
             for (int e = 0; e < D.sites; ++e)
-                NH_TRY(product(m->ekv[e], &s->a_eng[e], t, ys[e], 2 * D.d, flags, st), "engram kv");
+                NH_TRY(product(m->ekv[e], &B.a_eng[e], t, ys[e], 2 * D.d, flags, st), "engram kv");
         }
     }
     NH_TRY(nh::fwd_engram_hist(D, m->glob, S, p0, t, st), "engram history");
     for (int l = 0; l < D.layers; ++l) {
         const nh::LayerDev* prev = l > 0 ? &m->layers[l - 1] : nullptr;
         NH_TRY(nh::fwd_layer(D, m->glob, S, prev, &m->layers[l], 0, t, m->qkvg[l]->m.bits, 0, st), "layer");
-        NH_TRY(product(m->qkvg[l], &s->a_in, t, S.proj, D.nq, flags, st), "q|k|v|gate");
+        NH_TRY(product(m->qkvg[l], &B.a_in, t, S.proj, D.nq, flags, st), "q|k|v|gate");
         if (t == 1 && nh::dec_group_fits(D, p0, m->layers[l].window)) {
             NH_TRY(nh::fwd_dec_attn(D, S, m->layers[l], l, p0, m->out[l]->m.bits, st), "decode attention");
         } else if (t == 1 && nh::dec_chunks_fits(D)) {
@@ -642,7 +653,7 @@ int feed(nh_session* s, int t, int outputs, float* out, float* cells, hipStream_
             NH_TRY(nh::fwd_attend(D, S, m->layers[l], l, p0, t, sp, st), "attend");
             NH_TRY(nh::fwd_attn_out(D, S, m->layers[l], l, p0, t, m->out[l]->m.bits, sp, st), "attention out");
         }
-        NH_TRY(product(m->out[l], &s->a_att, t, S.o, D.d, flags, st), "out");
+        NH_TRY(product(m->out[l], &B.a_att, t, S.o, D.d, flags, st), "out");
     }
     // the last layer's post block, the lane mean and final norm of the rows
     // the outputs want, then the head (head_logits per row, decode combine)
@@ -662,7 +673,7 @@ int feed(nh_session* s, int t, int outputs, float* out, float* cells, hipStream_
             // every row's logits in one launch when they are asked for, else
             // the last row's (head_logits: the decode combine either way)
             const bool all = rows > 1 && out;
-            nh_qact a = s->a_in;
+            nh_qact a = B.a_in;
             if (!all) {
                 a.d_xq += (size_t)(rows - 1) * Gd * nh::GROUP;
                 a.d_sx += (size_t)(rows - 1) * Gd;
@@ -790,7 +801,7 @@ int forward_ids(nh_session* s, const uint32_t* toks, int n, int outputs, float* 
         int t = std::min(nh::FWD_ROWS, n - i);
         const bool staged = s->ring > 0 && span_staged(s, t);
         if ((s->ring == 0 || staged) && t > 1)
-            while (t < nh::BATCH_ROWS && i + t < n && n - (i + t) > 1) t += std::min(nh::FWD_ROWS, n - (i + t));
+            while (t < s->dims.batch && i + t < n && n - (i + t) > 1) t += std::min(nh::FWD_ROWS, n - (i + t));
         const bool last = i + t == n;
         const int want =
             (!last && (outputs == NH_OUT_LAST_LOGITS || outputs == NH_OUT_LAST_HIDDEN)) ? NH_OUT_NONE : outputs;
@@ -889,33 +900,42 @@ int nh_session_new(const nh_model* m, int cap, nh_session** out) {
     D = m->dims;
     D.cap = cap;
     D.stage0 = (int)round_up((size_t)cap, 16);
-    D.kslots = D.stage0 + nh::BATCH_ROWS;
+    D.batch = std::min(nh::BATCH_MAX, (int)round_up((size_t)cap, nh::BATCH_MIN));
+    D.kslots = D.stage0 + D.batch;
     D.vcap = (int)round_up((size_t)D.kslots + 4, 16);
     int mc = 1;
     for (int n = 1; n <= cap; ++n) mc = std::max(mc, key_chunk_count(n, D.nkv));
     D.max_chunks = mc;
-    const size_t d = D.d, L = D.layers, c = cap, E = D.sites, R = nh::BATCH_ROWS, AR = nh::ACT_ROWS;
+    const size_t d = D.d, L = D.layers, c = cap, E = D.sites;
     const size_t half = D.qk / 2;
     const int Gd = (D.d + nh::GROUP - 1) / nh::GROUP, Ga = (D.nh * D.vd + nh::GROUP - 1) / nh::GROUP;
     Layout Y;
-    const size_t o_xs = Y.take(R * 4 * d * 4), o_u = Y.take(R * d * 4), o_x1 = Y.take(R * d * 4);
-    const size_t o_p = Y.take(R * 64 * 4), o_proj = Y.take(R * D.nq * 4), o_q = Y.take(R * D.nh * D.qk * 4);
-    const size_t o_o = Y.take(R * d * 4), o_ekv = Y.take(E * R * 2 * d * 4), o_ev = Y.take(E * R * d * 4);
+    // the row buffers (offsets for now) of R rows
+    auto take_rows = [&](nh_session::Rows& B, size_t R) {
+        nh::SessDev& S = B.S;
+        auto f = [&](float*& p, size_t n) { p = (float*)Y.take(n * 4); };
+        auto q = [&](int8_t*& p, size_t n) { p = (int8_t*)Y.take(n); };
+        f(S.xs, R * 4 * d), f(S.u, R * d), f(S.x1, R * d), f(S.p, R * 64), f(S.proj, R * D.nq);
+        f(S.qbuf, R * D.nh * D.qk), f(S.o, R * d), f(S.ekv, E * R * 2 * d), f(S.evals, E * R * d);
+        f(S.rope_c, R * half), f(S.rope_s, R * half), f(S.hid, R * d);
+        f(S.po, R * D.nh * mc * D.vd), f(S.pm, R * D.nh * mc), f(S.psum, R * D.nh * mc);
+        q(S.xq_in, R * Gd * nh::GROUP), f(S.sx_in, R * Gd);
+        q(S.xq_att, R * Ga * nh::GROUP), f(S.sx_att, R * Ga);
+        q(S.xq_eng, E * R * Gd * nh::GROUP), f(S.sx_eng, E * R * Gd);
+        S.flags = (uint8_t*)Y.take(R);
+        B.rows = (int)R;
+    };
+    take_rows(s->step, 1);
     const size_t o_lg = Y.take(round_up(D.out_rows, nh::PANEL_ROWS) * 4);
-    const size_t o_rc = Y.take(R * half * 4), o_rs = Y.take(R * half * 4);
     const size_t o_rrc = Y.take(nh::ROPE_RING * half * 4), o_rrs = Y.take(nh::ROPE_RING * half * 4);
-    const size_t o_hid = Y.take(R * d * 4), o_lh = Y.take(d * 4), o_tok = Y.take(c * 4);
-    const size_t o_po = Y.take(R * D.nh * mc * D.vd * 4), o_pm = Y.take(R * D.nh * mc * 4),
-                 o_ps = Y.take(R * D.nh * mc * 4);
+    const size_t o_lh = Y.take(d * 4), o_am = Y.take(16), o_st = Y.take(16), o_dc = Y.take(nh::DCOUNT_SLOTS * 4);
+    const size_t o_tok = Y.take(c * 4);
     const size_t o_hist = Y.take(L * D.hist_slots * D.W * 4);
     const size_t ksl = D.kslots;
     const size_t o_k8 = Y.take(L * ksl * D.nkv * D.qk), o_ks = Y.take(L * ksl * D.nkv * 4);
     const size_t o_v8 = Y.take(L * D.nkv * D.vd * D.vcap), o_vs = Y.take(L * ksl * D.nkv * 4);
     const size_t o_e8 = Y.take(E * c * d), o_es = Y.take(E * c * (d / 32) * 4);
-    const size_t o_xi = Y.take(AR * Gd * nh::GROUP), o_si = Y.take(AR * Gd * 4);
-    const size_t o_xa = Y.take(AR * Ga * nh::GROUP), o_sa = Y.take(AR * Ga * 4);
-    const size_t o_xe = Y.take(E * AR * Gd * nh::GROUP), o_se = Y.take(E * AR * Gd * 4);
-    const size_t o_am = Y.take(16), o_st = Y.take(16), o_fl = Y.take(R), o_dc = Y.take(nh::DCOUNT_SLOTS * 4);
+    take_rows(s->many, D.batch);
     hipError_t e = hipMalloc(&s->d_buf, Y.size);
     if (e == hipSuccess) e = hipMemset(s->d_buf, 0, Y.size);
     if (e == hipSuccess) e = hipHostMalloc((void**)&s->h_status, sizeof(int32_t), hipHostMallocDefault);
@@ -927,38 +947,44 @@ int nh_session_new(const nh_model* m, int cap, nh_session** out) {
     }
     s->bytes = Y.size;
     uint8_t* b = (uint8_t*)s->d_buf;
-    nh::SessDev& S = s->S;
-    S.xs = (float*)(b + o_xs), S.u = (float*)(b + o_u), S.x1 = (float*)(b + o_x1), S.p = (float*)(b + o_p);
-    S.proj = (float*)(b + o_proj), S.qbuf = (float*)(b + o_q), S.o = (float*)(b + o_o);
-    S.ekv = (float*)(b + o_ekv), S.evals = (float*)(b + o_ev), S.logits = (float*)(b + o_lg);
-    S.rope_c = (float*)(b + o_rc), S.rope_s = (float*)(b + o_rs), S.tokens = (uint32_t*)(b + o_tok);
-    S.rope_rc = (float*)(b + o_rrc), S.rope_rs = (float*)(b + o_rrs);
-    S.hid = (float*)(b + o_hid), S.last_hid = (float*)(b + o_lh);
-    S.po = (float*)(b + o_po), S.pm = (float*)(b + o_pm), S.psum = (float*)(b + o_ps);
-    S.hist = (float*)(b + o_hist), S.k8 = (int8_t*)(b + o_k8), S.ks = (float*)(b + o_ks);
-    S.v8t = (int8_t*)(b + o_v8), S.vs = (float*)(b + o_vs), S.ev8 = (int8_t*)(b + o_e8), S.evs = (float*)(b + o_es);
-    S.xq_in = (int8_t*)(b + o_xi), S.sx_in = (float*)(b + o_si);
-    S.xq_att = (int8_t*)(b + o_xa), S.sx_att = (float*)(b + o_sa);
-    S.xq_eng = (int8_t*)(b + o_xe), S.sx_eng = (float*)(b + o_se);
-    S.argmax = (int32_t*)(b + o_am);
-    S.status = (int32_t*)(b + o_st);
-    S.flags = (uint8_t*)(b + o_fl);
-    S.dcount = (int32_t*)(b + o_dc);
+    nh::SessDev G{};  // what both sets share
+    G.logits = (float*)(b + o_lg), G.tokens = (uint32_t*)(b + o_tok);
+    G.rope_rc = (float*)(b + o_rrc), G.rope_rs = (float*)(b + o_rrs), G.last_hid = (float*)(b + o_lh);
+    G.hist = (float*)(b + o_hist), G.k8 = (int8_t*)(b + o_k8), G.ks = (float*)(b + o_ks);
+    G.v8t = (int8_t*)(b + o_v8), G.vs = (float*)(b + o_vs), G.ev8 = (int8_t*)(b + o_e8), G.evs = (float*)(b + o_es);
+    G.argmax = (int32_t*)(b + o_am), G.status = (int32_t*)(b + o_st), G.dcount = (int32_t*)(b + o_dc);
     D.spin_limit = nh::SPIN_LIMIT;
-    auto view = [](int8_t* xq, float* sx, int in_dim, int groups) {
-        nh_qact a{};
-        a.cap_rows = nh::ACT_ROWS;
-        a.rows = 1;
-        a.in_dim = in_dim;
-        a.groups = groups;
-        a.d_xq = xq;
-        a.d_sx = sx;
-        return a;
+    auto place = [&](nh_session::Rows& B) {
+        const nh::SessDev O = B.S;
+        nh::SessDev& S = B.S;
+        S = G;
+        auto f = [&](float*& p, const float* o) { p = (float*)(b + (size_t)o); };
+        auto q = [&](int8_t*& p, const int8_t* o) { p = (int8_t*)(b + (size_t)o); };
+        f(S.xs, O.xs), f(S.u, O.u), f(S.x1, O.x1), f(S.p, O.p), f(S.proj, O.proj), f(S.qbuf, O.qbuf), f(S.o, O.o);
+        f(S.ekv, O.ekv), f(S.evals, O.evals), f(S.rope_c, O.rope_c), f(S.rope_s, O.rope_s), f(S.hid, O.hid);
+        f(S.po, O.po), f(S.pm, O.pm), f(S.psum, O.psum);
+        q(S.xq_in, O.xq_in), f(S.sx_in, O.sx_in), q(S.xq_att, O.xq_att), f(S.sx_att, O.sx_att);
+        q(S.xq_eng, O.xq_eng), f(S.sx_eng, O.sx_eng);
+        S.flags = b + (size_t)O.flags;
+        auto view = [&](int8_t* xq, float* sx, int in_dim, int groups) {
+            nh_qact a{};
+            a.cap_rows = B.rows;
+            a.rows = 1;
+            a.in_dim = in_dim;
+            a.groups = groups;
+            a.d_xq = xq;
+            a.d_sx = sx;
+            return a;
+        };
+        B.a_in = view(S.xq_in, S.sx_in, D.d, Gd);
+        B.a_att = view(S.xq_att, S.sx_att, D.nh * D.vd, Ga);
+        for (int i = 0; i < D.sites; ++i)
+            B.a_eng.push_back(view(S.xq_eng + (size_t)i * B.rows * Gd * nh::GROUP, S.sx_eng + (size_t)i * B.rows * Gd,
+                                   D.d, Gd));
     };
-    s->a_in = view(S.xq_in, S.sx_in, D.d, Gd);
-    s->a_att = view(S.xq_att, S.sx_att, D.nh * D.vd, Ga);
-    for (int i = 0; i < D.sites; ++i)
-        s->a_eng.push_back(view(S.xq_eng + (size_t)i * AR * Gd * nh::GROUP, S.sx_eng + (size_t)i * AR * Gd, D.d, Gd));
+    place(s->step);
+    place(s->many);
+    s->S = s->many.S;
     *out = s;
     return NH_OK;
 }
@@ -1127,7 +1153,7 @@ int nh_session_head_logits(nh_session* s, float* logits, void* stream) {
     if (!s->have_hidden) return fail(NH_EINVAL, "no hidden state yet (no feed has returned outputs)");
     hipStream_t st = (hipStream_t)stream;
     const nh::Dims& D = s->dims;
-    nh_qact a = s->a_in;
+    nh_qact a = s->step.a_in;
     a.bits = s->m->head_bits;
     NH_TRY(nh::launch_act_prep(s->S.last_hid, 1, D.d, a.groups, s->m->head_bits, nullptr, a.d_xq, a.d_sx, st),
            "head A8");
@@ -1141,7 +1167,7 @@ int nh_session_head_logits_sparse(nh_session* s, const uint32_t* ids, int n, flo
     if (!s->have_hidden) return fail(NH_EINVAL, "no hidden state yet (no feed has returned outputs)");
     hipStream_t st = (hipStream_t)stream;
     const nh::Dims& D = s->dims;
-    nh_qact a = s->a_in;
+    nh_qact a = s->step.a_in;
     a.rows = 1;
     a.bits = s->m->head_bits;
     NH_TRY(nh::launch_act_prep(s->S.last_hid, 1, D.d, a.groups, s->m->head_bits, nullptr, a.d_xq, a.d_sx, st),
