@@ -545,7 +545,8 @@ __device__ __forceinline__ void put_t(float* T, int pitch, int i, float v) { T[(
 // scheduling barriers keep the compiler from sinking the reads back to
 // their use (which would leave every batch waiting a full LDS round trip).
 // Reads past the last batch are clamped to it (read and ignored).  A chain
-// step costs ~13 cycles (the dependent fma's latency) at any depth from 3
+// step costs ~9 cycles with one operand (the dependent fma's latency is 7.5),
+// ~16 with two (cond_weights), at any depth from 3
 // up, so 3 is used.  Requires nb >= 1.
 template <int DEPTH, typename Buf, typename Load, typename Chain>
 __device__ __forceinline__ void chain_pipe(int nb, Load load, Chain chain) {

@@ -27,6 +27,7 @@
 // (L / 16), both cut from the same 16-byte block of the group's activation
 // order, so each MFMA sums exactly its 64 products whatever order the
 // instruction visits k in.
+#include <algorithm>
 #include <type_traits>
 
 #include "nh_device.h"
@@ -483,6 +484,84 @@ static hipError_t run_gc(bool general, const GemmSet& g, const uint8_t* block, i
                    : run<BM, NW, 1, false, W4>(g, block, ldy, col0, dbg, s);
 }
 
+// ------------------------------------------------- small products
+// The same combine where 16 x 16 tiles are few: k_gemm walks a tile's K in
+// steps, each a trip to memory and a barrier, on workgroups that leave most
+// of the chip idle.  Here a workgroup owns one tile and its wavefronts split the
+// groups (GPS each), every load issued at once: a launch costs one memory
+// round trip.  A group's exact sums and their scales go to LDS, and the
+// group-ordered fma chains run from there, a thread an output (as k_gemv).
+constexpr int SPLIT_WAVES = 8;
+
+template <int GPS>
+__global__ __launch_bounds__(64 * SPLIT_WAVES) void k_gemm_split(
+    const uint4* __restrict__ w8, const uint16_t* __restrict__ norms, const uint4* __restrict__ xq,
+    const float* __restrict__ sx, float* __restrict__ y, const uint8_t* __restrict__ block, int blocked, int ldy,
+    int col0, int out, int M, int G, float cbs) {
+    extern __shared__ float part[];  // [G][2][16 tokens][16 rows]: sums, scales
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, q = lane >> 4, tile = blockIdx.x, m0 = (int)blockIdx.y * 16, tok = m0 + r;
+    const int g0 = wave * GPS;
+    if (g0 < G) {
+        v4i a[GPS][2], b[GPS][2];
+        uint16_t nv[GPS][4];
+        float s[GPS];
+        // (groups past G reload the last one; never stored)
+#pragma unroll
+        for (int j = 0; j < GPS; ++j) {
+            const int g = min(g0 + j, G - 1);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                a[j][h] = *reinterpret_cast<const v4i*>(w8 + ((size_t)(tile * G + g) * 2 + h) * 64 + lane);
+                b[j][h] = *reinterpret_cast<const v4i*>(xq + ((size_t)tok * G + g) * 8 + h * 4 + q);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) nv[j][v] = norms[(size_t)(tile * 16 + 4 * q + v) * G + g];
+            s[j] = sx[(size_t)tok * G + g];
+        }
+        const bool blk = tok < M ? (block ? block[tok] != 0 : tok < blocked) : true;
+#pragma unroll
+        for (int j = 0; j < GPS; ++j) {
+            v4i d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j][0], b[j][0], v4i{0, 0, 0, 0}, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j][1], b[j][1], d, 0, 0, 0);
+            if (g0 + j < G) {
+                float* o = part + (size_t)(g0 + j) * 512 + r * 16 + 4 * q;
+                float4 sc;
+                float* f = reinterpret_cast<float*>(&sc);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const float n = f16_bits_to_f32(nv[j][v]);
+                    f[v] = blk ? (n * cbs) * s[j] : n * (cbs * s[j]);
+                }
+                *reinterpret_cast<float4*>(o) = make_float4((float)d[0], (float)d[1], (float)d[2], (float)d[3]);
+                *reinterpret_cast<float4*>(o + 256) = sc;
+            }
+        }
+    }
+    __syncthreads();
+    if (tid >= 256) return;
+    float acc = 0.0f;
+#pragma unroll 4
+    for (int g = 0; g < G; ++g) acc = __builtin_fmaf(part[g * 512 + tid], part[g * 512 + 256 + tid], acc);
+    const int m = m0 + (tid >> 4), n = tile * 16 + (tid & 15);
+    if (m < M && n < out) y[(size_t)m * ldy + col0 + n] = acc;
+}
+
+static hipError_t run_split(const nh_qmat* w, const nh_qact* a, float* y, const uint8_t* block, int ldy, int col0,
+                            hipStream_t s) {
+    const QMatMeta& m = w->m;
+    const int M = a->rows, G = m.groups, gps = (G + SPLIT_WAVES - 1) / SPLIT_WAVES;
+    const int waves = std::max(4, (G + gps - 1) / gps);  // (256 threads run the chains)
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(m.out_pad / 16, (M + 15) / 16), dim3(64 * waves), (size_t)G * 2048, s,
+                           (const uint4*)w->d_w8, w->d_norms, (const uint4*)a->d_xq, a->d_sx, y, block, M / 4 * 4, ldy,
+                           col0, m.out, M, G, m.cbs);
+        return hipGetLastError();
+    };
+    return gps <= 1 ? go(k_gemm_split<1>) : gps == 2 ? go(k_gemm_split<2>) : gps == 3 ? go(k_gemm_split<3>)
+                                                                                       : go(k_gemm_split<4>);
+}
+
 static hipError_t gemm_dispatch(const GemmSet& g, const uint8_t* block, int ldy, int col0, int32_t* dbg,
                                 hipStream_t s) {
     const nh_qmat* w = g.w[0];
@@ -504,6 +583,13 @@ static hipError_t gemm_dispatch(const GemmSet& g, const uint8_t* block, int ldy,
     const int M = a->rows, cus = device_cus(), out_pad = w->m.out_pad;
     // (items over all the launch's products)
     auto items = [&](int rows, int bm) { return (long)g.n * ((out_pad + rows - 1) / rows) * ((M + bm - 1) / bm); };
+    // Tiles that fit the chip once (twice up to 16 groups, where two
+    // workgroups' LDS and loads share a CU): measured, us, k_gemm / this: 64 x
+    // 768 x 768 3.66 / 3.05, 16 x 768 x 8192 4.34 / 3.55, 64 x 3072 x 768 6.35 /
+    // 5.07, 118 x 4096 x 512 8.06 / 5.98; past the line 118 x 768 x 1568 4.11
+    // / 4.50, 160 x 4096 x 512 7.50 / 9.08.
+    if (g.n == 1 && !dbg && (long)out_pad / 16 * ((M + 15) / 16) <= (w->m.groups <= 16 ? 2L : 1L) * cus)
+        return run_split(w, a, g.y[0], block, ldy, col0, s);
     if (M > 48 && items(64, 64) >= cus)
         return general ? run<64, 4, 1, true, false>(g, block, ldy, col0, dbg, s)
                        : run<64, 4, 1, false, false>(g, block, ldy, col0, dbg, s);
