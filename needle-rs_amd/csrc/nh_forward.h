@@ -52,6 +52,7 @@ struct Dims {
     int orders[4];
     int cap;    // session positions
     int batch;  // rows of the row buffers: cap rounded up to whole BATCH_MIN, within BATCH_MIN .. BATCH_MAX
+                // (BATCH_MIN past 64 attention chunks)
     int kslots; // KV slots of a layer: a slot per position, then from stage0 on one per row of a feed
     int stage0; // cap rounded up to 16
     int vcap;   // row stride of the transposed int8 values: kslots + 4 rounded up to 16
