@@ -289,12 +289,17 @@ __global__ __launch_bounds__(64 * NW, DBG ? 1 : 2) void k_gemm(
             if (m >= M) continue;
             float* dst = y + (size_t)m * ldy + col0 + n0;
             if (vec_store && n0 + 3 < out) {
-                // (the opaque pointer keeps the 16-byte store whole: the
-                // compiler would share its first element with the other
-                // form's, a 4- and a 12-byte store; the 4096-row head 90.2 ->
-                // 80.5 us, a 1024-row projection 16.5 -> 16.0 us)
-                asm("" : "+v"(dst));
-                *reinterpret_cast<float4*>(dst) = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+                // The largest products' outputs leave as whole 16-byte stores
+                // with the streaming hint (plain, the compiler shares the first
+                // element with the other form's, a 4- and a 12-byte store). us:
+                // 1024 x 768 x 2304 10.8 -> 8.8, 4096 x 768 x 8192 80.9 -> 71.0,
+                // 2048 x 3072 x 3072 49.0 -> 46.5.  The smaller tiles keep the
+                // plain form: 256 x 3072 x 768 measured 6.70 -> 7.13 with whole
+                // stores.
+                if constexpr (BM == 64)
+                    __builtin_nontemporal_store(f32x4{acc[t][0], acc[t][1], acc[t][2], acc[t][3]}, reinterpret_cast<f32x4*>(dst));
+                else
+                    *reinterpret_cast<float4*>(dst) = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
             } else {
 #pragma unroll
                 for (int v = 0; v < 4; ++v)
