@@ -68,30 +68,37 @@ __device__ __forceinline__ void a8_oct(float (&v)[EL], int l, int bits, bool on,
     oct_stage<2>(v, l);
     oct_stage<4>(v, l);
     const float hs = bits_f32(0x3db504f3u);
+    // A maximum that keeps a NaN (v_maximum3_f32, at fmaxf's rate).
     float m = 0.0f;
 #pragma unroll
     for (int i = 0; i < EL; ++i) {
         v[i] *= hs;
-        m = fmaxf(m, fabsf(v[i]));
+        m = __builtin_elementwise_maximum(m, fabsf(v[i]));
     }
-    m = fmaxf(m, oct_xor<1>(m));
-    m = fmaxf(m, oct_xor<2>(m));
-    m = fmaxf(m, oct_xor<4>(m));
-    // Infinite inputs leave infinities and NaNs in a group: as in a8_group, a
-    // NaN at both positions p and p + 64 makes the maximum NaN (scale 1).
-    // (A NaN input makes every position NaN: maximum 0, scale 1.)
-    if (__any(m == __builtin_inff())) {
+    m = __builtin_elementwise_maximum(m, oct_xor<1>(m));
+    m = __builtin_elementwise_maximum(m, oct_xor<2>(m));
+    m = __builtin_elementwise_maximum(m, oct_xor<4>(m));
+    // Non-finite inputs, and finite ones that overflow, leave NaNs in a group.
+    // As in a8_group, one at both positions p and p + 64 makes the scale 1
+    // (also where the other positions are finite); one whose partner is not
+    // NaN is passed over by the maximum.
+    if (__any(m != m)) {
         int both = 0;
+        float mx = 0.0f;
 #pragma unroll
         for (int i = 0; i < EL; ++i) {
             const float o = oct_xor<4>(v[i]);
             both |= (v[i] != v[i]) & (o != o);
+            mx = fmaxf(mx, fabsf(v[i]));
         }
         float f = both ? 1.0f : 0.0f;
         f = fmaxf(f, oct_xor<1>(f));
         f = fmaxf(f, oct_xor<2>(f));
         f = fmaxf(f, oct_xor<4>(f));
-        if (f != 0.0f) m = 0.0f;
+        mx = fmaxf(mx, oct_xor<1>(mx));
+        mx = fmaxf(mx, oct_xor<2>(mx));
+        mx = fmaxf(mx, oct_xor<4>(mx));
+        if (m != m) m = f != 0.0f ? 0.0f : mx;
     }
     const float s = m > 0.0f ? m * bits_f32(0x3c010204u) : 1.0f;
     const float inv = 1.0f / s;
