@@ -675,7 +675,9 @@ static void attend_head(const nf_model* m, const nf_session* s, int l, const flo
     float* scale = (float*)malloc(chunk * sizeof(float));
     int32_t* dots = (int32_t*)malloc(chunk * sizeof(int32_t));
     int8_t* dig = (int8_t*)malloc(3 * chunk);
-    float pm[8], psum[8], po[8][64];
+    /* (a chunk holds at most 256 keys, so `count` grows with them) */
+    float* pm = (float*)malloc((count ? count : 1) * 66 * sizeof(float));
+    float *psum = pm + count, (*po)[64] = (float(*)[64])(psum + count);
     int np = 0;
     for (size_t c0 = 0; c0 < n; c0 += chunk) {
         const size_t len = chunk < n - c0 ? chunk : n - c0;
@@ -726,7 +728,7 @@ static void attend_head(const nf_model* m, const nf_session* s, int l, const flo
         const float inv = 1.0f / total;
         for (size_t i = 0; i < vd; ++i) out[i] = acc[i] * inv;
     }
-    free(sc), free(scale), free(dots), free(dig), free(slots);
+    free(sc), free(scale), free(dots), free(dig), free(slots), free(pm);
 }
 
 /* The test hook for attend_head: one head against keys written straight
