@@ -2012,11 +2012,11 @@ __global__ __launch_bounds__(AG_T * RP) __attribute__((amdgpu_waves_per_eu(RP ==
     int wv, int geom, Dims D, SessDev S, LayerDev L, int layer) {
     // (the staging's operands lead the arguments as scalars, preloaded at
     // wave launch: the queries, the layer's key rows, scales and value
-    // columns, the window | value stride << 16 and the geometry
+    // columns, the window | value stride / 16 << 16 and the geometry
     // nh | nkv | qk | vd; the parameters and the loads need no read of the
     // argument segment)
     const int g_nh = geom & 255, g_nkv = (geom >> 8) & 255, g_qk = (geom >> 16) & 255,
-              g_vd = (int)((unsigned)geom >> 24), window = wv & 0xffff, vcap = (int)((unsigned)wv >> 16);
+              g_vd = (int)((unsigned)geom >> 24), window = wv & 0xffff, vcap = (int)((unsigned)wv >> 16) * 16;
     constexpr int NTT = AG_T * RP, AG_COLS = SPAN ? AG_COLS_4 : AG_COLS_1;
     // (the row half and the wavefront are wave-uniform: in scalar registers,
     // so the lengths and bounds derived from them are too)
@@ -2344,10 +2344,12 @@ __global__ __launch_bounds__(AG_T * RP) __attribute__((amdgpu_waves_per_eu(RP ==
     }
 }
 
-// The geometry k_attend_group takes (its packed arguments).
+// The geometry k_attend_group takes (its packed arguments; the value stride,
+// a multiple of 16, in units of 16, so a session's staging slots behind its
+// capacity's take no capacity off the kernel).
 static bool attend_group_fits(const Dims& D, const LayerDev& L) {
     return D.nh / D.nkv <= AG_WAVES && D.nh < 256 && D.nkv < 256 && D.qk < 256 && D.vd < 256 && L.window >= 0 &&
-           L.window < 65536 && D.vcap < 65536;
+           L.window < 65536 && D.vcap / 16 < 65536;
 }
 
 bool attend_staged_fits(const Dims& D, const LayerDev& L) { return attend_group_fits(D, L); }
@@ -2387,7 +2389,8 @@ hipError_t fwd_attend(const Dims& D, const SessDev& S, const LayerDev& L, int la
         const float* ksl = S.ks + lc * D.nkv;
         const float* vsl = S.vs + lc * D.nkv;
         const int8_t* v8l = S.v8t + (size_t)layer * D.nkv * D.vd * D.vcap;
-        const int geom = D.nh | D.nkv << 8 | D.qk << 16 | D.vd << 24, wv = L.window | D.vcap << 16;
+        const int geom = D.nh | D.nkv << 8 | D.qk << 16 | D.vd << 24;
+        const int wv = (int)((unsigned)L.window | (unsigned)(D.vcap / 16) << 16);
         auto go = [&](auto kern, int rp) {
             hipLaunchKernelGGL(kern, dim3((t + rp - 1) / rp * D.nkv, most), dim3(rp * AG_T), 0, s, S.qbuf, k8l, ksl,
                                vsl, v8l, p0, t, wv, geom, D, S, L, layer);

@@ -103,6 +103,20 @@ int key_chunk_count(int n, int nkv) {
     return chunk ? (n + chunk - 1) / chunk : 0;
 }
 
+// The sizes of a session of `cap` positions over the model's geometry in D.
+void session_sizes(nh::Dims& D, int cap) {
+    D.cap = cap;
+    D.stage0 = (int)round_up((size_t)cap, 16);
+    int mc = 1;
+    for (int n = 1; n <= cap; ++n) mc = std::max(mc, key_chunk_count(n, D.nkv));
+    D.max_chunks = mc;
+    // (the chunk partials grow with both: at 2048 rows 100 MB a 16 chunks, so a
+    // capacity of more than 64 chunks keeps the smaller feeds)
+    D.batch = mc <= 64 ? std::min(nh::BATCH_MAX, (int)round_up((size_t)cap, nh::BATCH_MIN)) : nh::BATCH_MIN;
+    D.kslots = D.stage0 + D.batch;
+    D.vcap = (int)round_up((size_t)D.kslots + 4, 16);
+}
+
 }  // namespace
 
 struct nh_model {
@@ -898,16 +912,8 @@ int nh_session_new(const nh_model* m, int cap, nh_session** out) {
     s->m = m;
     nh::Dims& D = s->dims;
     D = m->dims;
-    D.cap = cap;
-    D.stage0 = (int)round_up((size_t)cap, 16);
-    int mc = 1;
-    for (int n = 1; n <= cap; ++n) mc = std::max(mc, key_chunk_count(n, D.nkv));
-    D.max_chunks = mc;
-    // (the chunk partials grow with both: at 2048 rows 100 MB a 16 chunks, so a
-    // capacity of more than 64 chunks keeps the smaller feeds)
-    D.batch = mc <= 64 ? std::min(nh::BATCH_MAX, (int)round_up((size_t)cap, nh::BATCH_MIN)) : nh::BATCH_MIN;
-    D.kslots = D.stage0 + D.batch;
-    D.vcap = (int)round_up((size_t)D.kslots + 4, 16);
+    session_sizes(D, cap);
+    const int mc = D.max_chunks;
     const size_t d = D.d, L = D.layers, c = cap, E = D.sites;
     const size_t half = D.qk / 2;
     const int Gd = (D.d + nh::GROUP - 1) / nh::GROUP, Ga = (D.nh * D.vd + nh::GROUP - 1) / nh::GROUP;
