@@ -27,8 +27,9 @@ constexpr int ENGRAM_TAPS = 4;      // ENGRAM_CONV_TAPS (config.rs:10)
 constexpr int ATT_CHUNK_MAX = 256;  // key_chunks never makes a chunk longer
 constexpr int ATT_THREADS = 256;
 constexpr int FWD_ROWS = 32;        // token rows of one prompt chunk (infer.rs:1105-1132)
-// Token rows of one feed (whole chunks of a prompt fed together): the least
-// and the most a session's row buffers hold, by its capacity (Dims::batch).
+// Token rows of one feed (whole chunks of a prompt fed together): the rows a
+// session's own buffers hold, and the most of a feed, by the capacity
+// (Dims::batch), in buffers that a model's sessions share.
 // More rows a launch fill the chip better and pay a layer's launches and
 // first loads less often: a 3000-token prompt 10.30 -> 8.57 ms (9.01 at 1024 rows).
 // Both are multiples of the GEMM's 64-token tiles.
@@ -51,12 +52,12 @@ struct Dims {
     int sites, ntab, eheads, seed_stride, slots, sub, dilation;
     int orders[4];
     int cap;    // session positions
-    int batch;  // rows of the row buffers: cap rounded up to whole BATCH_MIN, within BATCH_MIN .. BATCH_MAX
-                // (BATCH_MIN past 64 attention chunks)
+    int batch;  // a session's: the most rows of a feed, cap rounded up to whole BATCH_MIN, within
+                // BATCH_MIN .. BATCH_MAX (BATCH_MIN past 64 attention chunks); a feed's: its row buffers' rows
     int kslots; // KV slots of a layer: a slot per position, then from stage0 on one per row of a feed
     int stage0; // cap rounded up to 16
     int vcap;   // row stride of the transposed int8 values: kslots + 4 rounded up to 16
-    int max_chunks;  // attention chunks a position can need
+    int max_chunks;  // attention chunks a position can need (a feed's: that its row buffers have room for)
     int spin_limit;  // polls of an in-kernel wait before it gives up (SPIN_LIMIT)
     // per-feed state, set by the host before each feed
     int hist_lo;     // the first position the conv history still holds (LayerState::hist,
@@ -102,7 +103,7 @@ struct Globals {
 };
 
 // One session's state, all device memory.  Row buffers hold the rows of
-// the current feed (Dims::batch at most); activations feed the products.
+// the current feed (its Dims::batch at most); activations feed the products.
 struct SessDev {
     float* xs;        // [rows][4][d] residual lanes
     float* u;         // [rows][d] mHC read of the layer

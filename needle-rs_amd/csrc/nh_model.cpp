@@ -11,11 +11,14 @@
 // infer.rs:850-867, dequantized on the device with QMat::row), the RoPE
 // tables powf / sincosf (Tables::new, infer.rs:942-947) and the gate
 // constants.  A session is one HBM arena: residual lanes, KV caches, tap
-// and engram histories, activation buffers and logits.
+// and engram histories, activation buffers and logits; the row buffers of its
+// longest feeds are the model's sessions' together (WideRows).
 #include <math.h>
 #include <string.h>
 
 #include <algorithm>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -103,6 +106,11 @@ int key_chunk_count(int n, int nkv) {
     return chunk ? (n + chunk - 1) / chunk : 0;
 }
 
+// The attention chunks a row of a feed of several rows can need: one per
+// ATT_CHUNK_MAX keys (nested in the feed's rows, infer.rs:1888), where a step
+// splits fewer keys into more (D.max_chunks).
+int feed_chunks(int cap) { return (cap + nh::ATT_CHUNK_MAX - 1) / nh::ATT_CHUNK_MAX; }
+
 // The sizes of a session of `cap` positions over the model's geometry in D.
 void session_sizes(nh::Dims& D, int cap) {
     D.cap = cap;
@@ -117,6 +125,66 @@ void session_sizes(nh::Dims& D, int cap) {
     D.vcap = (int)round_up((size_t)D.kslots + 4, 16);
 }
 
+// The row buffers of feeds of more than BATCH_MIN rows: one set for all of a
+// model's sessions whose capacity takes such feeds, made by the first of them
+// and given back with the last.  (Each session holding its own took 278 MB for
+// 4,096 positions of Needle 3, where BATCH_MIN rows take 70.)  Nothing in them
+// outlives a feed, so feeds on several streams take turns: each waits on its
+// stream for the one before (such a feed fills the chip by itself).
+struct WideRows {
+    std::mutex mu;            // held while a call that uses them queues its feeds
+    void* buf = nullptr;
+    size_t bytes = 0;
+    hipEvent_t ev = nullptr;  // behind the last such call's
+    bool used = false;
+    ~WideRows() {
+        if (ev) (void)hipEventDestroy(ev);
+        if (buf) (void)hipFree(buf);
+    }
+};
+
+// Makes them at least `bytes` long, if the memory is there.
+void wide_reserve(WideRows& w, size_t bytes) {
+    std::lock_guard<std::mutex> lk(w.mu);
+    if (bytes <= w.bytes) return;
+    void* p = nullptr;
+    hipError_t e = w.ev ? hipSuccess : hipEventCreateWithFlags(&w.ev, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipMalloc(&p, bytes);
+    if (e == hipSuccess) e = hipMemset(p, 0, bytes);
+    if (e == hipSuccess) e = hipDeviceSynchronize();  // (and the feeds queued on the old ones)
+    if (e != hipSuccess) {
+        if (p) (void)hipFree(p);
+        (void)hipGetLastError();
+        return;
+    }
+    if (w.buf) (void)hipFree(w.buf);
+    w.buf = p;
+    w.bytes = bytes;
+}
+
+// One call's use of them, from its first such feed to the end of the scope (an
+// event behind whatever it queued, also if it failed part way).
+struct WideUse {
+    WideRows* w = nullptr;
+    hipStream_t st = nullptr;
+    std::unique_lock<std::mutex> lk;
+    hipError_t begin(WideRows* rows, hipStream_t stream) {
+        if (w) return hipSuccess;
+        std::unique_lock<std::mutex> l(rows->mu);
+        if (rows->used)
+            if (const hipError_t e = hipStreamWaitEvent(stream, rows->ev, 0); e != hipSuccess) return e;
+        w = rows, st = stream, lk = std::move(l);
+        return hipSuccess;
+    }
+    ~WideUse() {
+        if (!w) return;
+        if (hipEventRecord(w->ev, st) == hipSuccess)
+            w->used = true;
+        else
+            (void)hipStreamSynchronize(st);
+    }
+};
+
 }  // namespace
 
 struct nh_model {
@@ -130,6 +198,9 @@ struct nh_model {
     nh_qmat* head = nullptr;  // the embedding's first out_rows rows (shares its memory)
     int head_bits = 4;
     void* d_small = nullptr;
+    // (made and dropped by the sessions)
+    mutable std::mutex wide_mu;
+    mutable std::weak_ptr<WideRows> wide;
 
     ~nh_model() {
         if (d_small) (void)hipFree(d_small);
@@ -143,7 +214,7 @@ struct nh_session {
     nh::Dims dims{};
     nh::SessDev S{};  // (with the row buffers of `many`)
     void* d_buf = nullptr;
-    size_t bytes = 0;
+    size_t state_bytes = 0;  // of d_buf: all but the row buffers of `many`
     int len = 0;
     bool have_logits = false;  // S.logits holds the logits of position len - 1
     bool have_hidden = false;  // S.last_hid holds NatState::last_hidden
@@ -161,12 +232,17 @@ struct nh_session {
         nh::SessDev S{};
         nh_qact a_in{}, a_att{};
         std::vector<nh_qact> a_eng;
-        int rows = 0;
+        int rows = 0, chunks = 0;  // (attention chunk partials a row has room for)
     };
     // A step's are a set of their own, one row each, side by side: row 0 of
-    // buffers of Dims::batch rows would be a page each (eight steps at 2,900
-    // keys, 2048 rows: 4.50 ms so, 4.47 with the set).
+    // buffers of many rows would be a page each (eight steps at 2,900 keys,
+    // 2048 rows: 4.50 ms so, 4.47 with the set).
     Rows step, many;
+    // Feeds of more rows than `many` has: the model's WideRows, with this
+    // session's layout of them (offsets; placed anew for each feed).
+    std::shared_ptr<WideRows> wide;
+    Rows wide_at;
+    size_t wide_bytes = 0;
     // The status word as the stream last copied it (pinned), behind
     // ev_status; pending while that copy has not been read.
     int32_t* h_status = nullptr;
@@ -482,6 +558,87 @@ int build_model(nh_model* m, const nh::ArchiveSmall& sm) {
     return NH_OK;
 }
 
+// The row buffers of a feed of up to R rows, `chunks` attention chunks each:
+// their offsets in a layout (in the pointers' place until place_rows).
+void take_rows(Layout& Y, const nh::Dims& D, size_t R, size_t chunks, nh_session::Rows& B) {
+    const size_t d = D.d, E = D.sites, half = D.qk / 2;
+    const size_t Gd = (D.d + nh::GROUP - 1) / nh::GROUP, Ga = (D.nh * D.vd + nh::GROUP - 1) / nh::GROUP;
+    nh::SessDev& S = B.S;
+    auto f = [&](float*& p, size_t n) { p = (float*)Y.take(n * 4); };
+    auto q = [&](int8_t*& p, size_t n) { p = (int8_t*)Y.take(n); };
+    f(S.xs, R * 4 * d), f(S.u, R * d), f(S.x1, R * d), f(S.p, R * 64), f(S.proj, R * D.nq);
+    f(S.qbuf, R * D.nh * D.qk), f(S.o, R * d), f(S.ekv, E * R * 2 * d), f(S.evals, E * R * d);
+    f(S.rope_c, R * half), f(S.rope_s, R * half), f(S.hid, R * d);
+    f(S.po, R * D.nh * chunks * D.vd), f(S.pm, R * D.nh * chunks), f(S.psum, R * D.nh * chunks);
+    q(S.xq_in, R * Gd * nh::GROUP), f(S.sx_in, R * Gd);
+    q(S.xq_att, R * Ga * nh::GROUP), f(S.sx_att, R * Ga);
+    q(S.xq_eng, E * R * Gd * nh::GROUP), f(S.sx_eng, E * R * Gd);
+    S.flags = (uint8_t*)Y.take(R);
+    B.rows = (int)R;
+    B.chunks = (int)chunks;
+}
+
+// The buffers at their offsets from b on, beside what all of a session's sets
+// share, and the A8 views of them.
+void place_rows(nh_session::Rows& B, uint8_t* b, const nh::SessDev& shared, const nh::Dims& D) {
+    const int Gd = (D.d + nh::GROUP - 1) / nh::GROUP, Ga = (D.nh * D.vd + nh::GROUP - 1) / nh::GROUP;
+    const nh::SessDev O = B.S;
+    nh::SessDev& S = B.S;
+    S = shared;
+    auto f = [&](float*& p, const float* o) { p = (float*)(b + (size_t)o); };
+    auto q = [&](int8_t*& p, const int8_t* o) { p = (int8_t*)(b + (size_t)o); };
+    f(S.xs, O.xs), f(S.u, O.u), f(S.x1, O.x1), f(S.p, O.p), f(S.proj, O.proj), f(S.qbuf, O.qbuf), f(S.o, O.o);
+    f(S.ekv, O.ekv), f(S.evals, O.evals), f(S.rope_c, O.rope_c), f(S.rope_s, O.rope_s), f(S.hid, O.hid);
+    f(S.po, O.po), f(S.pm, O.pm), f(S.psum, O.psum);
+    q(S.xq_in, O.xq_in), f(S.sx_in, O.sx_in), q(S.xq_att, O.xq_att), f(S.sx_att, O.sx_att);
+    q(S.xq_eng, O.xq_eng), f(S.sx_eng, O.sx_eng);
+    S.flags = b + (size_t)O.flags;
+    auto view = [&](int8_t* xq, float* sx, int in_dim, int groups) {
+        nh_qact a{};
+        a.cap_rows = B.rows;
+        a.rows = 1;
+        a.in_dim = in_dim;
+        a.groups = groups;
+        a.d_xq = xq;
+        a.d_sx = sx;
+        return a;
+    };
+    B.a_in = view(S.xq_in, S.sx_in, D.d, Gd);
+    B.a_att = view(S.xq_att, S.sx_att, D.nh * D.vd, Ga);
+    for (int i = 0; i < D.sites; ++i)
+        B.a_eng.push_back(view(S.xq_eng + (size_t)i * B.rows * Gd * nh::GROUP, S.sx_eng + (size_t)i * B.rows * Gd, D.d,
+                               Gd));
+}
+
+// The model's WideRows, made if none of its sessions holds them (null: no memory).
+std::shared_ptr<WideRows> join_wide(const nh_model* m) {
+    std::lock_guard<std::mutex> lk(m->wide_mu);
+    std::shared_ptr<WideRows> w = m->wide.lock();
+    if (!w) {
+        try {
+            w = std::make_shared<WideRows>();
+        } catch (const std::bad_alloc&) {
+            return nullptr;
+        }
+        m->wide = w;
+    }
+    return w;
+}
+
+// The most rows a feed of the n tokens ahead takes on `st`: the session's own
+// rows', or the model's where they are large enough and the stream is not
+// being captured (a graph would use them without taking its turn).
+int most_rows(const nh_session* s, int n, hipStream_t st) {
+    if (n <= s->many.rows || !s->wide) return s->many.rows;
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &c) != hipSuccess || c != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return s->many.rows;
+    }
+    std::lock_guard<std::mutex> lk(s->wide->mu);
+    return s->wide->bytes >= s->wide_bytes ? s->dims.batch : s->many.rows;
+}
+
 // One product over the feed's rows: the decode combine for one row, the
 // prefill combine (block = i < t / 4 * 4) for more (QMat::matmul_into,
 // qlinear.rs:468-487).
@@ -600,16 +757,24 @@ int out_width(const nh_session* s, int outputs) {
 // staged: under an attention span, the staged form (span_staged held).
 // pick: the greedy loop's step, whose token is the argmax of the previous
 // step's logits, taken by the feed's first kernel.
+// use: of the model's WideRows, for a feed of more rows than the session's own.
 int feed(nh_session* s, int t, int outputs, float* out, float* cells, hipStream_t st, bool pick = false,
-         bool staged = false) {
+         bool staged = false, WideUse* use = nullptr) {
     const nh_model* m = s->m;
-    nh_session::Rows& B = t == 1 ? s->step : s->many;
+    nh_session::Rows wide_rows;
+    if (t > s->many.rows) {
+        NH_TRY(use->begin(s->wide.get(), st), "feed rows");
+        wide_rows = s->wide_at;
+        place_rows(wide_rows, (uint8_t*)s->wide->buf, s->S, s->dims);
+    }
+    nh_session::Rows& B = t == 1 ? s->step : t > s->many.rows ? wide_rows : s->many;
     nh::SessDev S = B.S;
     S.cells = cells;
     const int p0 = s->len;
     const uint8_t* flags = t > nh::FWD_ROWS ? S.flags : nullptr;
     nh::Dims D = s->dims;
     D.batch = B.rows;
+    D.max_chunks = B.chunks;
     D.hist_lo = p0 - s->hrows;
     D.rope_prev = t == 1 && s->rope_n > 0;
     D.sink = s->sink;
@@ -805,7 +970,8 @@ int forward_ids(nh_session* s, const uint32_t* toks, int n, int outputs, float* 
     NH_TRY(hipMemcpyAsync(s->S.tokens + s->len, toks, (size_t)n * 4, hipMemcpyHostToDevice, st), "tokens");
     s->toks.resize(s->len);
     s->toks.insert(s->toks.end(), toks, toks + n);
-    const int width = out_width(s, outputs);
+    const int width = out_width(s, outputs), most = most_rows(s, n, st);
+    WideUse use;
     int rows = 0;
     for (int i = 0; i < n;) {
         // whole chunks of 32 together while every chunk has two tokens or
@@ -815,14 +981,14 @@ int forward_ids(nh_session* s, const uint32_t* toks, int n, int outputs, float* 
         int t = std::min(nh::FWD_ROWS, n - i);
         const bool staged = s->ring > 0 && span_staged(s, t);
         if ((s->ring == 0 || staged) && t > 1)
-            while (t < s->dims.batch && i + t < n && n - (i + t) > 1) t += std::min(nh::FWD_ROWS, n - (i + t));
+            while (t < most && i + t < n && n - (i + t) > 1) t += std::min(nh::FWD_ROWS, n - (i + t));
         const bool last = i + t == n;
         const int want =
             (!last && (outputs == NH_OUT_LAST_LOGITS || outputs == NH_OUT_LAST_HIDDEN)) ? NH_OUT_NONE : outputs;
         const size_t cw = s->cell_floats();
         float* cdst = nullptr;
         if (want_cells) cdst = s->track_cells ? s->d_cells + (size_t)s->ncells * cw : cells ? cells + i * cw : nullptr;
-        const int r = feed(s, t, want, out ? out + (size_t)rows * width : nullptr, cdst, st, false, staged);
+        const int r = feed(s, t, want, out ? out + (size_t)rows * width : nullptr, cdst, st, false, staged, &use);
         if (r < 0) return reset_after(s, r);
         if (cdst && s->track_cells) {
             if (cells)
@@ -913,27 +1079,10 @@ int nh_session_new(const nh_model* m, int cap, nh_session** out) {
     nh::Dims& D = s->dims;
     D = m->dims;
     session_sizes(D, cap);
-    const int mc = D.max_chunks;
     const size_t d = D.d, L = D.layers, c = cap, E = D.sites;
     const size_t half = D.qk / 2;
-    const int Gd = (D.d + nh::GROUP - 1) / nh::GROUP, Ga = (D.nh * D.vd + nh::GROUP - 1) / nh::GROUP;
     Layout Y;
-    // the row buffers (offsets for now) of R rows
-    auto take_rows = [&](nh_session::Rows& B, size_t R) {
-        nh::SessDev& S = B.S;
-        auto f = [&](float*& p, size_t n) { p = (float*)Y.take(n * 4); };
-        auto q = [&](int8_t*& p, size_t n) { p = (int8_t*)Y.take(n); };
-        f(S.xs, R * 4 * d), f(S.u, R * d), f(S.x1, R * d), f(S.p, R * 64), f(S.proj, R * D.nq);
-        f(S.qbuf, R * D.nh * D.qk), f(S.o, R * d), f(S.ekv, E * R * 2 * d), f(S.evals, E * R * d);
-        f(S.rope_c, R * half), f(S.rope_s, R * half), f(S.hid, R * d);
-        f(S.po, R * D.nh * mc * D.vd), f(S.pm, R * D.nh * mc), f(S.psum, R * D.nh * mc);
-        q(S.xq_in, R * Gd * nh::GROUP), f(S.sx_in, R * Gd);
-        q(S.xq_att, R * Ga * nh::GROUP), f(S.sx_att, R * Ga);
-        q(S.xq_eng, E * R * Gd * nh::GROUP), f(S.sx_eng, E * R * Gd);
-        S.flags = (uint8_t*)Y.take(R);
-        B.rows = (int)R;
-    };
-    take_rows(s->step, 1);
+    take_rows(Y, D, 1, D.max_chunks, s->step);
     const size_t o_lg = Y.take(round_up(D.out_rows, nh::PANEL_ROWS) * 4);
     const size_t o_rrc = Y.take(nh::ROPE_RING * half * 4), o_rrs = Y.take(nh::ROPE_RING * half * 4);
     const size_t o_lh = Y.take(d * 4), o_am = Y.take(16), o_st = Y.take(16), o_dc = Y.take(nh::DCOUNT_SLOTS * 4);
@@ -943,7 +1092,8 @@ int nh_session_new(const nh_model* m, int cap, nh_session** out) {
     const size_t o_k8 = Y.take(L * ksl * D.nkv * D.qk), o_ks = Y.take(L * ksl * D.nkv * 4);
     const size_t o_v8 = Y.take(L * D.nkv * D.vd * D.vcap), o_vs = Y.take(L * ksl * D.nkv * 4);
     const size_t o_e8 = Y.take(E * c * d), o_es = Y.take(E * c * (d / 32) * 4);
-    take_rows(s->many, D.batch);
+    s->state_bytes = Y.size;
+    take_rows(Y, D, nh::BATCH_MIN, feed_chunks(cap), s->many);
     hipError_t e = hipMalloc(&s->d_buf, Y.size);
     if (e == hipSuccess) e = hipMemset(s->d_buf, 0, Y.size);
     if (e == hipSuccess) e = hipHostMalloc((void**)&s->h_status, sizeof(int32_t), hipHostMallocDefault);
@@ -953,7 +1103,6 @@ int nh_session_new(const nh_model* m, int cap, nh_session** out) {
         delete s;
         return fail(NH_ENOMEM, std::string("session allocation: ") + hipGetErrorString(e));
     }
-    s->bytes = Y.size;
     uint8_t* b = (uint8_t*)s->d_buf;
     nh::SessDev G{};  // what both sets share
     G.logits = (float*)(b + o_lg), G.tokens = (uint32_t*)(b + o_tok);
@@ -962,37 +1111,16 @@ int nh_session_new(const nh_model* m, int cap, nh_session** out) {
     G.v8t = (int8_t*)(b + o_v8), G.vs = (float*)(b + o_vs), G.ev8 = (int8_t*)(b + o_e8), G.evs = (float*)(b + o_es);
     G.argmax = (int32_t*)(b + o_am), G.status = (int32_t*)(b + o_st), G.dcount = (int32_t*)(b + o_dc);
     D.spin_limit = nh::SPIN_LIMIT;
-    auto place = [&](nh_session::Rows& B) {
-        const nh::SessDev O = B.S;
-        nh::SessDev& S = B.S;
-        S = G;
-        auto f = [&](float*& p, const float* o) { p = (float*)(b + (size_t)o); };
-        auto q = [&](int8_t*& p, const int8_t* o) { p = (int8_t*)(b + (size_t)o); };
-        f(S.xs, O.xs), f(S.u, O.u), f(S.x1, O.x1), f(S.p, O.p), f(S.proj, O.proj), f(S.qbuf, O.qbuf), f(S.o, O.o);
-        f(S.ekv, O.ekv), f(S.evals, O.evals), f(S.rope_c, O.rope_c), f(S.rope_s, O.rope_s), f(S.hid, O.hid);
-        f(S.po, O.po), f(S.pm, O.pm), f(S.psum, O.psum);
-        q(S.xq_in, O.xq_in), f(S.sx_in, O.sx_in), q(S.xq_att, O.xq_att), f(S.sx_att, O.sx_att);
-        q(S.xq_eng, O.xq_eng), f(S.sx_eng, O.sx_eng);
-        S.flags = b + (size_t)O.flags;
-        auto view = [&](int8_t* xq, float* sx, int in_dim, int groups) {
-            nh_qact a{};
-            a.cap_rows = B.rows;
-            a.rows = 1;
-            a.in_dim = in_dim;
-            a.groups = groups;
-            a.d_xq = xq;
-            a.d_sx = sx;
-            return a;
-        };
-        B.a_in = view(S.xq_in, S.sx_in, D.d, Gd);
-        B.a_att = view(S.xq_att, S.sx_att, D.nh * D.vd, Ga);
-        for (int i = 0; i < D.sites; ++i)
-            B.a_eng.push_back(view(S.xq_eng + (size_t)i * B.rows * Gd * nh::GROUP, S.sx_eng + (size_t)i * B.rows * Gd,
-                                   D.d, Gd));
-    };
-    place(s->step);
-    place(s->many);
+    place_rows(s->step, b, G, D);
+    place_rows(s->many, b, G, D);
     s->S = s->many.S;
+    if (D.batch > nh::BATCH_MIN) {
+        Layout W;
+        take_rows(W, D, D.batch, feed_chunks(cap), s->wide_at);
+        s->wide_bytes = W.size;
+        s->wide = join_wide(m);
+        if (s->wide) wide_reserve(*s->wide, s->wide_bytes);
+    }
     *out = s;
     return NH_OK;
 }
@@ -1056,7 +1184,7 @@ int nh_session_clone(const nh_session* s, void* stream, nh_session** out) {
     nh_session* c = nullptr;
     if (int rc = nh_session_new(s->m, s->dims.cap, &c)) return rc;
     hipStream_t st = (hipStream_t)stream;
-    hipError_t e = hipMemcpyAsync(c->d_buf, s->d_buf, s->bytes, hipMemcpyDeviceToDevice, st);
+    hipError_t e = hipMemcpyAsync(c->d_buf, s->d_buf, s->state_bytes, hipMemcpyDeviceToDevice, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) {
         delete c;

@@ -47,6 +47,7 @@ def compile_and_run(tmp_path, main):
         "#include <algorithm>\n#include <cstddef>\n#include <cstdint>\n#include <cstdio>\n",
         "using std::min; using std::max;\nnamespace nh {\n",
         "constexpr int BATCH_MIN = 512, BATCH_MAX = 2048;\n",
+        _constant(hdr, "ATT_CHUNK_MAX"),
         _constant(src, "NATIVE_TEAM"), _constant(src, "AG_WAVES"), _grab(hdr, "struct Dims {", "\n};\n"),
         "struct LayerDev { int window; };\n",
         _grab(src, "static bool attend_group_fits("),
@@ -54,6 +55,7 @@ def compile_and_run(tmp_path, main):
         "}\nusing namespace nh;\n",
         _grab(mod, "size_t round_up(", "}\n"),
         _grab(mod, "int key_chunk_count("),
+        _grab(mod, "int feed_chunks(", "}\n"),
         _grab(mod, "void session_sizes("),
         main,
     ]).replace("__host__ __device__ inline", "inline")
@@ -71,3 +73,30 @@ def test_every_capacity_keeps_grouped_attention(tmp_path):
     """The staging slots behind a capacity's own take no capacity off the
     grouped attention kernel."""
     compile_and_run(tmp_path, MAIN)
+
+
+CHUNKS = r"""
+int main() {
+    // a feed's rows (nested chunks): every count of keys up to the capacity
+    // fits the partials a row has room for, and some count fills them
+    for (int nkv = 1; nkv <= 8; ++nkv) {
+        int most = 0, count, size;
+        for (int n = 1; n <= 40000; ++n) {
+            key_chunks(n, nkv, true, count, size);
+            if (size > 256) return 1;
+            most = std::max(most, count);
+            if (most > feed_chunks(n)) { std::printf("%d keys: %d chunks\n", n, most); return 2; }
+            if (n % 256 == 0 && most != feed_chunks(n)) { std::printf("%d keys: %d of %d\n", n, most, feed_chunks(n)); return 3; }
+        }
+    }
+    std::printf("ok\n");
+    return 0;
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_feed_chunks(tmp_path):
+    """The chunk partials of a feed's rows hold what their keys need, not a
+    step's finer split."""
+    compile_and_run(tmp_path, CHUNKS)
