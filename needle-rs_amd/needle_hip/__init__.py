@@ -138,11 +138,18 @@ def init(device: int = 0):
     return lib
 
 
+# The current stream's handle without building a Stream object: torch's own
+# private calls, where this torch has them.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream(stream=None):
     if stream is not None:
         return stream.cuda_stream
-    # (the current stream's handle without building a Stream object)
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    if _raw_stream is None or _raw_device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_raw_device())
 
 
 def _dptr(t: torch.Tensor):
