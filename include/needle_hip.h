@@ -162,6 +162,12 @@ int nh_debug_partials(const nh_qmat* w, const nh_qact* a, int32_t* out, void* st
  * value with no meaning).  Modes 0 and 1 write nothing and ignore y. */
 int nh_debug_read_floor(const nh_qmat* w, const nh_qact* a, int mode, float* y, void* stream);
 
+/* No reference counterpart (check): the layer kernel's two mix8 passes
+ * (crates/needle-engine/src/infer.rs:2343-2380) over DEVICE operands, a factor
+ * f16 [32][32] and x f32 [32][32]: yt = factor^T x and yn = x factor, f32
+ * [32][32], each output an fma chain in the order of the summed index. */
+int nh_debug_mix8(const uint16_t* factor, const float* x, float* yt, float* yn, void* stream);
+
 /* ---- archives (QWeights, crates/needle-engine/src/weights.rs:136-148) --- */
 /* Weights::from_archive_mode with fast = true (weights.rs:314-467) over the
  * bytes of a .cact archive (Archive::from_raw, crates/needle-core/src/cact.rs:577-583),

@@ -202,9 +202,9 @@ __device__ __forceinline__ int wave_min_i32(int x) {
 
 // `(v * inv).round().clamp(-128, 127) as i8` (crates/needle-engine/src/qlinear.rs:137-139).
 // Rounding half away from zero as the truncation of v + copysign(the float
-// below 1/2, v): the same integer after the clamp for every float (checked
-// over all 2^32, NaN and infinities among them), in half the instructions of
-// roundf.
+// below 1/2, v): the same integer after the clamp for every float (all 2^32,
+// NaN and infinities among them: tests/test_roundings.py), in half the
+// instructions of roundf.
 __device__ __forceinline__ int8_t quant_one(float v, float inv) {
     const float r = v * inv;
     return (int8_t)(int)fminf(fmaxf(r + __builtin_copysignf(0x1.fffffep-2f, r), -128.0f), 127.0f);

@@ -204,6 +204,9 @@ bool dec_chunks_fits(const Dims& D);
 hipError_t fwd_dec_chunks(const Dims& D, const SessDev& S, const LayerDev& L, int layer, int p0, int out_bits,
                           const KeySpan* span, hipStream_t s);
 hipError_t fwd_argmax(const float* logits, int n, uint32_t* dst, hipStream_t s);
+// The layer kernel's two mix8 passes over a factor [32][32] (f16) and x
+// [32][32]: yt = factor^T x, yn = x factor.
+hipError_t fwd_mix8(const uint16_t* factor, const float* x, float* yt, float* yn, hipStream_t s);
 // (nrows at most 24; q in phi_at's order)
 hipError_t fwd_phi8(const float* rows, int nrows, int width, int8_t* q, float* scale, hipStream_t s);
 

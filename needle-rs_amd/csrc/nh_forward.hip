@@ -122,10 +122,9 @@ __host__ __device__ inline void key_chunks(int n, int nkv, bool nested, int& cou
     count = chunk ? (n + chunk - 1) / chunk : 0;
 }
 
-// The attended range of position p0: keys lo..p0.
 // roundf of a value >= 0 as an integer (the attention weights' 21-bit
 // digits): truncating v + the float below 1/2 gives the same for every float
-// in [0, 2^22) (checked over all of them), in two instructions.
+// in [0, 2^22) (tests/test_roundings.py), in two instructions.
 __device__ __forceinline__ int32_t round_digits(float v) { return (int32_t)(v + 0x1.fffffep-2f); }
 
 // slot_of (infer.rs:1749-1756): the KV slot of position p; the sink keeps
@@ -134,6 +133,7 @@ __device__ __forceinline__ int slot_of(const Dims& D, int p) {
     return (D.ring > 0 && p >= D.sink) ? (p - D.sink) % D.ring + D.sink : p;
 }
 
+// The attended range of position p0: keys lo..p0.
 __host__ __device__ inline int window_lo(int window, int p0) {
     return (window > 0 && p0 + 1 > window) ? p0 + 1 - window : 0;
 }
@@ -473,10 +473,9 @@ __device__ __forceinline__ void chain_pipe_any(int nb, Load load, Chain chain) {
 // sum_j ct[j][r] * rows[j][c] over 32 x 32, each output an fma chain from
 // j = 0.  v_mfma_f32_16x16x4_f32 runs exactly that chain: its four products
 // of an output are added one after the other in k order with one rounding
-// each (on gfx950 bit-identical to the fmaf chain over random, wide-range,
-// signed-zero and subnormal operands, and over the reference's results in
-// the forward tests), so eight of them in j order are the reference's 32
-// steps.  Four wavefronts take a 16 x 16 tile of the output each.  A pass is
+// each (bit-identical to the fmaf chain over random, wide-range, signed-zero,
+// subnormal and non-finite operands: tests/test_gpu_mix8.py), so eight of
+// them in j order are the reference's 32 steps.  Four wavefronts take a 16 x 16 tile of the output each.  A pass is
 // one chain of eight dependent MFMAs (34 cycles each) between two LDS round
 // trips, and a lane reads 8 + 8 operands for its 4 outputs; the same chains
 // on the vector ALU (2 x 2 outputs a thread, 64 + 64 operands read for 4
@@ -3441,6 +3440,38 @@ __global__ __launch_bounds__(1024) void k_argmax(const float* __restrict__ x, in
 
 hipError_t fwd_argmax(const float* logits, int n, uint32_t* dst, hipStream_t s) {
     hipLaunchKernelGGL(k_argmax, dim3(1), dim3(1024), 0, s, logits, n, dst);
+    return hipGetLastError();
+}
+
+// ------------------------------------------------------ one mix8 pass alone
+// Both passes of the layer kernel over given operands (nh_debug_mix8): the
+// factor into fragment order, x as each pass reads it.
+__global__ __launch_bounds__(MIX_T) void k_mix8(const uint16_t* __restrict__ factor, const float* __restrict__ x,
+                                                float* __restrict__ yt, float* __restrict__ yn) {
+    __shared__ alignas(16) uint16_t kf[HADA_N];
+    __shared__ alignas(16) float A[HADA_N], B[HADA_NB * BT_PITCH], C[HADA_N];
+    const int t = threadIdx.x;
+    for (int e = t; e < HADA_N; e += MIX_T) {
+        const int st = e & 7, lane = (e >> 3) & 63, tile = e >> 9;
+        kf[e] = factor[(4 * st + lane / 16) * HADA_NB + tile * 16 + lane % 16];
+        A[mix_in(e)] = x[e];
+    }
+    __syncthreads();
+    const uint4* f = reinterpret_cast<const uint4*>(kf);
+    mix8_t(t, f, A, B);
+    __syncthreads();
+    auto at = [](int e) { return (e >> 5) * BT_PITCH + (e & 3) * 8 + ((e & 31) >> 2); };
+    for (int e = t; e < HADA_N; e += MIX_T) yt[e] = B[at(e)];
+    __syncthreads();
+    for (int e = t; e < HADA_N; e += MIX_T) B[at(e)] = x[e];
+    __syncthreads();
+    mix8_n(t, B, f, C, HADA_NB);
+    __syncthreads();
+    for (int e = t; e < HADA_N; e += MIX_T) yn[e] = C[e];
+}
+
+hipError_t fwd_mix8(const uint16_t* factor, const float* x, float* yt, float* yn, hipStream_t s) {
+    hipLaunchKernelGGL(k_mix8, dim3(1), dim3(MIX_T), 0, s, factor, x, yt, yn);
     return hipGetLastError();
 }
 

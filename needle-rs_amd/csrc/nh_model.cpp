@@ -1234,6 +1234,13 @@ int nh_session_sync(nh_session* s, void* stream) {
     return check_status(s, st, true);
 }
 
+int nh_debug_mix8(const uint16_t* factor, const float* x, float* yt, float* yn, void* stream) {
+    if (!factor || !x || !yt || !yn) return fail(NH_EINVAL, "bad arguments");
+    if (!nh::ready()) return fail(NH_ESTATE, "nh_init has not been called");
+    NH_TRY(nh::fwd_mix8(factor, x, yt, yn, (hipStream_t)stream), "mix8");
+    return NH_OK;
+}
+
 int nh_session_debug_spin_limit(nh_session* s, int limit) {
     if (!s || limit < 0) return fail(NH_EINVAL, "bad arguments");
     s->dims.spin_limit = limit > 0 ? limit : 0;

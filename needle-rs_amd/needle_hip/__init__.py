@@ -72,6 +72,7 @@ SIGNATURES = {
     "nh_forward_outputs": (I, [P, P, I, I, P, C.c_int64, P]),
     "nh_forward_cells": (I, [P, P, I, I, P, C.c_int64, P, C.c_int64, P]),
     "nh_debug_read_floor": (I, [P, P, I, P, P]),
+    "nh_debug_mix8": (I, [P, P, P, P, P]),
     "nh_session_track_cells": (I, [P, I]),
     "nh_session_cell_rows": (I, [P]),
     "nh_session_cells": (I, [P, I, I, P, P]),
@@ -619,6 +620,15 @@ class Session:
         if getattr(self, "h", None) and _lib is not None:
             _lib.nh_session_free(self.h)
         self.h = None
+
+
+def debug_mix8(factor: torch.Tensor, x: torch.Tensor, stream=None):
+    """The layer kernel's two mix8 passes (infer.rs:2343-2380) over a factor f16
+    [32][32] and x f32 [32][32]: (factor^T x, x factor)."""
+    assert factor.numel() == x.numel() == 1024 and factor.dtype == torch.float16 and x.dtype == torch.float32
+    yt, yn = torch.empty_like(x), torch.empty_like(x)
+    _check(_lib.nh_debug_mix8(_dptr(factor), _dptr(x), _dptr(yt), _dptr(yn), _stream(stream)))
+    return yt, yn
 
 
 def head_logits_sparse(embedding: QMat, a: QAct, ids: torch.Tensor, out_rows: int, stream=None) -> torch.Tensor:
