@@ -220,11 +220,12 @@ int nh_model_out_rows(const nh_model* m);
 /* Model::session (model.rs:264-280) with room for `cap` positions: the KV
  * caches, tap and engram histories and every activation of feeds of up to 512
  * tokens in one HBM allocation.  A feed of more tokens (capacities above 512)
- * runs through row buffers that the model's sessions share, allocated here by
- * the first of them and released with the last: such feeds on different
- * streams run one after the other.  No feed allocates.  For Needle 3 a session
- * of 1,024 / 3,000 / 4,096 / 16,384 positions holds 71 / 107 / 124 / 313 MB and
- * its model's shared rows 101 / 254 / 279 / 591 MB. */
+ * runs through row buffers that the model's sessions share, allocated here (to
+ * the largest capacity so far) and released once the model and its sessions
+ * are freed: such feeds on different streams run one after the other.  No
+ * feed allocates.  For Needle 3 a session of 1,024 / 3,000 / 4,096 / 16,384
+ * positions holds 71 / 107 / 124 / 313 MB and its model's shared rows 101 /
+ * 254 / 279 / 591 MB. */
 int nh_session_new(const nh_model* m, int cap, nh_session** s);
 int nh_session_free(nh_session* s);
 /* Session::len (model.rs:72-74). */

@@ -126,11 +126,14 @@ void session_sizes(nh::Dims& D, int cap) {
 }
 
 // The row buffers of feeds of more than BATCH_MIN rows: one set for all of a
-// model's sessions whose capacity takes such feeds, made by the first of them
-// and given back with the last.  (Each session holding its own took 278 MB for
-// 4,096 positions of Needle 3, where BATCH_MIN rows take 70.)  Nothing in them
-// outlives a feed, so feeds on several streams take turns: each waits on its
-// stream for the one before (such a feed fills the chip by itself).
+// model's sessions, as large as the largest capacity among them has needed,
+// given back when the model and its sessions are gone.  (Each session holding
+// its own took 278 MB for 4,096 positions of Needle 3, where BATCH_MIN rows
+// take 70; given back with the last session, a program with one session at a
+// time paid for it each time: 184 us in place of 85 to make one of 4,096
+// positions, 534 in place of 267 to free it.)  Nothing in them outlives a feed, so feeds on several
+// streams take turns: each waits on its stream for the one before (such a feed
+// fills the chip by itself).
 struct WideRows {
     std::mutex mu;            // held while a call that uses them queues its feeds
     void* buf = nullptr;
@@ -198,9 +201,7 @@ struct nh_model {
     nh_qmat* head = nullptr;  // the embedding's first out_rows rows (shares its memory)
     int head_bits = 4;
     void* d_small = nullptr;
-    // (made and dropped by the sessions)
-    mutable std::mutex wide_mu;
-    mutable std::weak_ptr<WideRows> wide;
+    std::shared_ptr<WideRows> wide;  // (the sessions hold it too)
 
     ~nh_model() {
         if (d_small) (void)hipFree(d_small);
@@ -610,26 +611,11 @@ void place_rows(nh_session::Rows& B, uint8_t* b, const nh::SessDev& shared, cons
                                Gd));
 }
 
-// The model's WideRows, made if none of its sessions holds them (null: no memory).
-std::shared_ptr<WideRows> join_wide(const nh_model* m) {
-    std::lock_guard<std::mutex> lk(m->wide_mu);
-    std::shared_ptr<WideRows> w = m->wide.lock();
-    if (!w) {
-        try {
-            w = std::make_shared<WideRows>();
-        } catch (const std::bad_alloc&) {
-            return nullptr;
-        }
-        m->wide = w;
-    }
-    return w;
-}
-
 // The most rows a feed of the n tokens ahead takes on `st`: the session's own
 // rows', or the model's where they are large enough and the stream is not
 // being captured (a graph would use them without taking its turn).
 int most_rows(const nh_session* s, int n, hipStream_t st) {
-    if (n <= s->many.rows || !s->wide) return s->many.rows;
+    if (n <= s->many.rows || !s->wide) return s->many.rows;  // (null: a capacity of BATCH_MIN rows)
     hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &c) != hipSuccess || c != hipStreamCaptureStatusNone) {
         (void)hipGetLastError();
@@ -1042,6 +1028,12 @@ int nh_model_load(const uint8_t* bytes, uint64_t n, nh_model** out) {
         return fail(NH_ENOMEM, "out of host memory");
     }
     m->w = w;
+    try {
+        m->wide = std::make_shared<WideRows>();
+    } catch (const std::bad_alloc&) {
+        delete m;
+        return fail(NH_ENOMEM, "out of host memory");
+    }
     nh_weights_header(w, m->header, 49);
     rc = check_geometry(m, sm);
     if (rc == NH_OK) rc = build_model(m, sm);
@@ -1118,8 +1110,8 @@ int nh_session_new(const nh_model* m, int cap, nh_session** out) {
         Layout W;
         take_rows(W, D, D.batch, feed_chunks(cap), s->wide_at);
         s->wide_bytes = W.size;
-        s->wide = join_wide(m);
-        if (s->wide) wide_reserve(*s->wide, s->wide_bytes);
+        s->wide = m->wide;
+        wide_reserve(*s->wide, s->wide_bytes);
     }
     *out = s;
     return NH_OK;

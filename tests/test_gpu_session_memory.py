@@ -40,8 +40,10 @@ def free():
     return torch.cuda.mem_get_info()[0]
 
 
-def test_sessions_share_the_longest_feeds_rows(nh, model):
+def test_sessions_share_the_longest_feeds_rows(nh):
     cap, n = 4096, 6
+    start = free()
+    model = nh.Model.from_archive(archive(G, seed=142))
     state = cap * G.num_layers * G.num_kv_heads * (G.qk_head_dim + G.v_head_dim + 8) + \
         2048 * G.num_layers * G.num_kv_heads * (G.qk_head_dim + G.v_head_dim + 8) + \
         len(G.engram_sites) * cap * (G.d_model + G.d_model // 8)
@@ -53,9 +55,13 @@ def test_sessions_share_the_longest_feeds_rows(nh, model):
     bound = state + 513 * row_bytes(G, cap // 256) + (8 << 20)
     say(f"a session of {cap} positions: {each / 1e6:.1f} MB, the first {(before - held) / 1e6:.1f}; bound {bound / 1e6:.1f}")
     assert each <= bound
-    assert before - held <= bound + 2048 * row_bytes(G, cap // 256) + (8 << 20)
+    wide = 2048 * row_bytes(G, cap // 256) + (8 << 20)
+    assert before - held <= bound + wide
     del first, rest
-    assert before - free() <= 8 << 20
+    assert before - free() <= wide  # (the model keeps them for its next session)
+    del model
+    # (the code objects and small blocks the runtime loaded meanwhile stay)
+    assert start - free() <= 32 << 20 < wide // 4
 
 
 def feeds(s, sizes, seed, stream=None):
