@@ -17,9 +17,9 @@
 // other three are DPP moves, a third of the instructions of two positions a
 // lane (a8_group), and a lane's codes leave as two 8-byte stores (4-bit
 // order) or one of 16 bytes (2-bit).  Graph replay, us, before (a workgroup
-// a row, two positions a lane) and now: 4096 x 768 7.59 -> 4.70, with the
-// norm 10.39 -> 6.84; 1024 x 3072 8.36 -> 4.71, 11.64 -> 9.57; 512 x 768
-// 3.59 -> 3.25, 4.77 -> 4.70.
+// a row, two positions a lane) and now: 4096 x 768 7.10 -> 4.16, with the
+// norm 9.70 -> 6.25; 1024 x 3072 7.41 -> 4.03, 10.90 -> 8.99; 512 x 768
+// 2.82 -> 2.50, 4.19 -> 4.14.
 #include <algorithm>
 
 #include "nh_device.h"

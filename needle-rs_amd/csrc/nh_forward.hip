@@ -376,15 +376,16 @@ hipError_t fwd_engram_hist(const Dims& D, const Globals& G, const SessDev& S, in
 }
 
 // -------------------------------------------------------------- the layer
-// One workgroup of 1024 threads per token row; thread t owns element t of
-// every d- and hada_n-long vector (d <= 1024 = hada_n), and element t of each
-// of the 4 residual lanes, in registers.  Every global read is issued at the
-// start: the Kronecker factors and cond_v land in LDS, the elementwise
-// weights, the thread's cond_u column and its wavefront's Phi8 rows in
-// registers.  The LDS footprint stays under half a CU's, so two rows of a
-// batched feed run on a CU side by side.  The short serial chains (dot16 over d, the gates) run
-// in every wavefront that needs their result, so no barrier is spent on
-// handing it out.
+// One workgroup of 1024 threads, alone on its CU, per token row or per two
+// (a feed of more rows than CUs): 90 or 136 KB of LDS.  Thread t owns
+// element t of every d- and hada_n-long vector (d <= 1024 = hada_n), and
+// element t of each of the 4 residual lanes, in registers.  The previous
+// layer's reads are issued at the start: the Kronecker factors and cond_v
+// land in LDS, the elementwise weights and the thread's cond_u column in
+// registers; the next layer's elementwise reads follow the first barrier and
+// its Phi8 fragments go out beside cond_weights.  A short chain whose result
+// every wavefront needs runs in one wavefront and is handed out behind a
+// barrier, or in all of them where that measured faster (block_rinv_t).
 namespace {
 
 constexpr int MIX_T = 256;    // threads of one mix8: four wavefronts, a 16 x 16 tile of the output each

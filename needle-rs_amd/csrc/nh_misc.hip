@@ -185,7 +185,7 @@ hipError_t launch_cq_pack(const float* w, int rows, int d, int groups, const flo
 // row.  The norms follow, [alloc][G], zeros past the last row.  Packing a 3072 x
 // 768 f32 matrix took most of its time on the host (allocations, the tiling
 // in threads, a second upload): with the tiling here and one stream-ordered
-// temporary, 1629 -> 617 us for the pack and its download.
+// temporary, 1093 -> 619 us for the pack and its download.
 __global__ __launch_bounds__(256) void k_tile4(const uint32_t* __restrict__ packed, const uint16_t* __restrict__ norms,
                                                int out, int alloc, int G, uint64_t sel, uint32_t* __restrict__ tiled,
                                                uint16_t* __restrict__ dnorms) {
