@@ -30,6 +30,7 @@
 #include "nh_device.h"
 #include "nh_forward.h"
 #include "nh_internal.h"
+#include "nh_mix8.h"
 
 namespace nh {
 
@@ -388,8 +389,6 @@ hipError_t fwd_engram_hist(const Dims& D, const Globals& G, const SessDev& S, in
 // barrier, or in all of them where that measured faster (block_rinv_t).
 namespace {
 
-constexpr int MIX_T = 256;    // threads of one mix8: four wavefronts, a 16 x 16 tile of the output each
-constexpr int BT_PITCH = 36;  // floats per row of a first mix8's output (16-byte reads; rows 4 banks apart)
 // Transposed copies for the serial chains, so a chain lane reads its
 // operands as contiguous 16-byte vectors: a dot16 operand x[16 c + l] at
 // l * pitch + c (pitch TP_D for d-long vectors, TP_X for the 4 lanes);
@@ -468,73 +467,6 @@ __device__ __forceinline__ void chain_pipe_any(int nb, Load load, Chain chain) {
         chain_pipe_n<24, DEPTH, Buf>(load, ch);
     else
         chain_pipe<DEPTH, Buf>(nb, load, chain);
-}
-
-// mix8 (infer.rs:2343-2380), portable branch: out[r][c] =
-// sum_j ct[j][r] * rows[j][c] over 32 x 32, each output an fma chain from
-// j = 0.  v_mfma_f32_16x16x4_f32 runs exactly that chain: its four products
-// of an output are added one after the other in k order with one rounding
-// each (bit-identical to the fmaf chain over random, wide-range, signed-zero,
-// subnormal and non-finite operands: tests/test_gpu_mix8.py), so eight of
-// them in j order are the reference's 32 steps.  Four wavefronts take a 16 x 16 tile of the output each.  A pass is
-// one chain of eight dependent MFMAs (34 cycles each) between two LDS round
-// trips, and a lane reads 8 + 8 operands for its 4 outputs; the same chains
-// on the vector ALU (2 x 2 outputs a thread, 64 + 64 operands read for 4
-// outputs) were bound by LDS bandwidth.  With cond_weights' conversions apart
-// from its chain: 32 greedy tokens after a 118-token prompt 16.93 -> 16.58
-// ms, a 512-token prefill 1.328 -> 1.313 ms.
-//
-// Lane (q, i) = (lane / 16, lane % 16) supplies factor element [4 s + q][16 tile + i]
-// of step s, f16 in the staged fragment order: kf[tile * 64 + lane] holds
-// s = 0..7 (the same element as operand A of the transposed pass, where
-// the tile is the output's row block, and as operand B of the plain one,
-// where it is its column block), and gets out[4 q + v][i] of its tile.
-__device__ __forceinline__ f32x4 mix_chain(const uint4& f, const float (&x)[8], bool factor_rows) {
-    const uint32_t fw[4] = {f.x, f.y, f.z, f.w};
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-        const float k = h2f((uint16_t)(fw[s >> 1] >> (16 * (s & 1))));
-        acc = factor_rows ? __builtin_amdgcn_mfma_f32_16x16x4f32(k, x[s], acc, 0, 0, 0)
-                          : __builtin_amdgcn_mfma_f32_16x16x4f32(x[s], k, acc, 0, 0, 0);
-    }
-    return acc;
-}
-
-// Element t (row j = t / 32, column c = t % 32) of the transposed pass's
-// vector operand, column block major: a wavefront's reads of four rows x 16
-// columns are 64 consecutive floats.
-__device__ __forceinline__ int mix_in(int t) { return ((t >> 4) & 1) * (HADA_N / 2) + (t >> 5) * 16 + (t & 15); }
-
-// Transposed (ct = a factor, rows = the vector operand in mix_in order):
-// out[r][c] at out[r * BT_PITCH + 8 (c % 4) + c / 4], so that a lane of the
-// plain pass reads its eight k elements as two 16-byte vectors.
-__device__ __forceinline__ void mix8_t(int u, const uint4* kf, const float* rows, float* out) {
-    const int lane = u & 63, q = lane >> 4, i = lane & 15, rt = (u >> 6) & 1, ct = u >> 7;
-    const uint4 f = kf[rt * 64 + lane];
-    float x[8];
-#pragma unroll
-    for (int s = 0; s < 8; ++s) x[s] = rows[ct * (HADA_N / 2) + s * 64 + lane];
-    const f32x4 o = mix_chain(f, x, true);
-    const int c = ct * 16 + i;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) out[(rt * 16 + 4 * q + v) * BT_PITCH + (c & 3) * 8 + (c >> 2)] = o[v];
-}
-
-// Plain (ct = the output of mix8_t, rows = a factor): out[r][c] row-major,
-// rows r < rows_limit (a multiple of 8).
-__device__ __forceinline__ void mix8_n(int u, const float* ct, const uint4* kf, float* out, int rows_limit) {
-    const int lane = u & 63, q = lane >> 4, i = lane & 15, rt = (u >> 6) & 1, cb = u >> 7;
-    const uint4 f = kf[cb * 64 + lane];
-    const float4* xr = reinterpret_cast<const float4*>(ct + (rt * 16 + i) * BT_PITCH + q * 8);
-    const float4 x0 = xr[0], x1 = xr[1];
-    const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-    const f32x4 o = mix_chain(f, x, false);
-    const int r = rt * 16 + 4 * q;
-    if (r < rows_limit) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) out[(r + v) * HADA_NB + cb * 16 + i] = o[v];
-    }
 }
 
 // Element i of a dot16 operand into its transposed copy.
@@ -3441,38 +3373,6 @@ __global__ __launch_bounds__(1024) void k_argmax(const float* __restrict__ x, in
 
 hipError_t fwd_argmax(const float* logits, int n, uint32_t* dst, hipStream_t s) {
     hipLaunchKernelGGL(k_argmax, dim3(1), dim3(1024), 0, s, logits, n, dst);
-    return hipGetLastError();
-}
-
-// ------------------------------------------------------ one mix8 pass alone
-// Both passes of the layer kernel over given operands (nh_debug_mix8): the
-// factor into fragment order, x as each pass reads it.
-__global__ __launch_bounds__(MIX_T) void k_mix8(const uint16_t* __restrict__ factor, const float* __restrict__ x,
-                                                float* __restrict__ yt, float* __restrict__ yn) {
-    __shared__ alignas(16) uint16_t kf[HADA_N];
-    __shared__ alignas(16) float A[HADA_N], B[HADA_NB * BT_PITCH], C[HADA_N];
-    const int t = threadIdx.x;
-    for (int e = t; e < HADA_N; e += MIX_T) {
-        const int st = e & 7, lane = (e >> 3) & 63, tile = e >> 9;
-        kf[e] = factor[(4 * st + lane / 16) * HADA_NB + tile * 16 + lane % 16];
-        A[mix_in(e)] = x[e];
-    }
-    __syncthreads();
-    const uint4* f = reinterpret_cast<const uint4*>(kf);
-    mix8_t(t, f, A, B);
-    __syncthreads();
-    auto at = [](int e) { return (e >> 5) * BT_PITCH + (e & 3) * 8 + ((e & 31) >> 2); };
-    for (int e = t; e < HADA_N; e += MIX_T) yt[e] = B[at(e)];
-    __syncthreads();
-    for (int e = t; e < HADA_N; e += MIX_T) B[at(e)] = x[e];
-    __syncthreads();
-    mix8_n(t, B, f, C, HADA_NB);
-    __syncthreads();
-    for (int e = t; e < HADA_N; e += MIX_T) yn[e] = C[e];
-}
-
-hipError_t fwd_mix8(const uint16_t* factor, const float* x, float* yt, float* yn, hipStream_t s) {
-    hipLaunchKernelGGL(k_mix8, dim3(1), dim3(MIX_T), 0, s, factor, x, yt, yn);
     return hipGetLastError();
 }
 
